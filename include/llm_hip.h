@@ -143,7 +143,8 @@ typedef struct llh_metrics {
   uint64_t stream_slots;          /* streams holding a workspace slot (scratch and error word) now */
   uint64_t workspace_bytes;       /* device bytes of those slots' scratch now */
   uint64_t d256_decode_calls;     /* decode calls that ran the head_dim-256 kernel */
-  uint64_t generic_decode_calls;  /* llh_paged_decode* calls that ran the element-wise kernel */
+  uint64_t generic_decode_calls;  /* llh_paged_decode* calls outside the tuned kernels' shapes: the packed-row
+                                     kernel at head_dim 128 / 256 over 16-token blocks, else the element-wise one */
 } llh_metrics;
 int llh_ctx_metrics(const llh_ctx *ctx, llh_metrics *out);
 /* Sticky error flags the batched kernels raise instead of faulting: 1 = a

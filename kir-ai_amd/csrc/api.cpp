@@ -168,6 +168,85 @@ int plan_stream(const llh_ctx *ctx, int format, int num_seqs, int kv_heads, int 
   return units >= kStreamMinUnitsPerWave * waves ? wgs : 0;
 }
 
+// Split of the packed-row kernel (rows.hip).  A split holds at least one unit for each of
+// its four wavefronts.  Small steps take the split that gives one workgroup per compute
+// unit (two at head_dim 128): a workgroup's start and its merge cost more than a unit.
+// Steps of more than kSplitUnits units per workgroup take two rounds of them, which
+// levels ragged lengths.  Measured on MI355X in blocks of 16 tokens per split (us):
+//   16 x U[256, 4096], Hq16 / Hkv2, head_dim 256, fp8: 8: 29.6, 16: 20.0, 24: 23.6, 32: 26.1
+//   32 x U[256, 4096], the same over int8:             8: 36.5, 16: 32.0, 32: 30.5, 64: 45.0
+//   32 x U[256, 4096], Hq8 / Hkv4, head_dim 256, bf16: 16: 73.4, 32: 70.4, 64: 80.5
+//   32 x U[256, 4096], Hq24 / Hkv8, head_dim 128:      16: 70.4, 32: 61.3, 64: 67.0
+// `units`: the longest sequence's; `total`: all workgroup rows' together; `out_rows`:
+// (query row, head) pairs.
+struct SplitRows {
+  int split_units;
+  int max_splits;
+  size_t o_off, bytes;
+};
+SplitRows split_rows(const llh_ctx *ctx, const PoolView &pv, int units, long long total, size_t out_rows,
+                     size_t max_bytes) {
+  SplitRows r{};
+  const bool wide = pv.head_dim == kD256HeadDim;
+  const long long slots = (long long)ctx->cus * (wide ? 1 : 2);
+  const long long two_rounds = wide ? 16 : 8;
+  long long per = (total + slots - 1) / slots;
+  if (per > two_rounds) per = std::max(two_rounds, (per + 1) / 2);
+  r.split_units = (int)std::min<long long>(1 << 20, std::max<long long>(4, (per + 3) / 4 * 4));
+  const int opt = ctx->opt(LLH_OPT_DECODE_SPLIT_BLOCKS);
+  if (opt > 0) r.split_units = std::max(1, opt * kFastBlockTokens / rows_unit_keys(pv.head_dim));
+  r.max_splits = std::min(kRowsMaxSplits, std::max(1, (units + r.split_units - 1) / r.split_units));
+  if (units <= kRowsSingleUnits) r.max_splits = 1;
+  for (;; r.max_splits--) {
+    const size_t rows = r.max_splits > 1 ? out_rows * r.max_splits : 0;
+    r.o_off = align_up(rows * sizeof(float2));
+    r.bytes = align_up(r.o_off + rows * pv.head_dim * sizeof(float));
+    if (r.bytes <= max_bytes || r.max_splits == 1) return r;
+  }
+}
+
+// Split of a prefill call on the packed-row kernel: the context lengths are on the device,
+// so the bound is the table row's (or the window's), and a sequence spreads its own keys
+// over at most max_splits splits.
+SplitRows split_prefill_rows(const llh_ctx *ctx, const PoolView &pv, const llh_prefill_desc *d) {
+  const int group = d->num_q_heads / pv.kv_heads;
+  const int uk = rows_unit_keys(pv.head_dim);
+  const long long tiles = ((long long)d->max_chunk_len * group + 15) / 16 * pv.kv_heads * d->num_seqs;
+  long long span = (long long)d->max_blocks_per_seq * kFastBlockTokens;
+  if (d->window > 0) span = std::min<long long>(span, (long long)d->window + d->max_chunk_len);
+  const long long units = std::min<long long>((span + uk - 1) / uk + 1, 1 << 28);
+  const long long slots = (long long)ctx->cus * (pv.head_dim == kD256HeadDim && is16(pv.format) ? 1 : 2);
+  SplitRows r{};
+  r.split_units = 4;
+  r.max_splits = (int)std::min<long long>({(long long)kRowsMaxSplits, std::max(1LL, slots / tiles), (units + 3) / 4});
+  if (units <= kRowsSingleUnits) r.max_splits = 1;
+  const size_t rows = r.max_splits > 1 ? (size_t)d->total_q_rows * d->num_q_heads * r.max_splits : 0;
+  r.o_off = align_up(rows * sizeof(float2));
+  r.bytes = align_up(r.o_off + rows * pv.head_dim * sizeof(float));
+  return r;
+}
+
+// Whether a prefill call of the tuned shapes runs the packed-row kernel.  Its time per key
+// grows with the 16-row tiles of the call, that of the 128-row-tile kernels with the rounds
+// their workgroups (one or two heads of 128 rows each) take: measured on MI355X (us per
+// 1000 keys over bf16 blocks) 0.040 per tile against 28 per round at head_dim 128, 0.093
+// against 31 at head_dim 256; int8 / fp8 at head_dim 128 0.030 against 34.  The packed-row
+// kernel's second launch costs it about 5 us, so it must win by more: at equal
+// (256 workgroups) rounds, 8 x (1024 + chunk): head_dim 128, 256 tiles 27.0 against 36.6 us,
+// 1024 tiles 58.9 against 38.4; head_dim 256, 128 tiles 28.7 against 38.6, 256 tiles 40.8
+// against 38.3.
+bool prefill_takes_rows(const llh_ctx *ctx, const PoolView &pv, const llh_prefill_desc *d) {
+  if (d->max_chunk_len <= 0 || ctx->opt(LLH_OPT_PREFILL_HEADS_PER_WG)) return false;
+  const int group = d->num_q_heads / pv.kv_heads;
+  const long long tiles = ((long long)d->max_chunk_len * group + 15) / 16 * pv.kv_heads;
+  if (tiles > 65535 || d->num_seqs > 65535) return false;  // grid dimensions
+  const bool wide = pv.head_dim == kD256HeadDim;
+  const long long wgs = ((long long)d->max_chunk_len + 127) / 128 * d->num_seqs *
+                        (wide || group % 2 ? d->num_q_heads : d->num_q_heads / 2);
+  const long long per_round = wide ? 128 : is16(pv.format) ? 256 : 512;
+  return tiles * d->num_seqs <= per_round * ((wgs + ctx->cus - 1) / ctx->cus);
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -710,6 +789,25 @@ int llh::plan_decode(llh_ctx *ctx, const llh_kv_pool *pool, const llh_decode_des
   plan->scores_off = 0;
   plan->bytes = align_up(plan->scores_off + (size_t)desc->num_seqs * desc->num_q_heads * plan->score_stride *
                                                  sizeof(float));
+  // head_dim 128 or 256 over 16-token blocks: the packed-row MFMA kernel.  Its partials take
+  // the place of the score rows (the step's workspace is never less than theirs, so what a
+  // caller reserved, or the no-allocation entry refused, stays as it was)
+  plan->rows = pv.format != LLH_KV_INT8_ROW && (pv.head_dim == kFastHeadDim || pv.head_dim == kD256HeadDim) &&
+               pv.block_tokens == kFastBlockTokens && rows_aligned && !ctx->opt(LLH_OPT_FORCE_GENERIC);
+  if (plan->rows) {
+    const int uk = rows_unit_keys(pv.head_dim);
+    const int units = (plan->score_stride + uk - 1) / uk + 1;
+    const long long tiles = (long long)pv.kv_heads * ((group + 15) / 16);
+    const long long total = desc->total_tokens_hint > 0
+                                ? tiles * ((long long)desc->total_tokens_hint / uk + desc->num_seqs)
+                                : tiles * units * desc->num_seqs;
+    const SplitRows sr = split_rows(ctx, pv, units, total, (size_t)desc->num_seqs * desc->num_q_heads, max_bytes);
+    plan->split_units = sr.split_units;
+    plan->max_splits = sr.max_splits;
+    plan->ml_off = 0;
+    plan->o_off = sr.o_off;
+    plan->bytes = std::max(plan->bytes, sr.bytes);
+  }
   return LLH_OK;
 }
 
@@ -762,6 +860,33 @@ int llh::launch_planned_decode(llh_ctx *ctx, const llh_kv_pool *pool, const llh_
     if (e != hipSuccess) return ctx->hip_fail(e, "decode launch");
     return LLH_OK;
   }
+  ctx->generic_decode_calls++;
+  if (plan.rows) {
+    RowsArgs r{};
+    r.pool = pv;
+    r.q = static_cast<const uint16_t *>(d_q);
+    r.out = static_cast<uint16_t *>(d_out);
+    r.context_lens = desc->d_seq_lens;
+    r.tables = desc->d_block_tables;
+    r.ws_o = reinterpret_cast<float *>(ws + plan.o_off);
+    r.ws_ml = reinterpret_cast<float2 *>(ws + plan.ml_off);
+    r.err = err;
+    r.num_seqs = desc->num_seqs;
+    r.q_heads = desc->num_q_heads;
+    r.max_blocks = desc->max_blocks_per_seq;
+    r.window = desc->window;
+    r.split_units = plan.split_units;
+    r.max_splits = plan.max_splits;
+    r.max_span = plan.score_stride;
+    r.zero_bad = 1;
+    r.flag_nonfinite = 1;
+    r.scale = score_scale;
+    r.scale_log2e = score_scale * 1.4426950408889634f;
+    r.gate = static_cast<const uint16_t *>(desc->d_gate);
+    const hipError_t e = launch_rows(r, 1, /*exact_weights=*/true, s);
+    if (e != hipSuccess) return ctx->hip_fail(e, "decode launch");
+    return LLH_OK;
+  }
   GenericDecodeArgs g{};
   g.pool = pv;
   g.q = d_q;
@@ -779,7 +904,6 @@ int llh::launch_planned_decode(llh_ctx *ctx, const llh_kv_pool *pool, const llh_
   g.score_stride = plan.score_stride;
   g.scale = score_scale;
   g.gate = static_cast<const uint16_t *>(desc->d_gate);
-  ctx->generic_decode_calls++;
   hipError_t e = launch_decode_generic(g, 0, 0, s);
   if (e != hipSuccess) return ctx->hip_fail(e, "generic decode launch");
   return LLH_OK;
@@ -995,7 +1119,35 @@ int llh_paged_prefill(llh_ctx *ctx, const llh_kv_pool *pool, const llh_prefill_d
   ctx->prefill_calls++;
   auto ev = ctx->timing_begin(static_cast<hipStream_t>(stream));
   hipError_t e;
-  if (fast) {
+  WsLease lease;
+  SplitRows sr{};
+  bool rows = (fast || fast256) && prefill_takes_rows(ctx, pv, desc);
+  if (rows) {
+    sr = split_prefill_rows(ctx, pv, desc);
+    rows = lease.try_acquire(ctx, static_cast<hipStream_t>(stream), sr.bytes);
+  }
+  if (rows) {
+    RowsArgs r{};
+    r.pool = pv;
+    r.q = a.q;
+    r.out = a.out;
+    r.chunk_starts = a.chunk_starts;
+    r.context_lens = a.context_lens;
+    r.tables = a.tables;
+    r.ws_o = reinterpret_cast<float *>(lease.base() + sr.o_off);
+    r.ws_ml = reinterpret_cast<float2 *>(lease.base());
+    r.err = a.err;
+    r.num_seqs = a.num_seqs;
+    r.q_heads = a.q_heads;
+    r.max_blocks = a.max_blocks;
+    r.window = a.window;
+    r.split_units = sr.split_units;
+    r.max_splits = sr.max_splits;
+    r.scale = score_scale;
+    r.scale_log2e = a.scale_log2e;
+    r.gate = a.gate;
+    e = launch_rows(r, desc->max_chunk_len, /*exact_weights=*/false, static_cast<hipStream_t>(stream));
+  } else if (fast) {
     // two query heads of a kv head per workgroup share its K/V tile stream when the group is even
     const int group = desc->num_q_heads / pv.kv_heads;
     const int hpw_env = ctx->opt(LLH_OPT_PREFILL_HEADS_PER_WG);

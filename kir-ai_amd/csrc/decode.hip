@@ -178,17 +178,6 @@ __device__ __forceinline__ void finalize_state(SoftmaxState<G> &st) {
 }
 
 
-// Two signed int8 codes (bytes b, b+1 of w) as a packed bf16 pair (exact).
-__device__ __forceinline__ uint32_t i8x2_to_bf16(uint32_t w, int b) {
-  return pack_bf16((float)(int8_t)(w >> (8 * b)), (float)(int8_t)(w >> (8 * b + 8)));
-}
-
-// Two OCP e4m3 codes (bytes 2*HI, 2*HI+1 of w) as a packed bf16 pair (exact).
-template <bool HI>
-__device__ __forceinline__ uint32_t fp8x2_to_bf16(uint32_t w) {
-  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, HI));
-}
-
 // One V word of a quantized pool (dim 16j + c, tokens 4g..4g+3) as two packed
 // bf16 pairs: (token 0, token 1) and (token 2, token 3).
 template <int FMT>

@@ -189,6 +189,20 @@ struct WsLease {
     lock = std::unique_lock<std::mutex>(w->mu);
     return ctx->grow_locked(*w, bytes);
   }
+  // The stream's workspace grown to `bytes`, or nothing: false while the stream is being
+  // captured (a captured launch would keep a pointer that a later call may free) and when
+  // the memory cannot be had; the caller then takes a path without scratch.
+  bool try_acquire(llh_ctx *ctx, hipStream_t s, size_t bytes) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return false;
+    w = ctx->slot(s);
+    if (!w) return false;
+    lock = std::unique_lock<std::mutex>(w->mu);
+    if (ctx->grow_locked(*w, bytes) == LLH_OK) return true;
+    (void)hipGetLastError();
+    lock.unlock();
+    return false;
+  }
   int32_t *err() const { return w->err; }
   char *base() const { return static_cast<char *>(w->ptr); }
 };
@@ -203,7 +217,9 @@ struct DecodePlan {
   bool empty = false;  // nothing to launch (no sequences)
   bool fast = false;   // tuned kernels (else the reference-order kernel)
   bool d256 = false;   // tuned: the head_dim-256 (G = 8, bf16 / fp16) kernels (split-K, or stream when stream_wgs > 0)
+  bool rows = false;   // packed-row kernel (rows.hip): head_dim 128 / 256 shapes the tuned kernels do not take
   int group = 0;
+  int split_units = 0;  // rows: least units per split
   int split_blocks = 0, max_splits = 0, stream_wgs = 0;
   size_t ml_off = 0, o_off = 0, desc_off = 0;  // tuned: partial (max, sum), partial outputs, segment descriptors
   int score_stride = 0;

@@ -123,6 +123,38 @@ struct PrefillArgs {
   const uint16_t *gate;     // null, or [T][Hq][D] bf16: out = attention * sigmoid(gate)
 };
 
+// Packed query rows over split keys (rows.hip): decode steps outside the tuned shapes
+// and prefill calls of few rows.  Workspace: partial rows [T][Hq][max_splits].
+constexpr int kRowsMaxSplits = 64;
+constexpr int kRowsSingleUnits = 8;  // sequences of at most this many units are never split
+struct RowsArgs {
+  PoolView pool;            // head_dim 128 or 256, 16-token blocks, any format but int8 rows
+  const uint16_t *q;        // [T][Hq][D] bf16
+  uint16_t *out;            // [T][Hq][D] bf16
+  const int32_t *chunk_starts;  // [num_seqs + 1], or null: decode, one row per sequence
+  const int32_t *context_lens;  // [num_seqs]
+  const int32_t *tables;
+  float *ws_o;              // [T][Hq][max_splits][D]
+  float2 *ws_ml;            // [T][Hq][max_splits]  (max in log2 units, sum)
+  int32_t *err;
+  int32_t num_seqs;
+  int32_t q_heads;
+  int32_t max_blocks;
+  int32_t window;
+  int32_t split_units;      // least units (rows_unit_keys keys) per split
+  int32_t max_splits;       // longer sequences take longer splits
+  int32_t max_span;         // > 0: a longer attended span raises kErrTooManySplits
+  int32_t zero_bad;         // keys of a block outside the pool: 1 = score 0 and a zero value, 0 = masked
+  int32_t flag_nonfinite;   // 1: a non-finite score raises kErrNonFinite
+  float scale;
+  float scale_log2e;
+  const uint16_t *gate;
+};
+int rows_unit_keys(int head_dim);
+// max_rows: host bound on a sequence's query rows; exact_weights: softmax weights keep
+// f32 precision in p . v (always so for int8 / fp8 blocks)
+hipError_t launch_rows(const RowsArgs &a, int max_rows, bool exact_weights, hipStream_t s);
+
 struct WriteBlocksArgs {
   PoolView pool;
   void *k_dst;

@@ -1,0 +1,571 @@
+// Paged attention of few query rows over many keys, on gfx950 MFMA with split keys.
+//
+// The query rows that share a kv head -- the G heads of a decode token, or the heads of
+// a short prefill chunk -- are packed sixteen to a tile (row r = token * G + head), and
+// the keys of a sequence are split over workgroups and, inside one, over its four
+// wavefronts.  A wavefront walks units of 64 keys (32 at head_dim 256): it loads the unit's K and V straight into MFMA operand registers (every
+// byte is used by one wavefront, so LDS would only add a copy), and the next unit's
+// loads are in flight behind the current unit's math.  Wavefronts merge in LDS, splits
+// in paged_rows_merge_kernel.
+//
+// It serves
+//  * decode steps outside the tuned kernels' shapes (head_dim 128 or 256, 16-token
+//    blocks): other group sizes, and int8 / fp8 blocks at head_dim 256 -- the
+//    contract of decode_generic_kernel (f32 softmax weights, non-finite scores
+//    flagged, a block outside the pool scoring 0);
+//  * prefill calls of few rows, where a 128-row tile per head would leave most of the
+//    chip idle (contract of paged_prefill_kernel: positions [lo(pos), pos]).
+// Reference: crates/llm-backend/src/core/native_attention.rs:356-464,707-773.
+//
+// S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_16x16x32 (A 16 x 32: lane l holds row
+// l % 16, k 8 (l / 16) .. +8; B 32 x 16: column l % 16, same k; D: column l % 16, rows
+// 4 (l / 16) .. +4).  The rows of a K operand may be any keys, so they are chosen such
+// that the scores a lane receives belong to adjacent keys of one block, the keys of one
+// load of a V^T row: in step s of 32 keys (blocks 2s, 2s+1), tile j = 0, 1 gives lane
+// group g the keys 32 s + 8 g + 4 j + i.  So P^T goes from the accumulators to the B
+// operand without leaving its lane.
+//
+// int8 / fp8 codes enter the MFMA exactly (as bf16); their scales multiply the scores
+// and the weights in f32.  PARTS = 3 splits every f32 weight into three 16-bit terms
+// (24 bits, the whole f32 significand) for three P V products; PARTS = 1 rounds the
+// weights once, as the tuned 16-bit prefill does.
+//
+// Bound: the chain lengths -> table entry -> K / V at the start of a workgroup and, in long
+// splits, the latency of one unit's loads (one unit in flight per wavefront); HBM traffic
+// is each K / V byte once per 16-row tile.  Measured on MI355X: decode, 16 x U[256, 4096]
+// tokens, Hq16 / Hkv2, head_dim 256, fp8: 3139 us on the element-wise kernel, 19.7 us here
+// (32 MB, 1.6 TB/s); a chunk of 8 tokens over 4099 cached ones, Hq16 / Hkv8, head_dim 128,
+// bf16: 119.5 us on 128-row tiles, 12.6 us here (17 MB, 1.3 TB/s).
+#include "wave_ops.h"
+
+namespace llh {
+
+namespace {
+
+constexpr int BT = kFastBlockTokens;
+constexpr int TILE = 16;  // packed query rows per tile
+constexpr int WAVES = 4;
+
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
+typedef __attribute__((ext_vector_type(8))) _Float16 f16x8_t;
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+
+template <int OP>
+__device__ __forceinline__ f32x4_t mfma16(const u32x4_t &a, const u32x4_t &b, const f32x4_t &c) {
+  if constexpr (OP == kF16)
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c,
+                                                   0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b),
+                                                    c, 0, 0, 0);
+}
+
+__device__ __forceinline__ u32x4_t ld16(const char *p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x4_t *>(p));
+}
+
+// Eight codes as eight bf16 elements (exact).
+template <int FMT>
+__device__ __forceinline__ u32x4_t codes8(uint32_t lo, uint32_t hi) {
+  if constexpr (FMT == kInt8)
+    return u32x4_t{i8x2_to_bf16(lo, 0), i8x2_to_bf16(lo, 2), i8x2_to_bf16(hi, 0), i8x2_to_bf16(hi, 2)};
+  else
+    return u32x4_t{fp8x2_to_bf16<false>(lo), fp8x2_to_bf16<true>(lo), fp8x2_to_bf16<false>(hi),
+                   fp8x2_to_bf16<true>(hi)};
+}
+
+// The keys of a sequence and their split, the same in every kernel of a call.
+struct SeqSplit {
+  int c0, chunk, ctx;  // first query row, query rows, context length
+  int lo;              // first position any row attends
+  int unit0, units;    // units of UK keys
+  int per_split, n_splits;
+  bool skip;           // nothing to compute (flags: why)
+  int flags;
+};
+
+template <int UK>
+__device__ __forceinline__ SeqSplit seq_split(const RowsArgs &a, int b) {
+  SeqSplit s;
+  s.flags = 0;
+  s.c0 = a.chunk_starts ? a.chunk_starts[b] : b;
+  s.chunk = a.chunk_starts ? a.chunk_starts[b + 1] - s.c0 : 1;
+  s.ctx = a.context_lens[b];
+  const int first = s.ctx - s.chunk;  // position of the first row
+  s.lo = a.window > 0 ? max(0, first - a.window + 1) : 0;
+  const int span = max(0, s.ctx - s.lo);
+  if (a.max_span > 0 && span > a.max_span) s.flags = kErrTooManySplits;
+  else if ((int64_t)span > (int64_t)a.max_blocks * BT) s.flags = kErrSpan;
+  s.skip = s.flags != 0 || s.chunk <= 0 || (a.chunk_starts && s.ctx < s.chunk);
+  s.unit0 = s.lo / UK;
+  s.units = span > 0 ? (s.ctx - 1) / UK - s.unit0 + 1 : 0;
+  // short sequences are not split: the second launch costs about what four units cost a
+  // wavefront
+  s.per_split = s.units <= kRowsSingleUnits ? kRowsSingleUnits
+                                            : max(a.split_units, (s.units + a.max_splits - 1) / a.max_splits);
+  s.n_splits = (s.units + s.per_split - 1) / s.per_split;
+  return s;
+}
+
+// keys per unit: K and V of a unit take 64 operand registers each in 16-bit formats (32 in
+// 8-bit ones)
+template <int D>
+constexpr int kUnitKeys = D == 256 ? 32 : 64;
+
+template <int D, int FMT, int PARTS>
+__global__ __launch_bounds__(64 * WAVES, D == 256 && is16(FMT) ? 1 : 2) void paged_rows_kernel(const RowsArgs a) {
+  constexpr bool Q8 = !is16(FMT);
+  constexpr int OP = FMT == kF16 ? kF16 : kBf16;
+  constexpr int UK = kUnitKeys<D>;
+  constexpr int NT = UK / 16;          // score tiles of 16 keys
+  constexpr int NS = UK / 32;          // P V steps of 32 keys
+  constexpr int KS = D / 32;           // k-steps of a score
+  constexpr int KL = Q8 ? D / 64 : KS; // 16-byte loads of a K operand row
+  constexpr int ND = D / 16;           // output tiles
+  constexpr int ES = Q8 ? 1 : 2;
+
+  const int Hkv = a.pool.kv_heads;
+  const int G = a.q_heads / Hkv;
+  const int split = blockIdx.x;
+  const int kvh = blockIdx.y % Hkv;
+  const int tile = blockIdx.y / Hkv;
+  const int b = blockIdx.z;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15;  // packed query row of the tile; operand row of K and V
+  const int g = lane >> 4;    // k group of the operands
+
+  const SeqSplit sq = seq_split<UK>(a, b);
+  if (sq.skip) {
+    if (sq.flags && tid == 0) atomicOr(a.err, sq.flags);
+    return;
+  }
+  const int rows = sq.chunk * G;
+  const int row0 = tile * TILE;
+  if (row0 >= rows || split >= max(sq.n_splits, 1)) return;
+  if (sq.units == 0) {  // empty context: zero output (weighted sum of nothing)
+    for (int i = tid; i < min(TILE, rows - row0) * D; i += 64 * WAVES) {
+      const int r = row0 + i / D;
+      a.out[((size_t)(sq.c0 + r / G) * a.q_heads + kvh * G + r % G) * D + i % D] = 0;
+    }
+    return;
+  }
+
+  // this lane's query row (columns past the last repeat it and are never stored)
+  const int my_row = min(row0 + col, rows - 1);
+  const int my_tok = my_row / G;
+  const int first_pos = sq.ctx - sq.chunk;
+  const int my_pos = first_pos + my_tok;
+  const int my_lo = a.window > 0 ? max(0, my_pos - a.window + 1) : 0;
+  // positions of the tile's first and last row bound what it attends
+  const int tile_pos0 = first_pos + row0 / G;
+  const int tile_pos1 = first_pos + (min(row0 + TILE, rows) - 1) / G;
+  const int tile_lo0 = a.window > 0 ? max(0, tile_pos0 - a.window + 1) : 0;
+
+  // units of this split that the tile attends, dealt to the wavefronts in turn
+  const int ub = max(sq.unit0 + split * sq.per_split, tile_lo0 / UK);
+  const int ue = min(min(sq.unit0 + (split + 1) * sq.per_split, sq.unit0 + sq.units), tile_pos1 / UK + 1);
+  const int n = max(0, (ue - ub - wave + WAVES - 1) / WAVES);
+
+  // ---- Q^T operand: k-step ks, this lane's 8 dims of its row ----
+  // 16-bit: dims 32 ks + 8 g; 8-bit: a 16-byte K load spans two k-steps, dims
+  // 64 (ks / 2) + 16 g + 8 (ks % 2)
+  u32x4_t qb[KS];
+  {
+    const uint16_t *qr = a.q + ((size_t)(sq.c0 + my_tok) * a.q_heads + kvh * G + my_row % G) * D;
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++)
+      qb[ks] = *reinterpret_cast<const u32x4_t *>(qr + (Q8 ? 64 * (ks >> 1) + 16 * g + 8 * (ks & 1) : 32 * ks + 8 * g));
+  }
+  float c = a.scale_log2e, c_nat = a.scale;
+  if constexpr (FMT == kF16) {  // the row's q scaled into fp16 (lanes col + 16 g hold its dims)
+    uint32_t w[4 * KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) w[4 * ks + e] = qb[ks][e];
+    int mx = bf16_absmax_bits<4 * KS>(w);
+    mx = max(mx, __float_as_int(xor16_other(__int_as_float(mx), lane)));
+    mx = max(mx, __float_as_int(xor32_other(__int_as_float(mx), lane)));
+    const F16Scaling sc = f16_scaling(mx);
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) qb[ks][e] = bf16x2_to_f16x2(w[4 * ks + e], sc.inv);
+    c *= sc.step;
+    c_nat *= sc.step;
+  }
+
+  f32x4_t oacc[ND];
+#pragma unroll
+  for (int d = 0; d < ND; d++) oacc[d] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  float m_run = -INFINITY, l_run = 0.0f;
+  bool bad = false, nonfinite = false;
+  const bool zero_bad = a.zero_bad != 0;
+
+  const int32_t *table = a.tables + (size_t)b * a.max_blocks;
+  const int gk = col >> 2;  // lane group whose scores this lane's K operand row feeds
+  struct Entries {
+    int k[NS], v[NS];
+  };
+  // block (of the unit) that holds this lane's K rows / V columns, entry i
+  auto blk_of = [&](int grp, int i) __attribute__((always_inline)) { return 2 * i + (grp >> 1); };
+  auto fetch = [&](int u, Entries &e) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NS; i++) {
+      e.k[i] = table[(uint32_t)(u * NT + blk_of(gk, i)) % (uint32_t)a.max_blocks];
+      e.v[i] = table[(uint32_t)(u * NT + blk_of(g, i)) % (uint32_t)a.max_blocks];
+    }
+  };
+  // pool block of an entry: block 0 where the unit's block is not attended or lies
+  // outside the pool (miss: attended but outside)
+  auto resolve = [&](int u, int grp, int i, int e, bool &miss) __attribute__((always_inline)) -> size_t {
+    const int pos = (u * NT + blk_of(grp, i)) * BT;
+    const bool needed = pos < sq.ctx && pos + BT > tile_lo0;
+    const bool ok = e >= 0 && (int64_t)e < a.pool.n_blocks;
+    miss = needed && !ok;
+    return (size_t)(needed && ok ? e : 0) * Hkv + kvh;
+  };
+  // byte offsets of this lane's operand rows in a block's K (tile 0) and V (output tile 0)
+  const uint32_t k_lane = (8 * (gk & 1) + (col & 3)) * D * ES + 16 * g;
+  const uint32_t v_lane = (col * BT + 8 * (g & 1)) * ES;
+  u32x4_t kr[NT][KL];
+  typedef __attribute__((ext_vector_type(2 * ES))) uint32_t vword_t;  // 8 keys of a V^T row
+  vword_t vr[NS][ND];
+  // int8: the (K, V) fp16 scale pairs of this lane's 8 keys; fp8: the f32 scales of its block
+  u32x4_t sreg[NS][2] = {};
+  auto load_k = [&](int u, const Entries &e) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NS; i++) {
+      bool miss;
+      const size_t bh = resolve(u, gk, i, e.k[i], miss);
+      const char *kb = reinterpret_cast<const char *>(a.pool.k) + bh * (BT * D * ES) + k_lane;
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int x = 0; x < KL; x++) kr[2 * i + j][x] = ld16(kb + 4 * j * D * ES + 64 * x);
+    }
+  };
+  auto load_v = [&](int u, const Entries &e, uint32_t &miss) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NS; i++) {
+      bool ms;
+      const size_t bh = resolve(u, g, i, e.v[i], ms);
+      miss = (miss & ~(1u << i)) | (ms ? 1u << i : 0u);
+      const char *vb = reinterpret_cast<const char *>(a.pool.v) + bh * (BT * D * ES) + v_lane;
+      if constexpr (FMT == kInt8) {
+        const u32x4_t *sp = reinterpret_cast<const u32x4_t *>(reinterpret_cast<const uint16_t *>(a.pool.k_scales) +
+                                                              int8_scale_index(bh, 8 * (g & 1), BT));
+        sreg[i][0] = sp[0];
+        sreg[i][1] = sp[1];
+      }
+      if constexpr (FMT == kFp8) {
+        const uint2 t = *reinterpret_cast<const uint2 *>(reinterpret_cast<const uint32_t *>(a.pool.k_scales) +
+                                                         fp8_scale_index(bh));
+        sreg[i][0][0] = t.x;
+        sreg[i][0][1] = t.y;
+      }
+#pragma unroll
+      for (int d = 0; d < ND; d++)
+        vr[i][d] = __builtin_nontemporal_load(reinterpret_cast<const vword_t *>(vb + 16 * d * BT * ES));
+    }
+  };
+
+  // scores of the unit in kr (raw, over this lane's keys: key_of below)
+  float sc[4 * NT];
+  auto scores = [&]() __attribute__((always_inline)) {
+    f32x4_t acc[NT];
+#pragma unroll
+    for (int j = 0; j < NT; j++) acc[j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int x = 0; x < KL; x++)
+#pragma unroll
+      for (int j = 0; j < NT; j++) {
+        if constexpr (Q8) {
+          acc[j] = mfma16<OP>(codes8<FMT>(kr[j][x][0], kr[j][x][1]), qb[2 * x], acc[j]);
+          acc[j] = mfma16<OP>(codes8<FMT>(kr[j][x][2], kr[j][x][3]), qb[2 * x + 1], acc[j]);
+        } else {
+          acc[j] = mfma16<OP>(kr[j][x], qb[x], acc[j]);
+        }
+      }
+#pragma unroll
+    for (int x = 0; x < 4 * NT; x++) sc[x] = acc[x >> 2][x & 3];
+  };
+  // position of score x (0 .. 4 NT - 1) of this lane in the unit
+  auto key_of = [&](int x) __attribute__((always_inline)) {
+    return 32 * (x >> 3) + 8 * g + (x & 7);
+  };
+
+  // f32 scale (0: K, 1: V) of score x's key
+  auto scale_of = [&](int x, int tensor) __attribute__((always_inline)) {
+    if constexpr (FMT == kInt8) {
+      const uint32_t pair = sreg[x >> 3][(x >> 2) & 1][x & 3];
+      return f16_bits_to_f32(tensor ? pair >> 16 : pair & 0xffffu);
+    } else {
+      return __uint_as_float(sreg[x >> 3][0][tensor]);
+    }
+  };
+
+  u32x4_t pb[NS][PARTS];
+  auto softmax = [&](int u, uint32_t vmiss) __attribute__((always_inline)) {
+    const int base = u * UK;
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int x = 0; x < 4 * NT; x++) {
+      float s = sc[x];
+      if constexpr (Q8) s *= scale_of(x, 0);
+      sc[x] = s;
+    }
+#pragma unroll
+    for (int x = 0; x < 4 * NT; x++) {
+      const int p = base + key_of(x);
+      const bool miss = vmiss & (1u << (x >> 3));
+      const bool on = (p >= my_lo) & (p <= my_pos) & (!miss | zero_bad);
+      const float s = miss ? 0.0f : sc[x];
+      nonfinite |= on & !(fabsf(s * c_nat) < INFINITY);
+      sc[x] = on ? s * c : -INFINITY;
+      tmax = fmaxf(tmax, sc[x]);
+    }
+    tmax = fmaxf(tmax, xor16_other(tmax, lane));
+    tmax = fmaxf(tmax, xor32_other(tmax, lane));
+    // lazy rescale: the reference max moves only when a row's max grows by more than 8
+    const bool grow = tmax > m_run + 8.0f;  // true on a row's first finite unit
+    if (__any(grow)) {
+      const float nm = grow ? tmax : m_run;
+      const float alpha = grow ? fast_exp2(m_run - nm) : 1.0f;
+      m_run = nm;
+      l_run *= alpha;
+#pragma unroll
+      for (int d = 0; d < ND; d++) oacc[d] *= alpha;
+    }
+    const float mref = m_run == -INFINITY ? 0.0f : m_run;
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+      float p[8];
+#pragma unroll
+      for (int x = 0; x < 8; x++) {
+        p[x] = fast_exp2(sc[8 * s + x] - mref);
+        if constexpr (PARTS > 1 || Q8) l_run += p[x];
+        // the scale of a slot that is not attended may be anything
+        if constexpr (Q8)
+          p[x] = (sc[8 * s + x] == -INFINITY) | ((vmiss >> s & 1u) != 0) ? 0.0f : p[x] * scale_of(8 * s + x, 1);
+      }
+#pragma unroll
+      for (int q = 0; q < PARTS; q++) {
+#pragma unroll
+        for (int x = 0; x < 4; x++) {
+          const uint32_t w = pack_16<OP>(p[2 * x], p[2 * x + 1]);
+          pb[s][q][x] = w;
+          if constexpr (PARTS == 1 && !Q8) l_run = dot2_ones_16<OP>(w, l_run);
+          if (q + 1 < PARTS) {  // the rest of the weight, exactly
+            if constexpr (OP == kF16) {
+              p[2 * x] -= f16_bits_to_f32(w & 0xffffu);
+              p[2 * x + 1] -= f16_bits_to_f32(w >> 16);
+            } else {
+              p[2 * x] -= bf16_lo(w);
+              p[2 * x + 1] -= bf16_hi(w);
+            }
+          }
+        }
+      }
+    }
+  };
+  auto accumulate = [&](int u, uint32_t vmiss) __attribute__((always_inline)) {
+    const int base = u * UK;
+    // V slots outside the attended positions may hold anything (0 * NaN is NaN)
+    constexpr int PW = Q8 ? 4 : 2;  // elements per word
+    vword_t vmask[NS];
+#pragma unroll
+    for (int i = 0; i < NS; i++) {
+      const int p0 = base + 32 * i + 8 * g;
+      const bool miss = vmiss & (1u << i);
+#pragma unroll
+      for (int w = 0; w < 2 * ES; w++) {
+        uint32_t mask = 0;
+#pragma unroll
+        for (int e = 0; e < PW; e++) {
+          const int p = p0 + PW * w + e;
+          mask |= !miss & (p >= tile_lo0) & (p < sq.ctx) ? (Q8 ? 0xffu : 0xffffu) << (32 / PW * e) : 0u;
+        }
+        vmask[i][w] = mask;
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+      constexpr int GRP = 4;  // output tiles whose independent products hide each other's latency
+#pragma unroll
+      for (int d0 = 0; d0 < ND; d0 += GRP) {
+        u32x4_t va[GRP];
+#pragma unroll
+        for (int d = 0; d < GRP; d++) {
+          const vword_t v = vr[s][d0 + d] & vmask[s];
+          if constexpr (Q8) va[d] = codes8<FMT>(v[0], v[1]);
+          else va[d] = v;
+        }
+#pragma unroll
+        for (int q = 0; q < PARTS; q++)
+#pragma unroll
+          for (int d = 0; d < GRP; d++) oacc[d0 + d] = mfma16<OP>(va[d], pb[s][q], oacc[d0 + d]);
+      }
+    }
+  };
+
+  if (n > 0) {
+    Entries e;
+    uint32_t vmiss = 0;
+    int u = ub + wave;
+    fetch(u, e);
+    load_k(u, e);
+    __builtin_amdgcn_sched_barrier(0);  // K before V, as in the loop
+    load_v(u, e, vmiss);
+    fetch(n > 1 ? u + WAVES : u, e);
+    asm volatile("");  // keeps the compiler from merging these loads with the loop's
+    // The last unit is peeled off: loads under a condition would make the compiler
+    // wait for every load in flight.
+    for (int k = 0; k + 1 < n; k++) {
+      bad |= vmiss != 0;
+      scores();
+      softmax(u, vmiss);
+      // the next K loads into the registers this unit's scores have read, and nothing of
+      // P V (which waits for V) moves above them
+      __builtin_amdgcn_sched_barrier(0);
+      load_k(u + WAVES, e);
+      __builtin_amdgcn_sched_barrier(0);
+      accumulate(u, vmiss);
+      __builtin_amdgcn_sched_barrier(0);
+      load_v(u + WAVES, e, vmiss);
+      u += WAVES;
+      fetch(k + 2 < n ? u + WAVES : u, e);
+    }
+    bad |= vmiss != 0;
+    scores();
+    softmax(u, vmiss);
+    accumulate(u, vmiss);
+  }
+  if (__any(bad) && lane == 0) atomicOr(a.err, kErrBadBlock);
+  if (a.flag_nonfinite && __any(nonfinite) && lane == 0) atomicOr(a.err, kErrNonFinite);
+
+  // ---- merge the four wavefronts ----
+  __shared__ __attribute__((aligned(16))) float s_o[WAVES][TILE][D];
+  __shared__ float s_m[WAVES][TILE], s_l[WAVES][TILE];
+  l_run += xor16_other(l_run, lane);
+  l_run += xor32_other(l_run, lane);
+  if (g == 0) {
+    s_m[wave][col] = m_run;
+    s_l[wave][col] = l_run;
+  }
+#pragma unroll
+  for (int d = 0; d < ND; d++) *reinterpret_cast<f32x4_t *>(&s_o[wave][col][16 * d + 4 * g]) = oacc[d];
+  __syncthreads();
+  const int live = min(TILE, rows - row0);
+  for (int i = tid; i < live * (D / 4); i += 64 * WAVES) {
+    const int r = i / (D / 4);
+    const int d = 4 * (i % (D / 4));
+    const float mm = fmaxf(fmaxf(s_m[0][r], s_m[1][r]), fmaxf(s_m[2][r], s_m[3][r]));
+    const float mref = mm == -INFINITY ? 0.0f : mm;
+    float ll = 0.0f;
+    f32x4_t oo = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) {
+      const float f = fast_exp2(s_m[w][r] - mref);
+      ll += s_l[w][r] * f;
+      oo += *reinterpret_cast<const f32x4_t *>(&s_o[w][r][d]) * f;
+    }
+    const int pr = row0 + r;
+    const size_t orow = (size_t)(sq.c0 + pr / G) * a.q_heads + kvh * G + pr % G;
+    if (sq.n_splits == 1) {
+      const float inv = ll > 0.0f ? 1.0f / ll : (ll == 0.0f ? 0.0f : ll);
+      const size_t o = orow * D + d;
+#pragma unroll
+      for (int x = 0; x < 4; x++) a.out[o + x] = f32_to_bf16_rne(gated(oo[x] * inv, a.gate, o + x));
+    } else {
+      const size_t p = orow * a.max_splits + split;
+      *reinterpret_cast<f32x4_t *>(&a.ws_o[p * D + d]) = oo;
+      if (d == 0) a.ws_ml[p] = make_float2(mm, ll);
+    }
+  }
+}
+
+// Merge of the n <= N splits of one (query row, head): every partial row in flight at
+// once, the (max, sum) pairs one per lane, split weights through v_readlane.
+template <int D, int N>
+__device__ __forceinline__ void rows_merge(const RowsArgs &a, size_t orow, int last, int d) {
+  const size_t p0 = orow * a.max_splits;
+  float o_sp[N];
+#pragma unroll
+  for (int i = 0; i < N; i++) o_sp[i] = a.ws_o[(p0 + min(i, last)) * D + d];
+  const int li = d & 63;
+  const float2 ml = a.ws_ml[p0 + min(li, last)];
+  const float mx = li <= last ? ml.x : -INFINITY;
+  float mm = fmaxf(mx, dpp<0xB1>(mx));
+  mm = fmaxf(mm, dpp<0x4E>(mm));
+  mm = fmaxf(mm, dpp<0x141>(mm));
+  mm = fmaxf(mm, dpp<0x140>(mm));
+  mm = fmaxf(mm, xor16_other(mm, li));
+  mm = fmaxf(mm, xor32_other(mm, li));
+  const float mref = (mm == -INFINITY) ? 0.0f : mm;
+  const float f = li <= last ? fast_exp2(mx - mref) : 0.0f;
+  float ll = row_sum16(f * ml.y);
+  ll += xor16_other(ll, li);
+  ll += xor32_other(ll, li);
+  float oo = 0.0f;
+#pragma unroll
+  for (int i = 0; i < N; i++) oo += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), i)) * o_sp[i];
+  const float inv = ll > 0.0f ? 1.0f / ll : (ll == 0.0f ? 0.0f : ll);
+  a.out[orow * D + d] = f32_to_bf16_rne(gated(oo * inv, a.gate, orow * D + d));
+}
+
+template <int D, int UK>
+__global__ __launch_bounds__(D) void paged_rows_merge_kernel(const RowsArgs a) {
+  const int b = blockIdx.y;
+  const SeqSplit sq = seq_split<UK>(a, b);
+  const int tok = blockIdx.x / a.q_heads;
+  if (sq.skip || tok >= sq.chunk || sq.n_splits <= 1) return;
+  const size_t orow = (size_t)sq.c0 * a.q_heads + blockIdx.x;
+  const int last = sq.n_splits - 1;
+  const int d = threadIdx.x;
+  if (last < 8) return rows_merge<D, 8>(a, orow, last, d);
+  if (last < 16) return rows_merge<D, 16>(a, orow, last, d);
+  if (last < 32) return rows_merge<D, 32>(a, orow, last, d);
+  return rows_merge<D, kRowsMaxSplits>(a, orow, last, d);
+}
+
+template <int D, int FMT, int PARTS>
+hipError_t launch_rows_t(const RowsArgs &a, int max_rows, hipStream_t s) {
+  const int tiles = (max_rows * (a.q_heads / a.pool.kv_heads) + TILE - 1) / TILE;
+  hipLaunchKernelGGL((paged_rows_kernel<D, FMT, PARTS>), dim3(a.max_splits, a.pool.kv_heads * tiles, a.num_seqs),
+                     dim3(64 * WAVES), 0, s, a);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || a.max_splits <= 1) return e;
+  hipLaunchKernelGGL((paged_rows_merge_kernel<D, kUnitKeys<D>>), dim3(max_rows * a.q_heads, a.num_seqs), dim3(D),
+                     0, s, a);
+  return hipGetLastError();
+}
+
+template <int D>
+hipError_t launch_rows_d(const RowsArgs &a, int max_rows, bool exact_weights, hipStream_t s) {
+  switch (a.pool.format) {
+    case kBf16:
+      return exact_weights ? launch_rows_t<D, kBf16, 3>(a, max_rows, s) : launch_rows_t<D, kBf16, 1>(a, max_rows, s);
+    case kF16:
+      return exact_weights ? launch_rows_t<D, kF16, 3>(a, max_rows, s) : launch_rows_t<D, kF16, 1>(a, max_rows, s);
+    case kInt8:
+      return launch_rows_t<D, kInt8, 3>(a, max_rows, s);
+    case kFp8:
+      return launch_rows_t<D, kFp8, 3>(a, max_rows, s);
+  }
+  return hipErrorInvalidValue;
+}
+
+}  // namespace
+
+int rows_unit_keys(int head_dim) { return head_dim == 256 ? 32 : 64; }
+
+hipError_t launch_rows(const RowsArgs &a, int max_rows, bool exact_weights, hipStream_t s) {
+  if (a.max_splits < 1 || a.max_splits > kRowsMaxSplits || max_rows < 1) return hipErrorInvalidValue;
+  return a.pool.head_dim == 256 ? launch_rows_d<256>(a, max_rows, exact_weights, s)
+                                : launch_rows_d<128>(a, max_rows, exact_weights, s);
+}
+
+}  // namespace llh

@@ -1,0 +1,168 @@
+"""The packed-row kernel (rows.hip): decode steps at head_dim 128 / 256 outside the tuned
+kernels' shapes and short prefill chunks, against the oracle's per-head loop (crates/llm-backend/src/core/
+native_attention.rs:707-773) on the pool the GPU holds.
+
+It keeps f32 softmax weights, so its outputs are held to more than the parity bar: the
+bf16 rounding of the f32 result (2^-9 of the value; 2^-8 allowed) plus 2e-5 for the f32
+sums (scores of a few units: 2^-24 x about 10 terms' error, times values up to 5)."""
+import math
+
+import numpy as np
+import pytest
+
+import llm_hip
+import oracle
+from helpers import from_dev_bf16, to_dev
+from llm_hip import workloads
+from test_gpu_decode import build_case, oracle_decode
+
+pytestmark = pytest.mark.gpu
+
+BT = 16
+FMTS = {"bf16": llm_hip.KV_BF16, "f16": llm_hip.KV_F16, "int8": llm_hip.KV_INT8, "fp8": llm_hip.KV_FP8_E4M3}
+# lengths at the edges of blocks, of units of 32 and 64 keys, of one and several splits
+EDGES = [0, 1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 129, 255, 256, 257, 511, 700]
+
+
+def assert_f32_weights(out, ref, what):
+    g = oracle.bf16_to_f32(out.ravel())
+    r = ref.ravel()
+    bad = ~(np.abs(g - r) <= np.abs(r) * 2.0**-8 + 2e-5)
+    assert not bad.any(), f"{what}: {bad.sum()} of {r.size}, worst {np.abs(g - r)[bad].max():.3e}"
+
+
+def decode(ctx, pool, lens, tables, q, Hq, D, window, scale, gate=None, noalloc=False):
+    import torch
+
+    out = torch.full((len(lens) * Hq * D,), 0x7FC0, dtype=torch.int16, device="cuda")
+    desc = ctx.decode_desc(to_dev(lens), to_dev(tables), Hq, int(lens.max()), window,
+                           gate=None if gate is None else to_dev(gate))
+    before = ctx.metrics()["generic_decode_calls"]
+    (ctx.paged_decode_noalloc if noalloc else ctx.paged_decode)(pool, desc, to_dev(q), out, scale)
+    torch.cuda.synchronize()
+    assert ctx.metrics()["generic_decode_calls"] == before + 1
+    return from_dev_bf16(out)
+
+
+@pytest.mark.parametrize("window", [0, 1, 100])
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("D,Hq,Hkv", [(256, 8, 4), (256, 20, 1), (256, 6, 2), (128, 12, 4), (128, 34, 2)])
+def test_rows_decode(ctx, D, Hq, Hkv, fmt, window):
+    """Groups of 2, 20 (two tiles), 3 and 17; every edge length, empty included."""
+    lens = np.array(EDGES, np.int32)
+    batch = workloads.paged_batch(lens, BT, 0.10, 7 + D + Hq)
+    pool, q = build_case(ctx, batch, Hq, Hkv, FMTS[fmt], 50 + Hq, head_dim=D)
+    scale = 1.0 / math.sqrt(D)
+    out = decode(ctx, pool, lens, batch.tables, q, Hq, D, window, scale)
+    assert ctx.device_errors() == 0, ctx.last_error()
+    ref = oracle_decode(pool, batch, FMTS[fmt], Hq, Hkv, window, q, scale, head_dim=D)
+    assert_f32_weights(out, ref, f"D{D} {Hq}/{Hkv} {fmt} W{window}")
+    # the no-allocation entry gives the same bits from its own scratch
+    assert np.array_equal(out, decode(ctx, pool, lens, batch.tables, q, Hq, D, window, scale, noalloc=True))
+
+
+@pytest.mark.parametrize("fmt", ["int8", "fp8"])
+def test_rows_decode_many_splits_and_gate(ctx, fmt):
+    """The head_dim-256 group of 8 over quantised blocks, gated: one long sequence (the
+    merge's 64 splits, several units per wavefront) beside short ones."""
+    D, Hq, Hkv = 256, 16, 2
+    lens = np.array([17000, 3, 4000], np.int32)
+    batch = workloads.paged_batch(lens, BT, 0.10, 11)
+    pool, q = build_case(ctx, batch, Hq, Hkv, FMTS[fmt], 12, head_dim=D)
+    gate = oracle.normal_bf16(99, q.size)
+    out = decode(ctx, pool, lens, batch.tables, q, Hq, D, 0, 0.0625, gate=gate)
+    assert ctx.device_errors() == 0, ctx.last_error()
+    ref = oracle_decode(pool, batch, FMTS[fmt], Hq, Hkv, 0, q, 0.0625, head_dim=D)
+    g = oracle.bf16_to_f32(gate).astype(np.float64)
+    assert_f32_weights(out, (ref.ravel() / (1.0 + np.exp(-g))).astype(np.float32), fmt)
+
+
+def test_rows_decode_flags(ctx):
+    """The reference-order kernel's flags: a block outside the pool scores 0 with a zero
+    value, a non-finite score and a length beyond the call's bound are flagged."""
+    D, Hq, Hkv = 256, 8, 4
+    lens = np.array([40, 200], np.int32)
+    batch = workloads.paged_batch(lens, BT, 0.10, 21)
+    pool, q = build_case(ctx, batch, Hq, Hkv, llm_hip.KV_BF16, 22, head_dim=D)
+    tables = batch.tables.copy()
+    tables[1, 3] = batch.n_blocks + 4
+    out = decode(ctx, pool, lens, tables, q, Hq, D, 0, 0.0625)
+    assert ctx.device_errors() == llm_hip.ERR_FLAG_BAD_BLOCK
+    assert np.array_equal(out, decode(ctx, pool, lens, tables, q, Hq, D, 0, 0.0625))
+    ctx.device_errors()
+    opool = oracle.Pool.from_raw(llm_hip.KV_BF16, BT, Hkv, D, batch.n_blocks, pool.raw())
+    _, k, v = opool.gather_f32(batch.tables[1], 0, 200)
+    k, v = (x.reshape(200, Hkv, D).astype(np.float64) for x in (k, v))
+    k[48:64] = v[48:64] = 0.0
+    qf = oracle.bf16_to_f32(q).reshape(2, Hq, D)[1].astype(np.float64)
+    for h in range(Hq):
+        s = k[:, h // 2] @ qf[h] * 0.0625
+        p = np.exp(s - s.max())
+        ref = (p / p.sum()) @ v[:, h // 2]
+        assert_f32_weights(out.reshape(2, Hq, D)[1, h], ref.astype(np.float32), f"bad block, head {h}")
+    qi = q.copy()
+    qi.reshape(2, Hq, D)[1, 5, 7] = 0x7F80  # an infinite query element
+    decode(ctx, pool, lens, batch.tables, qi, Hq, D, 0, 0.0625)
+    assert ctx.device_errors() & llm_hip.ERR_FLAG_NON_FINITE
+    import torch
+
+    desc = ctx.decode_desc(to_dev(lens), to_dev(batch.tables), Hq, 100)  # 200 > 100
+    o = torch.zeros(2 * Hq * D, dtype=torch.int16, device="cuda")
+    ctx.paged_decode(pool, desc, to_dev(q), o, 0.0625)
+    torch.cuda.synchronize()
+    assert ctx.device_errors() == llm_hip.ERR_FLAG_TOO_MANY_SPLITS
+
+
+@pytest.mark.parametrize("window", [0, 33])
+@pytest.mark.parametrize("D,Hq,Hkv,fmt", [(128, 16, 8, "bf16"), (128, 8, 1, "f16"), (128, 6, 2, "int8"),
+                                          (128, 8, 2, "fp8"), (256, 16, 2, "bf16"), (256, 8, 4, "f16")])
+def test_rows_prefill(ctx, opts, D, Hq, Hkv, fmt, window):
+    """Short ragged chunks (an empty one included) over prefixes at unit and split edges: the
+    packed-row kernel, the 128-row-tile kernel on the same call, and -- under graph capture,
+    where no scratch may be taken -- the latter again; all against the oracle."""
+    import torch
+
+    from helpers import assert_parity
+
+    chunk = [8, 0, 1, 13, 5]
+    prefix = [0, 40, 2100, 243, 507]
+    lens = np.array([p + c for p, c in zip(prefix, chunk)], np.int32)
+    batch = workloads.paged_batch(lens, BT, 0.10, 31)
+    pool, _ = build_case(ctx, batch, Hq, Hkv, FMTS[fmt], 32, head_dim=D)
+    starts = np.concatenate([[0], np.cumsum(chunk)]).astype(np.int32)
+    T = int(starts[-1])
+    q = oracle.normal_bf16(35, T * Hq * D)
+    gate = oracle.normal_bf16(36, T * Hq * D)
+    scale = 1.0 / math.sqrt(D)
+    keep = [to_dev(a) for a in (starts, batch.seq_lens, batch.tables, q, gate)]
+    out = torch.zeros(T * Hq * D, dtype=torch.int16, device="cuda")
+    desc = ctx.prefill_desc(keep[0], keep[1], keep[2], Hq, max(chunk), window, total_q_rows=T, gate=keep[4])
+    opool = oracle.Pool.from_raw(FMTS[fmt], BT, Hkv, D, batch.n_blocks, pool.raw())
+    st, ref = opool.prefill(Hq, starts, batch.seq_lens, batch.tables, window, q, scale, threads=16)
+    assert st == oracle.OK
+    ref = ref.ravel() / (1.0 + np.exp(-oracle.bf16_to_f32(gate).astype(np.float64)))
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        ctx.paged_prefill(pool, desc, keep[3], out, scale, stream=stream)
+    stream.synchronize()
+    rows = from_dev_bf16(out)
+    assert_parity(rows, ref.astype(np.float32), what="packed rows")
+    opts(llm_hip.OPT_PREFILL_HEADS_PER_WG, 1)
+    out.zero_()
+    ctx.paged_prefill(pool, desc, keep[3], out, scale)
+    torch.cuda.synchronize()
+    tiles = from_dev_bf16(out)
+    assert_parity(tiles, ref.astype(np.float32), what="128-row tiles")
+    opts(llm_hip.OPT_PREFILL_HEADS_PER_WG, 0)
+    bytes0 = ctx.metrics()["workspace_bytes"]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        ctx.paged_prefill(pool, desc, keep[3], out, scale, stream=torch.cuda.current_stream())
+    assert ctx.metrics()["workspace_bytes"] == bytes0
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_parity(from_dev_bf16(out), ref.astype(np.float32), what="captured")
+    assert ctx.device_errors() == 0, ctx.last_error()
+    ctx.release_stream(stream)
