@@ -138,7 +138,8 @@ typedef struct llh_metrics {
   uint64_t shape_errors;
   uint64_t stream_decode_calls; /* decode calls that ran the persistent stream kernel */
   uint64_t trait_tuned_calls;   /* trait-mirror attention calls served by the tuned decode kernels */
-  uint64_t generic_prefill_calls; /* prefill calls that ran the element-wise kernel */
+  uint64_t generic_prefill_calls; /* prefill calls outside the tile kernels' shapes: int8 / fp8 blocks at
+                                     head_dim 256 (packed rows), else the element-wise kernel */
   uint64_t fused_append_calls;    /* llh_paged_decode_append calls served by one launch */
   uint64_t stream_slots;          /* streams holding a workspace slot (scratch and error word) now */
   uint64_t workspace_bytes;       /* device bytes of those slots' scratch now */
@@ -325,10 +326,13 @@ typedef struct llh_prefill_desc {
 
 /* d_q, d_out: [total_q_rows][Hq][head_dim] bf16 (2-byte aligned).  Every pool
  * format: int8 / fp8 blocks are dequantised, so the result is attention over
- * the dequantised cache (layer.rs:650-656).  head_dim 128 with 16-token blocks
- * and 16-byte aligned rows runs the MFMA kernel (codes * scale rounded to bf16
- * as the key/value tiles are staged); every other shape with head_dim <= 512
- * runs an element-wise kernel (sequential f32 dot products, online softmax in
+ * the dequantised cache (layer.rs:650-656).  head_dim 128 and 256 with 16-token
+ * blocks and 16-byte aligned rows run MFMA kernels: 128-row tiles (int8 / fp8 at
+ * head_dim 128: codes * scale rounded to bf16 as the key/value tiles are staged),
+ * or, for calls of few rows and for int8 / fp8 at head_dim 256, packed 16-row
+ * tiles over split keys, whose partial results live in the stream's workspace (a
+ * stream under capture gets none: its calls do not split).  Every other shape with
+ * head_dim <= 512 runs an element-wise kernel (sequential f32 dot products, online softmax in
  * f32); head_dim > 512 returns LLH_ERR_UNSUPPORTED. */
 int llh_paged_prefill(llh_ctx *ctx, const llh_kv_pool *pool, const llh_prefill_desc *desc, const void *d_q,
                       void *d_out, float score_scale, void *stream);

@@ -239,7 +239,6 @@ bool prefill_takes_rows(const llh_ctx *ctx, const PoolView &pv, const llh_prefil
   if (d->max_chunk_len <= 0 || ctx->opt(LLH_OPT_PREFILL_HEADS_PER_WG)) return false;
   const int group = d->num_q_heads / pv.kv_heads;
   const long long tiles = ((long long)d->max_chunk_len * group + 15) / 16 * pv.kv_heads;
-  if (tiles > 65535 || d->num_seqs > 65535) return false;  // grid dimensions
   const bool wide = pv.head_dim == kD256HeadDim;
   const long long wgs = ((long long)d->max_chunk_len + 127) / 128 * d->num_seqs *
                         (wide || group % 2 ? d->num_q_heads : d->num_q_heads / 2);
@@ -1121,11 +1120,19 @@ int llh_paged_prefill(llh_ctx *ctx, const llh_kv_pool *pool, const llh_prefill_d
   hipError_t e;
   WsLease lease;
   SplitRows sr{};
-  bool rows = (fast || fast256) && prefill_takes_rows(ctx, pv, desc);
+  // int8 / fp8 blocks at head_dim 256 always run the packed-row kernel, unsplit where no
+  // scratch may be taken
+  const bool rows_only = tuned_shape && !fast && !fast256 && pv.format != LLH_KV_INT8_ROW &&
+                         pv.head_dim == kD256HeadDim && desc->max_chunk_len > 0;
+  bool rows = rows_only || ((fast || fast256) && prefill_takes_rows(ctx, pv, desc));
   if (rows) {
     sr = split_prefill_rows(ctx, pv, desc);
-    rows = lease.try_acquire(ctx, static_cast<hipStream_t>(stream), sr.bytes);
+    if (!lease.try_acquire(ctx, static_cast<hipStream_t>(stream), sr.bytes)) {
+      rows = rows_only;
+      sr.max_splits = 1;
+    }
   }
+  if (rows_only) ctx->generic_prefill_calls++;
   if (rows) {
     RowsArgs r{};
     r.pool = pv;
@@ -1134,8 +1141,10 @@ int llh_paged_prefill(llh_ctx *ctx, const llh_kv_pool *pool, const llh_prefill_d
     r.chunk_starts = a.chunk_starts;
     r.context_lens = a.context_lens;
     r.tables = a.tables;
-    r.ws_o = reinterpret_cast<float *>(lease.base() + sr.o_off);
-    r.ws_ml = reinterpret_cast<float2 *>(lease.base());
+    if (sr.max_splits > 1) {
+      r.ws_o = reinterpret_cast<float *>(lease.base() + sr.o_off);
+      r.ws_ml = reinterpret_cast<float2 *>(lease.base());
+    }
     r.err = a.err;
     r.num_seqs = a.num_seqs;
     r.q_heads = a.q_heads;

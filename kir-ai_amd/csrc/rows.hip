@@ -13,6 +13,7 @@
 //    blocks): other group sizes, and int8 / fp8 blocks at head_dim 256 -- the
 //    contract of decode_generic_kernel (f32 softmax weights, non-finite scores
 //    flagged, a block outside the pool scoring 0);
+//  * prefill over int8 / fp8 blocks at head_dim 256, again with f32 weights;
 //  * prefill calls of few rows, where a 128-row tile per head would leave most of the
 //    chip idle (contract of paged_prefill_kernel: positions [lo(pos), pos]).
 // Reference: crates/llm-backend/src/core/native_attention.rs:356-464,707-773.
@@ -35,7 +36,9 @@
 // is each K / V byte once per 16-row tile.  Measured on MI355X: decode, 16 x U[256, 4096]
 // tokens, Hq16 / Hkv2, head_dim 256, fp8: 3139 us on the element-wise kernel, 19.7 us here
 // (32 MB, 1.6 TB/s); a chunk of 8 tokens over 4099 cached ones, Hq16 / Hkv8, head_dim 128,
-// bf16: 119.5 us on 128-row tiles, 12.6 us here (17 MB, 1.3 TB/s).
+// bf16: 119.5 us on 128-row tiles, 12.6 us here (17 MB, 1.3 TB/s); 2 x (1024 + 250) tokens,
+// Hq16 / Hkv2, head_dim 256, int8: 10.6 ms element-wise, 48 us here (197 TFLOP/s: the code
+// conversions, repeated by every 16-row tile, bound it).
 #include "wave_ops.h"
 
 namespace llh {
@@ -126,10 +129,10 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 && is16(FMT) ? 1 : 2) void pag
 
   const int Hkv = a.pool.kv_heads;
   const int G = a.q_heads / Hkv;
-  const int split = blockIdx.x;
-  const int kvh = blockIdx.y % Hkv;
-  const int tile = blockIdx.y / Hkv;
-  const int b = blockIdx.z;
+  const int split = blockIdx.x % a.max_splits;
+  const int kvh = blockIdx.x / a.max_splits % Hkv;
+  const int tile = blockIdx.x / a.max_splits / Hkv;
+  const int b = blockIdx.y;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -534,7 +537,7 @@ __global__ __launch_bounds__(D) void paged_rows_merge_kernel(const RowsArgs a) {
 template <int D, int FMT, int PARTS>
 hipError_t launch_rows_t(const RowsArgs &a, int max_rows, hipStream_t s) {
   const int tiles = (max_rows * (a.q_heads / a.pool.kv_heads) + TILE - 1) / TILE;
-  hipLaunchKernelGGL((paged_rows_kernel<D, FMT, PARTS>), dim3(a.max_splits, a.pool.kv_heads * tiles, a.num_seqs),
+  hipLaunchKernelGGL((paged_rows_kernel<D, FMT, PARTS>), dim3(a.max_splits * a.pool.kv_heads * tiles, a.num_seqs),
                      dim3(64 * WAVES), 0, s, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || a.max_splits <= 1) return e;

@@ -115,7 +115,8 @@ def test_rows_decode_flags(ctx):
 
 @pytest.mark.parametrize("window", [0, 33])
 @pytest.mark.parametrize("D,Hq,Hkv,fmt", [(128, 16, 8, "bf16"), (128, 8, 1, "f16"), (128, 6, 2, "int8"),
-                                          (128, 8, 2, "fp8"), (256, 16, 2, "bf16"), (256, 8, 4, "f16")])
+                                          (128, 8, 2, "fp8"), (256, 16, 2, "bf16"), (256, 8, 4, "f16"),
+                                          (256, 16, 2, "int8"), (256, 12, 4, "fp8")])
 def test_rows_prefill(ctx, opts, D, Hq, Hkv, fmt, window):
     """Short ragged chunks (an empty one included) over prefixes at unit and split edges: the
     packed-row kernel, the 128-row-tile kernel on the same call, and -- under graph capture,
@@ -147,6 +148,8 @@ def test_rows_prefill(ctx, opts, D, Hq, Hkv, fmt, window):
     stream.synchronize()
     rows = from_dev_bf16(out)
     assert_parity(rows, ref.astype(np.float32), what="packed rows")
+    if D == 256 and fmt in ("int8", "fp8"):  # no tile kernel: packed rows always, f32 weights
+        assert_f32_weights(rows, ref.astype(np.float32), "packed rows")
     opts(llm_hip.OPT_PREFILL_HEADS_PER_WG, 1)
     out.zero_()
     ctx.paged_prefill(pool, desc, keep[3], out, scale)
