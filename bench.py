@@ -423,11 +423,11 @@ def measure_neighbours(ctx, steps: int, warmup: int) -> list:
     # prefill: C3's 8 x 512-token chunks, whole 16-token blocks (llh_kv_write_blocks), and
     # the same chunks at the Qwen3.6 shape (head_dim 256, Hkv 2, bf16)
     for fmt, nm, hd, H, shape, kern in (
-            (llm_hip.KV_BF16, "bf16", D, 4, "C3", "write_blocks_d128_kernel"),
-            (llm_hip.KV_INT8, "int8", D, 4, "C3", "write_blocks_d128_kernel"),
-            (llm_hip.KV_FP8_E4M3, "fp8", D, 4, "C3", "write_blocks_d128_kernel"),
-            (llm_hip.KV_F16, "fp16", D, 4, "C3", "write_blocks_d128_kernel"),
-            (llm_hip.KV_BF16, "bf16, head_dim 256", 256, 2, "Q36", "write_blocks16_d256_kernel")):
+            (llm_hip.KV_BF16, "bf16", D, 4, "C3", "write_blocks_vec_kernel"),
+            (llm_hip.KV_INT8, "int8", D, 4, "C3", "write_blocks_vec_kernel"),
+            (llm_hip.KV_FP8_E4M3, "fp8", D, 4, "C3", "write_blocks_vec_kernel"),
+            (llm_hip.KV_F16, "fp16", D, 4, "C3", "write_blocks_vec_kernel"),
+            (llm_hip.KV_BF16, "bf16, head_dim 256", 256, 2, "Q36", "write_blocks_vec_kernel")):
         nblk = 8 * 512 // BT
         pool = ctx.pool(fmt, BT, H, hd, 8192)
         ids = torch.randperm(8192, generator=g, device="cuda")[:nblk].to(torch.int32)

@@ -61,22 +61,38 @@ __device__ __forceinline__ uint4 bf16x8_to_f16x8(uint4 w) {
   return make_uint4(u[0], u[1], u[2], u[3]);
 }
 
-// Whole 16-token blocks of head_dim 128, every pool format but int8-row: one
-// workgroup of 256 lanes per (block, head).  Lane (t = lane / 16, c = lane % 16)
+// Max over the 2^k lanes (16 or 32) that hold one token row of Dh elements, in all of them.
+template <int Dh>
+__device__ __forceinline__ float token_max(float v) {
+  v = row16_max(v);
+  if constexpr (Dh == 256) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  }
+  return v;
+}
+
+// Whole 16-token blocks of head_dim Dh = 128 or 256, every pool format but int8-row: one
+// workgroup of 2 Dh lanes per (block, head).  Lane (t = lane / (Dh / 8), c = lane % (Dh / 8))
 // loads the 16 B of token t at dims 8c .. 8c+7 of K and of V (coalesced; fp16
 // pools convert them in registers), writes K rows straight out, and V is
 // transposed through LDS so that every lane then writes 16 B (bf16 / fp16) or
 // 8 B (int8 / fp8) of one dim row: every global access is a full,
-// coalesced vector access.  int8: the per-(token, head) scale is the 16 lanes'
+// coalesced vector access.  int8: the per-(token, head) scale is the token's lanes'
 // absmax, then the same f16 rounding and code rule as the generic kernel; fp8:
 // the per-(block, head) scale is the workgroup's absmax / 448, then the generic
-// kernel's encode, so both kernels write identical bytes.
-__global__ __launch_bounds__(256) void write_blocks_d128_kernel(const WriteBlocksArgs a) {
-  constexpr int BT = 16, Dh = 128;
+// kernel's encode, so both kernels write identical bytes.  At this size launch-bound:
+// 256 blocks, Hkv 2, head_dim 256, int8 (12.6 MB) 23.2 us on the element-wise kernel,
+// 6.8 us here (issue-bound; the head_dim-128 chunk of the same size takes the GPU 4.6 us).
+template <int Dh>
+__global__ __launch_bounds__(2 * Dh) void write_blocks_vec_kernel(const WriteBlocksArgs a) {
+  constexpr int BT = 16;
+  constexpr int LT = Dh / 8;   // lanes per token row
+  constexpr int NW = Dh / 32;  // wavefronts
   const int i = blockIdx.x;
   const int h = blockIdx.y;
   const int tid = threadIdx.x;
-  const int t = tid >> 4, c = tid & 15;
+  const int t = tid / LT, c = tid % LT;
   const int Hkv = a.pool.kv_heads;
   const int blk = a.blocks[i];
   if (blk < 0 || (int64_t)blk >= a.pool.n_blocks) {
@@ -107,7 +123,7 @@ __global__ __launch_bounds__(256) void write_blocks_d128_kernel(const WriteBlock
   }
   // quantised blocks: a NaN or an infinity in the block's rows is NonFiniteValue
   // in the reference (format.rs:713-716): flagged, and the block is left as it was.
-  // Each wave posts its verdict in LDS; the workgroup reads the four after a barrier
+  // Each wave posts its verdict in LDS; the workgroup reads them after a barrier
   // the kernel has anyway (fp8: the absmax reduction; int8: the V transpose), before
   // any global store.
   bool bad = false;
@@ -118,14 +134,19 @@ __global__ __launch_bounds__(256) void write_blocks_d128_kernel(const WriteBlock
     for (int k = 0; k < 2; k++)
       bad = bad || (u[k] & 0x7f80u) == 0x7f80u || (u[k] & 0x7f800000u) == 0x7f800000u;
   }
-  __shared__ __align__(16) uint32_t wave_bad[4];
+  __shared__ __align__(16) uint32_t wave_bad[NW];
   {
     const uint32_t wb = __any(bad) ? 1u : 0u;
     if ((tid & 63) == 0) wave_bad[tid >> 6] = wb;
   }
   const auto block_bad = [&]() {
-    const uint4 f = *reinterpret_cast<const uint4 *>(wave_bad);
-    return (f.x | f.y | f.z | f.w) != 0u;
+    uint32_t any = 0;
+#pragma unroll
+    for (int w = 0; w < NW; w += 4) {
+      const uint4 f = *reinterpret_cast<const uint4 *>(&wave_bad[w]);
+      any |= f.x | f.y | f.z | f.w;
+    }
+    return any != 0u;
   };
   __shared__ uint8_t lq[BT][Dh + 16];
   uint32_t codes[2][2];
@@ -133,7 +154,7 @@ __global__ __launch_bounds__(256) void write_blocks_d128_kernel(const WriteBlock
   if (a.pool.format == kFp8) {
     // one f32 scale per (block, head) and tensor: absmax over the block / 448,
     // codes as the generic kernel computes them (RNE e4m3 of x / scale)
-    __shared__ float red[2][4];
+    __shared__ float red[2][NW];
     float x[2][8];
     float mx[2] = {0.0f, 0.0f};
 #pragma unroll
@@ -156,7 +177,9 @@ __global__ __launch_bounds__(256) void write_blocks_d128_kernel(const WriteBlock
     }
 #pragma unroll
     for (int tensor = 0; tensor < 2; tensor++) {
-      const float m = fmaxf(fmaxf(red[tensor][0], red[tensor][1]), fmaxf(red[tensor][2], red[tensor][3]));
+      float m = 0.0f;
+#pragma unroll
+      for (int w = 0; w < NW; w++) m = fmaxf(m, red[tensor][w]);
       const float sc = m == 0.0f ? 0.0f : __fdiv_rn(m, 448.0f);
       uint32_t q[2] = {0u, 0u};
       if (sc >= 0x1p-90f) {  // block-uniform: the shared-divisor quotient (div_shared)
@@ -192,7 +215,7 @@ __global__ __launch_bounds__(256) void write_blocks_d128_kernel(const WriteBlock
       x[2 * j + 1] = bf16_to_f32((uint16_t)(u[j] >> 16));
       mx = fmaxf(mx, fmaxf(fabsf(x[2 * j]), fabsf(x[2 * j + 1])));
     }
-    mx = row16_max(mx);  // the token's 16 lanes
+    mx = token_max<Dh>(mx);
     const _Float16 s16 = (_Float16)(mx == 0.0f ? 0.0f : __fdiv_rn(mx, 127.0f));
     const float sc = (float)s16;
     uint32_t q[2] = {0u, 0u};
@@ -239,44 +262,6 @@ __global__ __launch_bounds__(256) void write_blocks_d128_kernel(const WriteBlock
 }
 
 // One workgroup per (block i, kv head).  Source rows src[i][t][h][d].
-// bf16 / fp16 pools at head_dim 256 (the Qwen3.5 / 3.6 full-attention layers), 16-token
-// blocks, 16-byte aligned rows: write_blocks_d128_kernel's 16-bit path at twice the row
-// width.  One workgroup of 512 per (block i, kv head); thread tid loads 16 bytes of token
-// tid/32's K and V rows (dims 8(tid%32) ..), stores K straight out and V through LDS, then
-// writes 16 bytes of V^T dim row tid/2 (tokens 8(tid&1) ..).
-__global__ __launch_bounds__(512) void write_blocks16_d256_kernel(const WriteBlocksArgs a) {
-  constexpr int BT = 16, Dh = 256;
-  const int i = blockIdx.x;
-  const int h = blockIdx.y;
-  const int tid = threadIdx.x;
-  const int t = tid >> 5, c = tid & 31;
-  const int Hkv = a.pool.kv_heads;
-  const int blk = a.blocks[i];
-  if (blk < 0 || (int64_t)blk >= a.pool.n_blocks) {
-    if (tid == 0) atomicOr(a.err, kErrBadBlock);
-    return;
-  }
-  const size_t bh = (size_t)blk * Hkv + h;
-  const size_t src = (((size_t)i * BT + t) * Hkv + h) * Dh + 8 * c;
-  uint4 kw = *reinterpret_cast<const uint4 *>(a.k + src);
-  uint4 vw = *reinterpret_cast<const uint4 *>(a.v + src);
-  if (a.pool.format == kF16) {  // each bf16 element widened (exact), then rounded to fp16
-    kw = bf16x8_to_f16x8(kw);
-    vw = bf16x8_to_f16x8(vw);
-  }
-  __shared__ uint16_t lv[BT][Dh + 8];
-  *reinterpret_cast<uint4 *>(reinterpret_cast<uint16_t *>(a.k_dst) + (bh * BT + t) * Dh + 8 * c) = kw;
-  *reinterpret_cast<uint4 *>(&lv[t][8 * c]) = vw;
-  __syncthreads();
-  const int d = tid >> 1, half = tid & 1;
-  uint32_t w[4];
-#pragma unroll
-  for (int j = 0; j < 4; j++)
-    w[j] = (uint32_t)lv[8 * half + 2 * j][d] | ((uint32_t)lv[8 * half + 2 * j + 1][d] << 16);
-  *reinterpret_cast<uint4 *>(reinterpret_cast<uint16_t *>(a.v_dst) + (bh * Dh + d) * BT + 8 * half) =
-      make_uint4(w[0], w[1], w[2], w[3]);
-}
-
 __global__ __launch_bounds__(256) void write_blocks_kernel(const WriteBlocksArgs a) {
   const int i = blockIdx.x;
   const int h = blockIdx.y;
@@ -901,14 +886,13 @@ hipError_t launch_write_blocks(const WriteBlocksArgs &a, hipStream_t s) {
   if (a.n <= 0) return hipSuccess;
   const bool aligned = reinterpret_cast<uintptr_t>(a.k) % 16 == 0 && reinterpret_cast<uintptr_t>(a.v) % 16 == 0 &&
                        reinterpret_cast<uintptr_t>(a.k_dst) % 16 == 0 && reinterpret_cast<uintptr_t>(a.v_dst) % 16 == 0;
-  const bool fast = a.pool.head_dim == 128 && a.pool.block_tokens == 16 && a.pool.format != kInt8Row && aligned;
-  const bool fast256 = a.pool.head_dim == 256 && a.pool.block_tokens == 16 && is16(a.pool.format) && aligned;
+  const bool fast = a.pool.block_tokens == 16 && aligned;
   if (a.pool.format == kInt8Row)
     hipLaunchKernelGGL(write_blocks_row_kernel, dim3(a.n), dim3(256), 0, s, a);
-  else if (fast)
-    hipLaunchKernelGGL(write_blocks_d128_kernel, dim3(a.n, a.pool.kv_heads), dim3(256), 0, s, a);
-  else if (fast256)
-    hipLaunchKernelGGL(write_blocks16_d256_kernel, dim3(a.n, a.pool.kv_heads), dim3(512), 0, s, a);
+  else if (fast && a.pool.head_dim == 128)
+    hipLaunchKernelGGL(write_blocks_vec_kernel<128>, dim3(a.n, a.pool.kv_heads), dim3(256), 0, s, a);
+  else if (fast && a.pool.head_dim == 256)
+    hipLaunchKernelGGL(write_blocks_vec_kernel<256>, dim3(a.n, a.pool.kv_heads), dim3(512), 0, s, a);
   else
     hipLaunchKernelGGL(write_blocks_kernel, dim3(a.n, a.pool.kv_heads), dim3(256), 0, s, a);
   return hipGetLastError();

@@ -1,5 +1,5 @@
 /* Exhaustive check of the shared-divisor quotient of the whole-block KV write kernel
- * (write_blocks_d128_kernel, kir-ai_amd/csrc/kvwrite.hip).
+ * (write_blocks_vec_kernel, kir-ai_amd/csrc/kvwrite.hip).
  *
  * The kernel quantises bf16 elements x by a scale s shared by a token row (int8: s is
  * the fp16 scale) or a whole block (fp8: s = RN(absmax / 448) for a bf16 absmax).

@@ -510,3 +510,42 @@ def test_quantised_block_write_flags_non_finite_rows(ctx, fmt, misalign):
     err = np.abs(kf.reshape(BT, Hkv, D) - x)
     # one e4m3 rounding (3 mantissa bits) or half an int8 step of the row's absmax / 127
     assert np.all(err <= 0.0625 * np.abs(x) + 0.03), err.max()
+
+
+@pytest.mark.parametrize("fmt", [llm_hip.KV_INT8, llm_hip.KV_FP8_E4M3])
+def test_block_write_quantised_head_dim_256(ctx, fmt):
+    """int8 / fp8 blocks at head_dim 256: the vector kernel's bytes equal the generic
+    kernel's (rows 2 bytes off alignment) over zero rows, rows whose maximum sits in either
+    half of the row, scales in the subnormal range, and blocks that hold a NaN or an
+    infinity (flagged and left as they were)."""
+    import torch
+
+    Hkv, Dh, n = 2, 256, 12
+    rng = np.random.default_rng(5)
+    x = rng.standard_normal((2, n, BT, Hkv, Dh)).astype(np.float32)
+    x[:, 1] = 0.0
+    x[:, 2, 3:5] = 0.0
+    x[:, 3, :, :, 0] = 90.0
+    x[:, 4, :, :, 255] = -90.0
+    x[:, 5] *= 1e-7
+    x[:, 6] *= 1e-38
+    x[0, 7, 9, 1, 200] = np.nan
+    x[1, 8, 0, 0, 130] = np.inf
+    bits = [oracle.f32_to_bf16(a.ravel()).reshape(a.shape) for a in x]
+    ids = np.arange(n, dtype=np.int32)[::-1].copy()
+    raws = []
+    for shift in (0, 1):
+        src = []
+        for b in bits:
+            flat = torch.zeros(b.size + 8, dtype=torch.int16, device="cuda")
+            flat[shift:shift + b.size] = to_dev(b).reshape(-1)
+            src.append(flat[shift:])
+        pool = ctx.pool(fmt, BT, Hkv, Dh, n)
+        zero = torch.zeros(bits[0].size, dtype=torch.int16, device="cuda")
+        ctx.write_blocks(pool, to_dev(ids), zero, zero)  # what a refused block keeps
+        ctx.write_blocks(pool, to_dev(ids), *src)
+        torch.cuda.synchronize()
+        assert ctx.device_errors() == llm_hip.ERR_FLAG_NON_FINITE
+        raws.append(pool.raw())
+    for key in raws[0]:
+        assert np.array_equal(raws[0][key], raws[1][key]), key

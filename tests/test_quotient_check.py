@@ -1,5 +1,5 @@
 """The whole-block KV write kernel's shared-divisor quotient (div_shared in
-kir-ai_amd/csrc/device_common.h, used by write_blocks_d128_kernel for int8 and fp8
+kir-ai_amd/csrc/device_common.h, used by write_blocks_vec_kernel for int8 and fp8
 pools) gives the codes of the correctly rounded division for every input it can see:
 tests/quotient_check.c runs all of them (every bf16 absmax, the scale the kernel
 derives from it, every bf16 element up to it) under IEEE and flush-to-zero
