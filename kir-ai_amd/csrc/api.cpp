@@ -168,6 +168,12 @@ int plan_stream(const llh_ctx *ctx, int format, int num_seqs, int kv_heads, int 
   return units >= kStreamMinUnitsPerWave * waves ? wgs : 0;
 }
 
+// Units up to which the packed-row kernel leaves a sequence whole: one for each of a
+// workgroup's wavefronts, or four where the call's tiles fill the chip by themselves.  (One
+// compute unit takes about 32 GB/s from memory, whatever it has in flight: 512 tokens of one
+// kv head, 256 KB, take 8 us on one and the second launch costs 4.)
+int rows_single(const llh_ctx *ctx, long long tiles) { return tiles >= ctx->cus ? 16 : 4; }
+
 // Split of the packed-row kernel (rows.hip).  A split holds at least one unit for each of
 // its four wavefronts.  Small steps take the split that gives one workgroup per compute
 // unit (two at head_dim 128): a workgroup's start and its merge cost more than a unit.
@@ -181,10 +187,11 @@ int plan_stream(const llh_ctx *ctx, int format, int num_seqs, int kv_heads, int 
 // (query row, head) pairs.
 struct SplitRows {
   int split_units;
+  int single_units;
   int max_splits;
   size_t o_off, bytes;
 };
-SplitRows split_rows(const llh_ctx *ctx, const PoolView &pv, int units, long long total, size_t out_rows,
+SplitRows split_rows(const llh_ctx *ctx, const PoolView &pv, long long tiles, int units, long long total, size_t out_rows,
                      size_t max_bytes) {
   SplitRows r{};
   const bool wide = pv.head_dim == kD256HeadDim;
@@ -196,7 +203,8 @@ SplitRows split_rows(const llh_ctx *ctx, const PoolView &pv, int units, long lon
   const int opt = ctx->opt(LLH_OPT_DECODE_SPLIT_BLOCKS);
   if (opt > 0) r.split_units = std::max(1, opt * kFastBlockTokens / rows_unit_keys(pv.head_dim));
   r.max_splits = std::min(kRowsMaxSplits, std::max(1, (units + r.split_units - 1) / r.split_units));
-  if (units <= kRowsSingleUnits) r.max_splits = 1;
+  r.single_units = rows_single(ctx, tiles);
+  if (units <= r.single_units) r.max_splits = 1;
   for (;; r.max_splits--) {
     const size_t rows = r.max_splits > 1 ? out_rows * r.max_splits : 0;
     r.o_off = align_up(rows * sizeof(float2));
@@ -219,7 +227,8 @@ SplitRows split_prefill_rows(const llh_ctx *ctx, const PoolView &pv, const llh_p
   SplitRows r{};
   r.split_units = 4;
   r.max_splits = (int)std::min<long long>({(long long)kRowsMaxSplits, std::max(1LL, slots / tiles), (units + 3) / 4});
-  if (units <= kRowsSingleUnits) r.max_splits = 1;
+  r.single_units = rows_single(ctx, tiles);
+  if (units <= r.single_units) r.max_splits = 1;
   const size_t rows = r.max_splits > 1 ? (size_t)d->total_q_rows * d->num_q_heads * r.max_splits : 0;
   r.o_off = align_up(rows * sizeof(float2));
   r.bytes = align_up(r.o_off + rows * pv.head_dim * sizeof(float));
@@ -242,6 +251,9 @@ bool prefill_takes_rows(const llh_ctx *ctx, const PoolView &pv, const llh_prefil
   const bool wide = pv.head_dim == kD256HeadDim;
   const long long wgs = ((long long)d->max_chunk_len + 127) / 128 * d->num_seqs *
                         (wide || group % 2 ? d->num_q_heads : d->num_q_heads / 2);
+  // contexts of a few tiles (by the table rows' bound) take the tile kernels as long:
+  // head_dim 256, 8 x 270 tokens 15.2 us on either, 7 x 230 13.0 against 14.0
+  if (wide && (long long)d->max_blocks_per_seq * kFastBlockTokens <= 320) return false;
   const long long per_round = wide ? 128 : is16(pv.format) ? 256 : 512;
   return tiles * d->num_seqs <= per_round * ((wgs + ctx->cus - 1) / ctx->cus);
 }
@@ -684,10 +696,49 @@ static int check_span(llh_ctx *ctx, const llh_kv_pool *pool, int32_t max_seq_len
   return LLH_OK;
 }
 
+// Whether a head_dim-128 decode step of the vector kernels' shapes runs the packed-row kernel.
+// Eight query heads per kv head fill half a matrix tile, and its MFMAs take the place of the
+// dot products that bound the vector kernels at this group size.  Measured on MI355X, Hq32 /
+// Hkv4, vector against packed rows (us): bf16 1 x 2000 12.0 / 12.0, 1 x 16000 41.4 / 14.6,
+// 4 x 4096 22.4 / 17.0, 32 x U[50, 500] 25.9 / 13.0, 32 x U[256, 4096] 54.9 / 38.8; int8
+// 1 x 16000 41.7 / 13.2, 32 x U[256, 4096] 58.5 / 35.7.  A few short sequences stay: bf16
+// 4 x U[500, 1000] 11.6 / 12.6.  At four heads per kv head it is faster where the sequences
+// are short enough for a unit or two per wavefront and fill the chip unsplit: Hq32 / Hkv8,
+// 32 x U[50, 500] bf16 16.6 / 14.1, int8 24.0 / 12.0, but 4 x U[500, 1000] 11.7 / 19.7 and
+// long ones 35.8 / 45.7 (16 x U[1000, 4000]); at two it is not (Hq16 / Hkv8, 32 x U[50, 500]
+// 12.3 / 14.0).
+static bool decode_prefers_rows(const PoolView &pv, int group, int num_seqs, int est_blocks) {
+  const long long tiles = (long long)num_seqs * pv.kv_heads;
+  if (group == 8) return tiles > 16 || est_blocks > 1024 / kFastBlockTokens + 1;
+  if (group == 4) return est_blocks <= 512 / kFastBlockTokens + 1 && tiles >= (is16(pv.format) ? 128 : 64);
+  return false;
+}
+
+// The packed-row kernel's split and workspace for a decode step; plan->bytes never shrinks.
+static void plan_rows(const llh_ctx *ctx, const PoolView &pv, const llh_decode_desc *desc, size_t max_bytes,
+                      llh::DecodePlan *plan) {
+  const int span = std::max(1, desc->window > 0 ? std::min(desc->window, desc->max_seq_len) : desc->max_seq_len);
+  const int uk = rows_unit_keys(pv.head_dim);
+  const int units = (span + uk - 1) / uk + (desc->window > 0 ? 1 : 0);  // a window may start inside a unit
+  const long long tiles = (long long)pv.kv_heads * ((plan->group + 15) / 16);
+  const long long total = desc->total_tokens_hint > 0
+                              ? tiles * ((long long)desc->total_tokens_hint / uk + desc->num_seqs)
+                              : tiles * units * desc->num_seqs;
+  const SplitRows sr = split_rows(ctx, pv, tiles * desc->num_seqs, units, total,
+                                  (size_t)desc->num_seqs * desc->num_q_heads, max_bytes);
+  plan->rows = true;
+  plan->split_units = sr.split_units;
+  plan->single_units = sr.single_units;
+  plan->max_splits = sr.max_splits;
+  plan->ml_off = 0;
+  plan->o_off = sr.o_off;
+  plan->bytes = std::max(plan->bytes, sr.bytes);
+}
+
 // Plans one decode step: validates the call, chooses the kernel and lays out
 // its workspace (offsets from the workspace base; plan->bytes in all).
 int llh::plan_decode(llh_ctx *ctx, const llh_kv_pool *pool, const llh_decode_desc *desc, const void *d_q,
-                     const void *d_out, float score_scale, DecodePlan *plan, size_t max_bytes) {
+                     const void *d_out, float score_scale, DecodePlan *plan, size_t max_bytes, bool keep_fused) {
   if (!ctx || !pool || !desc || !plan) return LLH_ERR_NULL;
   *plan = DecodePlan{};
   int st = check_desc_common(ctx, pool, desc->num_seqs, desc->num_q_heads, desc->max_blocks_per_seq, desc->window);
@@ -780,6 +831,15 @@ int llh::plan_decode(llh_ctx *ctx, const llh_kv_pool *pool, const llh_decode_des
     plan->desc_off = align_up(plan->o_off + rows * kFastHeadDim * sizeof(float));
     plan->bytes = align_up(plan->desc_off +
                            (plan->stream_wgs ? (size_t)desc->num_seqs * pv.kv_heads * 2 * sizeof(int32_t) : 0));
+    if (!keep_fused && ctx->opt(LLH_OPT_DECODE_KERNEL) == 0 &&
+        decode_prefers_rows(pv, group, desc->num_seqs, sp.est_blocks)) {
+      plan->fast = false;
+      // the lengths the vector kernels take
+      if (plan->stream_wgs) plan->max_len = std::max(1, desc->max_seq_len);
+      else plan->max_span = plan->max_splits * plan->split_blocks * kFastBlockTokens;
+      plan->stream_wgs = 0;
+      plan_rows(ctx, pv, desc, max_bytes, plan);
+    }
     return LLH_OK;
   }
   // any other shape: the reference-order kernel, with a score row per (sequence, head)
@@ -791,21 +851,11 @@ int llh::plan_decode(llh_ctx *ctx, const llh_kv_pool *pool, const llh_decode_des
   // head_dim 128 or 256 over 16-token blocks: the packed-row MFMA kernel.  Its partials take
   // the place of the score rows (the step's workspace is never less than theirs, so what a
   // caller reserved, or the no-allocation entry refused, stays as it was)
-  plan->rows = pv.format != LLH_KV_INT8_ROW && (pv.head_dim == kFastHeadDim || pv.head_dim == kD256HeadDim) &&
-               pv.block_tokens == kFastBlockTokens && rows_aligned && !ctx->opt(LLH_OPT_FORCE_GENERIC);
-  if (plan->rows) {
-    const int uk = rows_unit_keys(pv.head_dim);
-    const int units = (plan->score_stride + uk - 1) / uk + 1;
-    const long long tiles = (long long)pv.kv_heads * ((group + 15) / 16);
-    const long long total = desc->total_tokens_hint > 0
-                                ? tiles * ((long long)desc->total_tokens_hint / uk + desc->num_seqs)
-                                : tiles * units * desc->num_seqs;
-    const SplitRows sr = split_rows(ctx, pv, units, total, (size_t)desc->num_seqs * desc->num_q_heads, max_bytes);
-    plan->split_units = sr.split_units;
-    plan->max_splits = sr.max_splits;
-    plan->ml_off = 0;
-    plan->o_off = sr.o_off;
-    plan->bytes = std::max(plan->bytes, sr.bytes);
+  if (pv.format != LLH_KV_INT8_ROW && (pv.head_dim == kFastHeadDim || pv.head_dim == kD256HeadDim) &&
+      pv.block_tokens == kFastBlockTokens && rows_aligned && !ctx->opt(LLH_OPT_FORCE_GENERIC)) {
+    plan->exact = true;
+    plan->max_span = plan->score_stride;
+    plan_rows(ctx, pv, desc, max_bytes, plan);
   }
   return LLH_OK;
 }
@@ -817,6 +867,17 @@ int llh::launch_planned_decode(llh_ctx *ctx, const llh_kv_pool *pool, const llh_
                                const uint16_t *v_new) {
   const PoolView &pv = pool->view;
   ctx->decode_calls++;
+  struct TimingHook {
+    llh_ctx *ctx;
+    std::pair<hipEvent_t, hipEvent_t> ev;
+  } th{ctx, {nullptr, nullptr}};
+  const LaunchHook hook = [](void *u, int phase, hipStream_t st) {
+    auto *t = static_cast<TimingHook *>(u);
+    if (phase == 0)
+      t->ev = t->ctx->timing_begin(st);
+    else
+      t->ctx->timing_end(0, t->ev, st);
+  };
   if (plan.fast) {
     DecodeArgs a{};
     a.pool = pv;
@@ -842,25 +903,14 @@ int llh::launch_planned_decode(llh_ctx *ctx, const llh_kv_pool *pool, const llh_
     a.k_new = k_new;
     a.v_new = v_new;
     a.gate = static_cast<const uint16_t *>(desc->d_gate);
-    struct TimingHook {
-      llh_ctx *ctx;
-      std::pair<hipEvent_t, hipEvent_t> ev;
-    } th{ctx, {nullptr, nullptr}};
-    const LaunchHook hook = [](void *u, int phase, hipStream_t st) {
-      auto *t = static_cast<TimingHook *>(u);
-      if (phase == 0)
-        t->ev = t->ctx->timing_begin(st);
-      else
-        t->ctx->timing_end(0, t->ev, st);
-    };
     hipError_t e = plan.d256 ? launch_decode_d256(a, desc->max_seq_len, s, timed ? &th : nullptr, timed ? hook : nullptr)
                              : launch_decode(a, plan.group, desc->max_seq_len, s, timed ? &th : nullptr,
                                              timed ? hook : nullptr);
     if (e != hipSuccess) return ctx->hip_fail(e, "decode launch");
     return LLH_OK;
   }
-  ctx->generic_decode_calls++;
   if (plan.rows) {
+    if (plan.exact) ctx->generic_decode_calls++;
     RowsArgs r{};
     r.pool = pv;
     r.q = static_cast<const uint16_t *>(d_q);
@@ -876,16 +926,19 @@ int llh::launch_planned_decode(llh_ctx *ctx, const llh_kv_pool *pool, const llh_
     r.window = desc->window;
     r.split_units = plan.split_units;
     r.max_splits = plan.max_splits;
-    r.max_span = plan.score_stride;
-    r.zero_bad = 1;
-    r.flag_nonfinite = 1;
+    r.single_units = plan.single_units;
+    r.max_span = plan.max_span;
+    r.max_len = plan.max_len;
+    r.zero_bad = plan.exact ? 1 : 0;
+    r.flag_nonfinite = plan.exact ? 1 : 0;
     r.scale = score_scale;
     r.scale_log2e = score_scale * 1.4426950408889634f;
     r.gate = static_cast<const uint16_t *>(desc->d_gate);
-    const hipError_t e = launch_rows(r, 1, /*exact_weights=*/true, s);
+    const hipError_t e = launch_rows(r, 1, plan.exact, s, timed ? &th : nullptr, timed ? hook : nullptr);
     if (e != hipSuccess) return ctx->hip_fail(e, "decode launch");
     return LLH_OK;
   }
+  ctx->generic_decode_calls++;
   GenericDecodeArgs g{};
   g.pool = pv;
   g.q = d_q;
@@ -992,7 +1045,7 @@ int llh_paged_decode_append(llh_ctx *ctx, llh_kv_pool *pool, const llh_decode_de
   if (desc->num_seqs > 0 && (!d_out || !d_k_new || !d_v_new))
     return ctx->fail(LLH_ERR_NULL, "null device pointer in decode call");
   DecodePlan plan;
-  int st = plan_decode(ctx, pool, desc, d_q, d_out, score_scale, &plan);
+  int st = plan_decode(ctx, pool, desc, d_q, d_out, score_scale, &plan, SIZE_MAX, /*keep_fused=*/true);
   if (st != LLH_OK || plan.empty) return st;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const PoolView &pv = pool->view;
@@ -1151,6 +1204,7 @@ int llh_paged_prefill(llh_ctx *ctx, const llh_kv_pool *pool, const llh_prefill_d
     r.max_blocks = a.max_blocks;
     r.window = a.window;
     r.split_units = sr.split_units;
+    r.single_units = sr.single_units;
     r.max_splits = sr.max_splits;
     r.scale = score_scale;
     r.scale_log2e = a.scale_log2e;

@@ -217,9 +217,12 @@ struct DecodePlan {
   bool empty = false;  // nothing to launch (no sequences)
   bool fast = false;   // tuned kernels (else the reference-order kernel)
   bool d256 = false;   // tuned: the head_dim-256 (G = 8, bf16 / fp16) kernels (split-K, or stream when stream_wgs > 0)
-  bool rows = false;   // packed-row kernel (rows.hip): head_dim 128 / 256 shapes the tuned kernels do not take
+  bool rows = false;   // packed-row kernel (rows.hip)
+  bool exact = false;  // rows: f32 softmax weights and the reference-order kernel's flags
   int group = 0;
-  int split_units = 0;  // rows: least units per split
+  int split_units = 0;   // rows: least units per split
+  int max_span = 0, max_len = 0;  // rows: attended tokens / length beyond which the device refuses a sequence (0: any)
+  int single_units = 0;  // rows: sequences of at most this many units are not split
   int split_blocks = 0, max_splits = 0, stream_wgs = 0;
   size_t ml_off = 0, o_off = 0, desc_off = 0;  // tuned: partial (max, sum), partial outputs, segment descriptors
   int score_stride = 0;
@@ -227,9 +230,11 @@ struct DecodePlan {
   size_t bytes = 0;
 };
 // max_bytes: the most workspace the caller can give; a layout choice that would
-// need more falls back to one that fits (llh_paged_decode_noalloc's scratch)
+// need more falls back to one that fits (llh_paged_decode_noalloc's scratch);
+// keep_fused: stay with the kernels that take a fused append
 int plan_decode(llh_ctx *ctx, const llh_kv_pool *pool, const llh_decode_desc *desc, const void *d_q,
-                const void *d_out, float score_scale, DecodePlan *plan, size_t max_bytes = SIZE_MAX);
+                const void *d_out, float score_scale, DecodePlan *plan, size_t max_bytes = SIZE_MAX,
+                bool keep_fused = false);
 // err: the device error word the kernels raise flags in; timed = false leaves out
 // the kernel-timing events (no event is created or recorded); k_new / v_new
 // (tuned kernels): fused append of each sequence's new token

@@ -126,7 +126,6 @@ struct PrefillArgs {
 // Packed query rows over split keys (rows.hip): decode steps outside the tuned shapes
 // and prefill calls of few rows.  Workspace: partial rows [T][Hq][max_splits].
 constexpr int kRowsMaxSplits = 64;
-constexpr int kRowsSingleUnits = 8;  // sequences of at most this many units are never split
 struct RowsArgs {
   PoolView pool;            // head_dim 128 or 256, 16-token blocks, any format but int8 rows
   const uint16_t *q;        // [T][Hq][D] bf16
@@ -143,7 +142,9 @@ struct RowsArgs {
   int32_t window;
   int32_t split_units;      // least units (rows_unit_keys keys) per split
   int32_t max_splits;       // longer sequences take longer splits
+  int32_t single_units;     // sequences of at most this many units are not split
   int32_t max_span;         // > 0: a longer attended span raises kErrTooManySplits
+  int32_t max_len;          // > 0: so does a longer context
   int32_t zero_bad;         // keys of a block outside the pool: 1 = score 0 and a zero value, 0 = masked
   int32_t flag_nonfinite;   // 1: a non-finite score raises kErrNonFinite
   float scale;
@@ -151,9 +152,6 @@ struct RowsArgs {
   const uint16_t *gate;
 };
 int rows_unit_keys(int head_dim);
-// max_rows: host bound on a sequence's query rows; exact_weights: softmax weights keep
-// f32 precision in p . v (always so for int8 / fp8 blocks)
-hipError_t launch_rows(const RowsArgs &a, int max_rows, bool exact_weights, hipStream_t s);
 
 struct WriteBlocksArgs {
   PoolView pool;
@@ -231,6 +229,10 @@ int matvec_ksplit(int rows, int cols, int n, int cus);
 // `hook(user, 0, s)` runs just before and `hook(user, 1, s)` just after the main
 // decode kernel is enqueued (before the merge): kernel timing records events there.
 typedef void (*LaunchHook)(void *user, int phase, hipStream_t s);
+// max_rows: host bound on a sequence's query rows; exact_weights: softmax weights keep
+// f32 precision in p . v (always so for int8 / fp8 blocks)
+hipError_t launch_rows(const RowsArgs &a, int max_rows, bool exact_weights, hipStream_t s, void *hook_user = nullptr,
+                       LaunchHook hook = nullptr);
 hipError_t launch_decode(const DecodeArgs &a, int group, int max_seq_len, hipStream_t s, void *hook_user = nullptr,
                          LaunchHook hook = nullptr);
 // head_dim 256, G = 8, bf16 pools, split-K (a.stream_wgs = 0, a.max_splits <= 64, no fused append)

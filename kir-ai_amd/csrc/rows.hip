@@ -97,15 +97,13 @@ __device__ __forceinline__ SeqSplit seq_split(const RowsArgs &a, int b) {
   const int first = s.ctx - s.chunk;  // position of the first row
   s.lo = a.window > 0 ? max(0, first - a.window + 1) : 0;
   const int span = max(0, s.ctx - s.lo);
-  if (a.max_span > 0 && span > a.max_span) s.flags = kErrTooManySplits;
+  if ((a.max_span > 0 && span > a.max_span) || (a.max_len > 0 && s.ctx > a.max_len)) s.flags = kErrTooManySplits;
   else if ((int64_t)span > (int64_t)a.max_blocks * BT) s.flags = kErrSpan;
   s.skip = s.flags != 0 || s.chunk <= 0 || (a.chunk_starts && s.ctx < s.chunk);
   s.unit0 = s.lo / UK;
   s.units = span > 0 ? (s.ctx - 1) / UK - s.unit0 + 1 : 0;
-  // short sequences are not split: the second launch costs about what four units cost a
-  // wavefront
-  s.per_split = s.units <= kRowsSingleUnits ? kRowsSingleUnits
-                                            : max(a.split_units, (s.units + a.max_splits - 1) / a.max_splits);
+  s.per_split = s.units <= a.single_units ? a.single_units
+                                          : max(a.split_units, (s.units + a.max_splits - 1) / a.max_splits);
   s.n_splits = (s.units + s.per_split - 1) / s.per_split;
   return s;
 }
@@ -465,7 +463,9 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 && is16(FMT) ? 1 : 2) void pag
   for (int i = tid; i < live * (D / 4); i += 64 * WAVES) {
     const int r = i / (D / 4);
     const int d = 4 * (i % (D / 4));
-    const float mm = fmaxf(fmaxf(s_m[0][r], s_m[1][r]), fmaxf(s_m[2][r], s_m[3][r]));
+    float mm = s_m[0][r];
+#pragma unroll
+    for (int w = 1; w < WAVES; w++) mm = fmaxf(mm, s_m[w][r]);
     const float mref = mm == -INFINITY ? 0.0f : mm;
     float ll = 0.0f;
     f32x4_t oo = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
@@ -535,28 +535,30 @@ __global__ __launch_bounds__(D) void paged_rows_merge_kernel(const RowsArgs a) {
 }
 
 template <int D, int FMT, int PARTS>
-hipError_t launch_rows_t(const RowsArgs &a, int max_rows, hipStream_t s) {
+hipError_t launch_rows_t(const RowsArgs &a, int max_rows, hipStream_t s, void *hu, LaunchHook hook) {
   const int tiles = (max_rows * (a.q_heads / a.pool.kv_heads) + TILE - 1) / TILE;
+  if (hook) hook(hu, 0, s);
   hipLaunchKernelGGL((paged_rows_kernel<D, FMT, PARTS>), dim3(a.max_splits * a.pool.kv_heads * tiles, a.num_seqs),
                      dim3(64 * WAVES), 0, s, a);
   hipError_t e = hipGetLastError();
+  if (hook) hook(hu, 1, s);
   if (e != hipSuccess || a.max_splits <= 1) return e;
-  hipLaunchKernelGGL((paged_rows_merge_kernel<D, kUnitKeys<D>>), dim3(max_rows * a.q_heads, a.num_seqs), dim3(D),
-                     0, s, a);
+  hipLaunchKernelGGL((paged_rows_merge_kernel<D, kUnitKeys<D>>), dim3(max_rows * a.q_heads, a.num_seqs), dim3(D), 0, s,
+                     a);
   return hipGetLastError();
 }
 
 template <int D>
-hipError_t launch_rows_d(const RowsArgs &a, int max_rows, bool exact_weights, hipStream_t s) {
+hipError_t launch_rows_d(const RowsArgs &a, int max_rows, bool exact_weights, hipStream_t s, void *hu, LaunchHook hook) {
   switch (a.pool.format) {
     case kBf16:
-      return exact_weights ? launch_rows_t<D, kBf16, 3>(a, max_rows, s) : launch_rows_t<D, kBf16, 1>(a, max_rows, s);
+      return exact_weights ? launch_rows_t<D, kBf16, 3>(a, max_rows, s, hu, hook) : launch_rows_t<D, kBf16, 1>(a, max_rows, s, hu, hook);
     case kF16:
-      return exact_weights ? launch_rows_t<D, kF16, 3>(a, max_rows, s) : launch_rows_t<D, kF16, 1>(a, max_rows, s);
+      return exact_weights ? launch_rows_t<D, kF16, 3>(a, max_rows, s, hu, hook) : launch_rows_t<D, kF16, 1>(a, max_rows, s, hu, hook);
     case kInt8:
-      return launch_rows_t<D, kInt8, 3>(a, max_rows, s);
+      return launch_rows_t<D, kInt8, 3>(a, max_rows, s, hu, hook);
     case kFp8:
-      return launch_rows_t<D, kFp8, 3>(a, max_rows, s);
+      return launch_rows_t<D, kFp8, 3>(a, max_rows, s, hu, hook);
   }
   return hipErrorInvalidValue;
 }
@@ -565,10 +567,10 @@ hipError_t launch_rows_d(const RowsArgs &a, int max_rows, bool exact_weights, hi
 
 int rows_unit_keys(int head_dim) { return head_dim == 256 ? 32 : 64; }
 
-hipError_t launch_rows(const RowsArgs &a, int max_rows, bool exact_weights, hipStream_t s) {
+hipError_t launch_rows(const RowsArgs &a, int max_rows, bool exact_weights, hipStream_t s, void *hu, LaunchHook hook) {
   if (a.max_splits < 1 || a.max_splits > kRowsMaxSplits || max_rows < 1) return hipErrorInvalidValue;
-  return a.pool.head_dim == 256 ? launch_rows_d<256>(a, max_rows, exact_weights, s)
-                                : launch_rows_d<128>(a, max_rows, exact_weights, s);
+  return a.pool.head_dim == 256 ? launch_rows_d<256>(a, max_rows, exact_weights, s, hu, hook)
+                                : launch_rows_d<128>(a, max_rows, exact_weights, s, hu, hook);
 }
 
 }  // namespace llh

@@ -169,3 +169,22 @@ def test_rows_prefill(ctx, opts, D, Hq, Hkv, fmt, window):
         assert_parity(from_dev_bf16(out), ref.astype(np.float32), what="captured")
     assert ctx.device_errors() == 0, ctx.last_error()
     ctx.release_stream(stream)
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+def test_rows_decode_group_of_eight(ctx, fmt):
+    """Groups of eight at head_dim 128, which the planner gives to the packed-row kernel,
+    against the vector kernels (forced) and the oracle: edge lengths, one long sequence,
+    a window."""
+    from helpers import assert_parity
+    from test_gpu_decode import run_decode
+
+    Hq, Hkv, D = 32, 4, 128
+    lens = np.array(EDGES + [5000], np.int32)
+    batch = workloads.paged_batch(lens, BT, 0.10, 61)
+    pool, q = build_case(ctx, batch, Hq, Hkv, FMTS[fmt], 62, head_dim=D)
+    for window in (0, 100):
+        ref = oracle_decode(pool, batch, FMTS[fmt], Hq, Hkv, window, q, 0.088, head_dim=D)
+        out = run_decode(ctx, pool, batch, q, Hq, window, 0.088)
+        assert_parity(out, ref, what=f"{fmt} W{window}")
+    assert ctx.device_errors() == 0, ctx.last_error()
