@@ -118,7 +118,9 @@ typedef enum llh_option {
   LLH_OPT_DECODE_STREAM_WGS = 2,     /* (LLH_DECODE_STREAM_WGS) stream-kernel workgroups, 0 = 2 per CU */
   LLH_OPT_FORCE_GENERIC = 3,         /* (LLH_FORCE_GENERIC) 1 = the element-wise decode and prefill
                                         kernels for every shape */
-  LLH_OPT_PREFILL_HEADS_PER_WG = 4,  /* (LLH_PREFILL_HEADS_PER_WG) 1 = one query head per prefill workgroup */
+  LLH_OPT_PREFILL_HEADS_PER_WG = 4,  /* (LLH_PREFILL_HEADS_PER_WG) 1 = prefill workgroups of 128 packed rows
+                                        (4 wavefronts), 2 = of 256; either also keeps short chunks off the
+                                        packed-row kernel; 0 = automatic */
   LLH_OPT_TRAIT_REFERENCE_ORDER = 5, /* (LLH_TRAIT_REFERENCE_ORDER) trait-mirror attention: 0 = the tuned
                                         kernels where the shape allows, 1 = the reference-order kernel always */
   LLH_OPT_COUNT = 6

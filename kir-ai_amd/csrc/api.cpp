@@ -235,27 +235,27 @@ SplitRows split_prefill_rows(const llh_ctx *ctx, const PoolView &pv, const llh_p
   return r;
 }
 
-// Whether a prefill call of the tuned shapes runs the packed-row kernel.  Its time per key
-// grows with the 16-row tiles of the call, that of the 128-row-tile kernels with the rounds
-// their workgroups (one or two heads of 128 rows each) take: measured on MI355X (us per
-// 1000 keys over bf16 blocks) 0.040 per tile against 28 per round at head_dim 128, 0.093
-// against 31 at head_dim 256; int8 / fp8 at head_dim 128 0.030 against 34.  The packed-row
-// kernel's second launch costs it about 5 us, so it must win by more: at equal
-// (256 workgroups) rounds, 8 x (1024 + chunk): head_dim 128, 256 tiles 27.0 against 36.6 us,
-// 1024 tiles 58.9 against 38.4; head_dim 256, 128 tiles 28.7 against 38.6, 256 tiles 40.8
-// against 38.3.
+// Whether a prefill call of the tuned shapes runs the packed-row kernel.  Its time grows with
+// its 16-row tiles times their keys; the tile kernels' has a floor (a second launch and
+// partial sums, or few workgroups).  Keys are bounded by the table rows (or the window).
+// Measured on MI355X, packed rows against tiles (us): head_dim 128, bf16, Hq16 / Hkv8,
+// 1 x (4096 + chunk): 64 row tiles 24.9 / 25.5, 128 36.4 / 34.9, 256 60.3 / 39.0; 1 x (1024 +
+// chunk): 256 25.7 / 26.8; 1 x (256 + chunk): 256 12.3 / 23.1; int8, 8 x (1024 + 32), 512 row
+// tiles 29.8 / 34.3; head_dim 256, Hq16 / Hkv2: 1 x 4096: 64 35.6 / 37.4, 128 63.1 / 40.4;
+// 8 x 1024: 128 28.9 / 29.4, and over 300 keys the tile kernel's single launch wins from 32 row
+// tiles on: 128 16.9 / 15.3.
 bool prefill_takes_rows(const llh_ctx *ctx, const PoolView &pv, const llh_prefill_desc *d) {
   if (d->max_chunk_len <= 0 || ctx->opt(LLH_OPT_PREFILL_HEADS_PER_WG)) return false;
   const int group = d->num_q_heads / pv.kv_heads;
-  const long long tiles = ((long long)d->max_chunk_len * group + 15) / 16 * pv.kv_heads;
-  const bool wide = pv.head_dim == kD256HeadDim;
-  const long long wgs = ((long long)d->max_chunk_len + 127) / 128 * d->num_seqs *
-                        (wide || group % 2 ? d->num_q_heads : d->num_q_heads / 2);
-  // contexts of a few tiles (by the table rows' bound) take the tile kernels as long:
-  // head_dim 256, 8 x 270 tokens 15.2 us on either, 7 x 230 13.0 against 14.0
-  if (wide && (long long)d->max_blocks_per_seq * kFastBlockTokens <= 320) return false;
-  const long long per_round = wide ? 128 : is16(pv.format) ? 256 : 512;
-  return tiles * d->num_seqs <= per_round * ((wgs + ctx->cus - 1) / ctx->cus);
+  const long long tiles = ((long long)d->max_chunk_len * group + 15) / 16 * pv.kv_heads * d->num_seqs;
+  long long keys = (long long)d->max_blocks_per_seq * kFastBlockTokens;
+  if (d->window > 0) keys = std::min<long long>(keys, (long long)d->window + d->max_chunk_len);
+  if (pv.head_dim == kD256HeadDim) {
+    if (keys <= 320) return tiles < 32;
+    return tiles <= 64 || (tiles <= 128 && tiles * keys <= 150000);
+  }
+  const long long budget = is16(pv.format) ? 400000 : 600000;
+  return tiles <= 64 || (tiles <= 512 && tiles * keys <= budget);
 }
 
 }  // namespace
@@ -1164,7 +1164,7 @@ int llh_paged_prefill(llh_ctx *ctx, const llh_kv_pool *pool, const llh_prefill_d
   a.q_heads = desc->num_q_heads;
   a.max_blocks = desc->max_blocks_per_seq;
   a.window = desc->window;
-  a.q_tiles = std::max(1, (desc->max_chunk_len + 127) / 128);
+  a.max_pieces = 1;
   a.scale_log2e = score_scale * 1.4426950408889634f;
   a.scale = score_scale;
   a.gate = static_cast<const uint16_t *>(desc->d_gate);
@@ -1186,6 +1186,43 @@ int llh_paged_prefill(llh_ctx *ctx, const llh_kv_pool *pool, const llh_prefill_d
     }
   }
   if (rows_only) ctx->generic_prefill_calls++;
+  // Items of `bm` rows, all heads of a kv head packed.  Where they make at most half as many
+  // groups of `cut` rows as there are compute units and the contexts may be long enough, they
+  // are cut into as many pieces as still give one workgroup per compute unit (more than that is
+  // a second round), with the partial sums in the stream's workspace (none under capture).
+  // Else, where they do not fill the compute units, only `least` heads are packed.  Measured on
+  // MI355X, least heads packed / all / all, cut (us): head_dim 128, Hq32 / Hkv4, 1 x (4096 + 512)
+  // 132 / 103 / 58, 8 x (1024 + 64) 38 / - / 33, 8 x (256 + 64) 17.3 / 19.7 / 29.6,
+  // 8 x (1536 + 512) 142 / 138 / -; head_dim 256, Hq16 / Hkv2, 2 x (1024 + 256) 59.6 / - / 36.2,
+  // 8 x (256 + 64) 17.2 / 22.6 / 29.2.
+  auto plan_pieces = [&](int bm, int cut, int least) {
+    const int G = desc->num_q_heads / pv.kv_heads;
+    const long long groups = (long long)pv.kv_heads * desc->num_seqs;
+    const long long tiles = std::max(1LL, ((long long)desc->max_chunk_len * G + bm - 1) / bm);
+    // every sequence's last group may be partial; a uniform batch is counted exactly
+    const long long cuts = std::max<long long>(
+        1, (long long)desc->total_q_rows == (long long)desc->max_chunk_len * desc->num_seqs
+               ? ((long long)desc->max_chunk_len * G + cut - 1) / cut * groups
+               : pv.kv_heads * (((long long)desc->total_q_rows * G + cut - 1) / cut + (desc->num_seqs + 1) / 2));
+    long long keys = (long long)desc->max_blocks_per_seq * kFastBlockTokens;
+    if (desc->window > 0) keys = std::min<long long>(keys, (long long)desc->window + desc->max_chunk_len);
+    const long long pieces = std::min<long long>(kPrefillMaxPieces, ctx->cus / cuts);
+    auto whole = [&](int pack) {
+      a.pack = pack;
+      a.q_tiles = (int32_t)std::max(1LL, ((long long)desc->max_chunk_len * pack + bm - 1) / bm);
+    };
+    if (pieces < 2 || desc->num_seqs > 64 || keys / 64 < prefill_cut_tiles((int)pieces, pv.head_dim))
+      return whole(cuts >= ctx->cus ? G : least);
+    a.pack = G;
+    a.q_tiles = (int32_t)tiles;
+    const size_t rows = (size_t)(tiles * groups * pieces * bm);
+    const size_t o_off = align_up(rows * sizeof(float2));
+    if (!lease.try_acquire(ctx, static_cast<hipStream_t>(stream), o_off + rows * pv.head_dim * sizeof(float)))
+      return whole(least);
+    a.max_pieces = (int32_t)pieces;
+    a.ws_ml = reinterpret_cast<float2 *>(lease.base());
+    a.ws_o = reinterpret_cast<float *>(lease.base() + o_off);
+  };
   if (rows) {
     RowsArgs r{};
     r.pool = pv;
@@ -1211,12 +1248,12 @@ int llh_paged_prefill(llh_ctx *ctx, const llh_kv_pool *pool, const llh_prefill_d
     r.gate = a.gate;
     e = launch_rows(r, desc->max_chunk_len, /*exact_weights=*/false, static_cast<hipStream_t>(stream));
   } else if (fast) {
-    // two query heads of a kv head per workgroup share its K/V tile stream when the group is even
-    const int group = desc->num_q_heads / pv.kv_heads;
-    const int hpw_env = ctx->opt(LLH_OPT_PREFILL_HEADS_PER_WG);
-    const int variant = (hpw_env == 1 || group % 2 != 0) ? kPrefillOneHead : kPrefillTwoHeads;
-    e = launch_prefill(a, variant, static_cast<hipStream_t>(stream));
+    const bool narrow = ctx->opt(LLH_OPT_PREFILL_HEADS_PER_WG) == 1;
+    // both workgroup sizes pack and cut alike, and give the same bits
+    plan_pieces(narrow ? 128 : 256, 256, desc->num_q_heads / pv.kv_heads % 2 ? 1 : 2);
+    e = launch_prefill(a, narrow ? kPrefillRows128 : kPrefillRows256, static_cast<hipStream_t>(stream));
   } else if (fast256) {
+    plan_pieces(128, 128, 1);
     e = launch_prefill_d256(a, static_cast<hipStream_t>(stream));
   } else {
     ctx->generic_prefill_calls++;

@@ -105,6 +105,12 @@ struct GenericDecodeArgs {
   const uint16_t *gate;     // null, or [B][Hq][D] bf16: out = attention * sigmoid(gate)
 };
 
+constexpr int kPrefillMaxPieces = 8;
+// 64-key tiles from which a sequence is cut into `pieces`: the tiles saved against the memory
+// traffic of the partial sums and the second launch (prefill_items.h)
+__host__ __device__ constexpr int prefill_cut_tiles(int pieces, int head_dim) {
+  return 36 / pieces + (head_dim == kD256HeadDim ? 7 : 4);
+}
 struct PrefillArgs {
   PoolView pool;
   const uint16_t *q;        // [T][Hq][128]
@@ -117,7 +123,11 @@ struct PrefillArgs {
   int32_t q_heads;
   int32_t max_blocks;
   int32_t window;
-  int32_t q_tiles;          // tiles of 128 rows per sequence in the grid
+  int32_t q_tiles;          // row tiles per (sequence, head group) in the grid
+  int32_t pack;             // query heads of a kv head packed into an item's rows
+  int32_t max_pieces;       // > 1: items may be cut into at most this many pieces (prefill_items.h)
+  float *ws_o;              // max_pieces > 1: [items][max_pieces][rows][D] partial outputs
+  float2 *ws_ml;            // [items][max_pieces][rows] (max in log2 units, sum)
   float scale_log2e;
   float scale;              // score_scale (generic kernel)
   const uint16_t *gate;     // null, or [T][Hq][D] bf16: out = attention * sigmoid(gate)
@@ -239,12 +249,10 @@ hipError_t launch_decode(const DecodeArgs &a, int group, int max_seq_len, hipStr
 hipError_t launch_decode_d256(const DecodeArgs &a, int max_seq_len, hipStream_t s, void *hook_user = nullptr,
                               LaunchHook hook = nullptr);
 hipError_t launch_decode_generic(const GenericDecodeArgs &a, int q_f32, int out_f32, hipStream_t s);
-// heads_per_wg: query heads of one kv head that share a workgroup's K/V tiles (1 or 2; 2 needs an even group)
-// prefill kernels: one query head per workgroup, or two heads of a kv head
-// sharing the K/V tiles
-enum { kPrefillOneHead = 1, kPrefillTwoHeads = 2 };
+// prefill workgroups of 128 packed query rows (4 wavefronts) or 256 (8 wavefronts)
+enum { kPrefillRows128 = 1, kPrefillRows256 = 2 };
 hipError_t launch_prefill(const PrefillArgs &a, int variant, hipStream_t s);
-// head_dim 256, bf16 pools, 16-token blocks (one query head per workgroup)
+// head_dim 256, bf16 / fp16 pools, 16-token blocks (128 packed query rows per workgroup)
 hipError_t launch_prefill_d256(const PrefillArgs &a, hipStream_t s);
 constexpr int kGenericPrefillMaxDim = 512;  // head_dim bound of the generic prefill kernel
 // Element-wise prefill for every other shape (any head_dim <= 512, block size,

@@ -7,21 +7,15 @@
 // "append then attend" loop (crates/llm-backend/src/core/native_attention.rs:356-464)
 // computed as one dense pass.
 //
-// One workgroup = 128 query rows of one query head (4 wavefronts x 32 rows).
-// Key tiles of 64 positions (4 pool blocks) are staged in LDS, double
-// buffered: while the wavefronts run the MFMAs of tile t, every lane already
-// holds its share of tile t+1 in registers, and stores it to the other buffer
-// afterwards (one barrier per tile).  When a kv head's group is even, one
-// workgroup of 8 wavefronts runs two of its query heads over the same K/V
-// tiles (half the tile loads and LDS stores per FLOP).  Tiles wholly outside the window or past
-// the last query are never loaded, and only tiles that straddle a boundary are
-// masked.
-//
-// Work mapping: workgroups are dispatched round-robin over the 8 XCDs, each
-// with its own L2.  The launch maps workgroup L to logical work item
-// w = (L % 8) * ceil(N / 8) + L / 8, and logical items run (sequence, kv head,
-// query tile, query head in group) with the head fastest, so each XCD works on
-// few (sequence, kv head) pairs at a time and their K/V tiles stay in its L2.
+// One workgroup = 256 packed query rows (8 wavefronts x 32 rows) of one kv head: row R of
+// the chunk is token R / G, head R % G, so the G heads of a token share every K / V tile and
+// a workgroup's rows are few tokens (little of the causal triangle is wasted).  Key tiles of
+// 64 positions (4 pool blocks) are staged in LDS, double buffered: while the wavefronts run
+// the MFMAs of tile t, every lane already holds its share of tile t+1 in registers, and
+// stores it to the other buffer afterwards (one barrier per tile).  Tiles wholly outside the
+// window or past the last query are never loaded, and only tiles that straddle a boundary
+// are masked.  Work items, their order and the cutting of long items when a call has few:
+// prefill_items.h.
 //
 // int8 / fp8 pools are dequantised while a tile is stored to LDS (code * scale in
 // f32, rounded to bf16), so the MFMA path is the same for every format: the
@@ -41,6 +35,7 @@
 // 16-key step is {4h..4h+3, 8+4h..8+4h+3} for lane half h; the V^T operand is
 // read from LDS with the same key order, so no transpose is ever done.
 // Softmax statistics are kept per query column in log2 units (online softmax).
+#include "prefill_items.h"
 #include "wave_ops.h"
 
 namespace llh {
@@ -49,7 +44,6 @@ namespace {
 
 constexpr int D = kFastHeadDim;
 constexpr int BT = kFastBlockTokens;
-constexpr int BM = 128;          // query rows per workgroup
 constexpr int BN = 64;           // key positions per tile
 constexpr int KBLK = BN / BT;    // pool blocks per tile
 constexpr int K_STRIDE = D + 8;  // bf16 elements per K row in LDS (272 B: conflict-free b128 reads)
@@ -234,67 +228,36 @@ __device__ __forceinline__ void store_tile(uint16_t *k_lds, uint16_t *v_lds, int
 
 template <int HPW, int FMT>
 __global__ __launch_bounds__(kPrefillThreads * HPW, 2 / HPW) void paged_prefill_kernel(const PrefillArgs a) {
-  // ---- XCD-aware logical work item ----
+  constexpr int BM = 128 * HPW;  // packed query rows per workgroup
+  const PrefillItem it = prefill_item<BM, 256>(a);
+  if (it.skip) {
+    if (it.flags && threadIdx.x == 0) atomicOr(a.err, it.flags);
+    return;
+  }
   const int Hq = a.q_heads;
-  const int Hkv = a.pool.kv_heads;
-  const int GW = Hq / Hkv / HPW;  // workgroups per (kv head, query tile)
-  const int n_items = a.q_tiles * Hkv * GW * a.num_seqs;
-  const int per_xcd = (n_items + 7) / 8;
-  // Within one XCD's items, the longest go first: when its block of items is
-  // whole (sequence, kv head) groups, dispatch i takes tile q_tiles-1-r of
-  // group g (r = i / (groups * GW)), so the first round runs the tiles with
-  // the longest causal reach and the last round the shortest.
-  const int per_group = a.q_tiles * GW;
-  const int di = blockIdx.x / 8;
-  int local = di;
-  if (per_xcd % per_group == 0) {
-    const int groups = per_xcd / per_group;
-    local = ((di / GW) % groups) * per_group + (a.q_tiles - 1 - di / (groups * GW)) * GW + di % GW;
-  }
-  const int w = (blockIdx.x % 8) * per_xcd + local;
-  if (w >= n_items) return;
-  const int tile = (w / GW) % a.q_tiles;
-  const int kvh = (w / (GW * a.q_tiles)) % Hkv;
-  const int b = w / (GW * a.q_tiles * Hkv);
-  const int qh = (kvh * GW + w % GW) * HPW + (threadIdx.x >> 8);  // this wavefront's query head
-
-  const int c0 = a.chunk_starts[b];
-  const int chunk = a.chunk_starts[b + 1] - c0;
-  const int ctx = a.context_lens[b];
-  const int i0 = tile * BM;
-  if (i0 >= chunk || chunk <= 0 || ctx < chunk) return;
-  {
-    // every key of the chunk's first row through the last must be resident at once:
-    // a longer span would alias its own table entries (rows are read modulo max_blocks)
-    const int first_lo = a.window > 0 ? max(0, ctx - chunk - a.window + 1) : 0;
-    if (ctx - first_lo > a.max_blocks * BT) {
-      if (threadIdx.x == 0 && tile == 0) atomicOr(a.err, kErrSpan);
-      return;
-    }
-  }
+  const int G = a.pack;
+  const int kvh = it.kvh, c0 = it.c0, chunk = it.chunk, ctx = it.ctx, i0 = it.row0;
+  const int rows = chunk * G;
 
   const int tid = threadIdx.x;
-  const int ltid = tid & (kPrefillThreads - 1);  // thread index within the head's 4 wavefronts
+  const int ltid = tid & (kPrefillThreads - 1);  // thread index within its 4 wavefronts
   const int kb0 = (tid / kPrefillThreads) * (KBLK / HPW);  // first tile block this thread loads
   const int lane = tid & 63;
-  const int wave = ltid >> 6;
+  const int wave = tid >> 6;
   const int h = lane >> 5;     // lane half
   const int col = lane & 31;   // query column of this lane
   const int prefix = ctx - chunk;
-
-  // rows of this workgroup and of this wavefront
-  const int rows_wg = min(BM, chunk - i0);
-  const int qpos_first = prefix + i0;                 // position of the first row
-  const int qpos_last = prefix + i0 + rows_wg - 1;    // position of the last valid row
-  const int my_row = i0 + wave * 32 + col;            // chunk row of this lane's query
-  const bool row_ok = my_row < chunk;
-  const int my_pos = prefix + my_row;
+  const int my_row = i0 + wave * 32 + col;  // packed row of this lane's query
+  const bool row_ok = my_row < rows;
+  const int my_tok = min(my_row, rows - 1) / G;
+  const int my_head = it.head0 + min(my_row, rows - 1) % G;
+  const int my_pos = prefix + my_tok;
   const int my_lo = a.window > 0 ? max(0, my_pos - a.window + 1) : 0;
 
   // ---- Q^T operand: 8 k-steps of 16 dims; lane holds dims 16ks + 8h .. +8 of its row ----
   u32x4_t qb[8];
   {
-    const uint16_t *qrow = a.q + ((size_t)(c0 + (row_ok ? my_row : 0)) * Hq + qh) * D;
+    const uint16_t *qrow = a.q + ((size_t)(c0 + my_tok) * Hq + my_head) * D;
 #pragma unroll
     for (int ks = 0; ks < 8; ks++) {
       u32x4_t t = *reinterpret_cast<const u32x4_t *>(qrow + ks * 16 + h * 8);
@@ -333,18 +296,16 @@ __global__ __launch_bounds__(kPrefillThreads * HPW, 2 / HPW) void paged_prefill_
   float m_run = -INFINITY;
   float l_run = 0.0f;
 
-  // key range of the workgroup
-  const int klo = a.window > 0 ? max(0, qpos_first - a.window + 1) : 0;
-  const int khi = qpos_last + 1;  // exclusive
-  const int t_begin = (klo / BN) * BN;
-  const int32_t *table = a.tables + (size_t)b * a.max_blocks;
-  // wavefront-level bounds for masking decisions
+  const int klo = it.klo;
+  const int t_begin = it.t_begin, khi = it.t_end;  // this piece's key tiles
+  const int32_t *table = a.tables + (size_t)it.b * a.max_blocks;
+  // positions of the wavefront's first and last row, for masking decisions
   const int wrow0 = i0 + wave * 32;
-  const int wpos_first = prefix + wrow0;
-  const int wpos_last = prefix + min(wrow0 + 31, chunk - 1);
+  const int wpos_first = prefix + min(wrow0, rows - 1) / G;
+  const int wpos_last = prefix + min(wrow0 + 31, rows - 1) / G;
   const int wlo_first = a.window > 0 ? max(0, wpos_first - a.window + 1) : 0;
   const int wlo_last = a.window > 0 ? max(0, wpos_last - a.window + 1) : 0;
-  const bool wave_live = wrow0 < chunk;
+  const bool wave_live = wrow0 < rows;
 
   TileRegs<FMT, KBLK / HPW> next;
   bool bad = false;
@@ -482,8 +443,19 @@ __global__ __launch_bounds__(kPrefillThreads * HPW, 2 / HPW) void paged_prefill_
   if (bad && tid == 0) atomicOr(a.err, kErrBadBlock);  // a needed block was missing: its keys read as zeros
   const float l_tot = l_run + xor32_other(l_run, lane);
   if (!row_ok) return;
+  if (it.pieces > 1) {  // this piece's unnormalised sums, for prefill_merge_kernel
+    const size_t p = (size_t)it.slot * BM + wave * 32 + col;
+    if (h == 0) a.ws_ml[p] = make_float2(m_run, l_tot);
+#pragma unroll
+    for (int mt = 0; mt < 4; mt++)
+#pragma unroll
+      for (int jq = 0; jq < 4; jq++)
+        *reinterpret_cast<float4 *>(&a.ws_o[p * D + mt * 32 + jq * 8 + 4 * h]) =
+            make_float4(oacc[mt][4 * jq], oacc[mt][4 * jq + 1], oacc[mt][4 * jq + 2], oacc[mt][4 * jq + 3]);
+    return;
+  }
   const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-  const size_t obase = ((size_t)(c0 + my_row) * Hq + qh) * D;
+  const size_t obase = ((size_t)(c0 + my_tok) * Hq + my_head) * D;
   uint16_t *orow = a.out + obase;
 #pragma unroll
   for (int mt = 0; mt < 4; mt++) {
@@ -500,7 +472,7 @@ __global__ __launch_bounds__(kPrefillThreads * HPW, 2 / HPW) void paged_prefill_
 
 template <int FMT>
 void launch_prefill_fmt(const PrefillArgs &a, int variant, int grid, hipStream_t s) {
-  if (variant == kPrefillTwoHeads)
+  if (variant == kPrefillRows256)
     hipLaunchKernelGGL((paged_prefill_kernel<2, FMT>), dim3(grid), dim3(2 * kPrefillThreads), 0, s, a);
   else
     hipLaunchKernelGGL((paged_prefill_kernel<1, FMT>), dim3(grid), dim3(kPrefillThreads), 0, s, a);
@@ -616,8 +588,8 @@ __global__ __launch_bounds__(256) void prefill_generic_kernel(const PrefillArgs 
 }  // namespace
 
 hipError_t launch_prefill(const PrefillArgs &a, int variant, hipStream_t s) {
-  const int n_items = a.q_tiles * (a.q_heads / (variant == kPrefillOneHead ? 1 : 2)) * a.num_seqs;
-  const int grid = (n_items + 7) / 8 * 8;
+  const bool wide = variant == kPrefillRows256;
+  const int grid = wide ? prefill_grid<256>(a) : prefill_grid<128>(a);
   switch (a.pool.format) {
     case kBf16:
       launch_prefill_fmt<kBf16>(a, variant, grid, s);
@@ -634,7 +606,9 @@ hipError_t launch_prefill(const PrefillArgs &a, int variant, hipStream_t s) {
     default:
       return hipErrorInvalidValue;
   }
-  return hipGetLastError();
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || a.max_pieces <= 1) return e;
+  return wide ? launch_prefill_merge<D, 256, 256>(a, s) : launch_prefill_merge<D, 128, 256>(a, s);
 }
 
 hipError_t launch_prefill_generic(const PrefillArgs &a, int total_rows, hipStream_t s) {

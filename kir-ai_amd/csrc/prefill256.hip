@@ -22,7 +22,7 @@
 // of keys 16kb + 4g .. +4 (g = l/16) for query row l%16, and the P^T operand of a
 // 32-key step s takes keys {32s + 4g .. +4, 32s + 16 + 4g .. +4} in its k-slots
 // 8g..8g+7; the V^T operand reads the same keys (one 16-byte LDS read).
-#include "device_common.h"
+#include "prefill_items.h"
 #include "wave_ops.h"
 
 namespace llh {
@@ -177,39 +177,15 @@ __device__ __forceinline__ void store_tile(uint16_t *k_lds, uint16_t *v_lds, int
 
 template <int FMT>
 __global__ __launch_bounds__(kThreads, 1) void paged_prefill_d256_kernel(const PrefillArgs a) {
-  // ---- XCD-aware logical work item (as the head_dim-128 kernel) ----
+  const PrefillItem it = prefill_item<BM, BM>(a);
+  if (it.skip) {
+    if (it.flags && threadIdx.x == 0) atomicOr(a.err, it.flags);
+    return;
+  }
   const int Hq = a.q_heads;
-  const int Hkv = a.pool.kv_heads;
-  const int GW = Hq / Hkv;  // workgroups per (kv head, query tile): one per query head
-  const int n_items = a.q_tiles * Hkv * GW * a.num_seqs;
-  const int per_xcd = (n_items + 7) / 8;
-  const int per_group = a.q_tiles * GW;
-  const int di = blockIdx.x / 8;
-  int local = di;
-  if (per_xcd % per_group == 0) {
-    const int groups = per_xcd / per_group;
-    local = ((di / GW) % groups) * per_group + (a.q_tiles - 1 - di / (groups * GW)) * GW + di % GW;
-  }
-  const int w = (blockIdx.x % 8) * per_xcd + local;
-  if (w >= n_items) return;
-  const int tile = (w / GW) % a.q_tiles;
-  const int kvh = (w / (GW * a.q_tiles)) % Hkv;
-  const int b = w / (GW * a.q_tiles * Hkv);
-  const int qh = kvh * GW + w % GW;
-
-  const int c0 = a.chunk_starts[b];
-  const int chunk = a.chunk_starts[b + 1] - c0;
-  const int ctx = a.context_lens[b];
-  const int i0 = tile * BM;
-  if (i0 >= chunk || chunk <= 0 || ctx < chunk) return;
-  {
-    // every key of the chunk's first row through the last must be resident at once
-    const int first_lo = a.window > 0 ? max(0, ctx - chunk - a.window + 1) : 0;
-    if (ctx - first_lo > a.max_blocks * BT) {
-      if (threadIdx.x == 0 && tile == 0) atomicOr(a.err, kErrSpan);
-      return;
-    }
-  }
+  const int G = a.pack;
+  const int kvh = it.kvh, c0 = it.c0, chunk = it.chunk, ctx = it.ctx, i0 = it.row0;
+  const int rows = chunk * G;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -217,18 +193,17 @@ __global__ __launch_bounds__(kThreads, 1) void paged_prefill_d256_kernel(const P
   const int g = lane >> 4;   // k-slot group of the MFMA operands
   const int r = lane & 15;   // query row of the wavefront; also the A-operand row
   const int prefix = ctx - chunk;
-  const int rows_wg = min(BM, chunk - i0);
-  const int qpos_first = prefix + i0;
-  const int qpos_last = prefix + i0 + rows_wg - 1;
   const int my_row = i0 + wave * ROWS + r;
-  const bool row_ok = my_row < chunk;
-  const int my_pos = prefix + my_row;
+  const bool row_ok = my_row < rows;
+  const int my_tok = min(my_row, rows - 1) / G;
+  const int my_head = it.head0 + min(my_row, rows - 1) % G;
+  const int my_pos = prefix + my_tok;
   const int my_lo = a.window > 0 ? max(0, my_pos - a.window + 1) : 0;
 
   // ---- Q^T operand: 8 k-steps of 32 dims; lane holds dims 32ks + 8g .. +8 of its row ----
   u32x4_t qb[8];
   {
-    const uint16_t *qrow = a.q + ((size_t)(c0 + (row_ok ? my_row : 0)) * Hq + qh) * D;
+    const uint16_t *qrow = a.q + ((size_t)(c0 + my_tok) * Hq + my_head) * D;
 #pragma unroll
     for (int ks = 0; ks < 8; ks++) {
       u32x4_t t = *reinterpret_cast<const u32x4_t *>(qrow + ks * 32 + g * 8);
@@ -265,16 +240,16 @@ __global__ __launch_bounds__(kThreads, 1) void paged_prefill_d256_kernel(const P
   float m_run = -INFINITY;
   float l_run = 0.0f;
 
-  const int klo = a.window > 0 ? max(0, qpos_first - a.window + 1) : 0;
-  const int khi = qpos_last + 1;  // exclusive
-  const int t_begin = (klo / BN) * BN;
-  const int32_t *table = a.tables + (size_t)b * a.max_blocks;
+  const int klo = it.klo;
+  const int t_begin = it.t_begin, khi = it.t_end;  // this piece's key tiles
+  const int32_t *table = a.tables + (size_t)it.b * a.max_blocks;
+  // positions of the wavefront's first and last row
   const int wrow0 = i0 + wave * ROWS;
-  const int wpos_first = prefix + wrow0;
-  const int wpos_last = prefix + min(wrow0 + ROWS - 1, chunk - 1);
+  const int wpos_first = prefix + min(wrow0, rows - 1) / G;
+  const int wpos_last = prefix + min(wrow0 + ROWS - 1, rows - 1) / G;
   const int wlo_first = a.window > 0 ? max(0, wpos_first - a.window + 1) : 0;
   const int wlo_last = a.window > 0 ? max(0, wpos_last - a.window + 1) : 0;
-  const bool wave_live = wrow0 < chunk;
+  const bool wave_live = wrow0 < rows;
   const int vsw = 8 * (g ^ v_swz(r));  // element offset of this lane's V^T chunk pair (dims 16db + r)
 
   Tile256 next;
@@ -403,8 +378,15 @@ __global__ __launch_bounds__(kThreads, 1) void paged_prefill_d256_kernel(const P
   if (bad && tid == 0) atomicOr(a.err, kErrBadBlock);  // a needed block was missing: its keys read as zeros
   const float l_tot = row_sum4(l_run);
   if (!row_ok) return;
+  if (it.pieces > 1) {  // this piece's unnormalised sums, for prefill_merge_kernel
+    const size_t p = (size_t)it.slot * BM + wave * ROWS + r;
+    if (g == 0) a.ws_ml[p] = make_float2(m_run, l_tot);
+#pragma unroll
+    for (int db = 0; db < 16; db++) *reinterpret_cast<f32x4_t *>(&a.ws_o[p * D + db * 16 + 4 * g]) = oacc[db];
+    return;
+  }
   const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-  const size_t obase = ((size_t)(c0 + my_row) * Hq + qh) * D;
+  const size_t obase = ((size_t)(c0 + my_tok) * Hq + my_head) * D;
   uint16_t *orow = a.out + obase;
 #pragma unroll
   for (int db = 0; db < 16; db++) {
@@ -419,13 +401,13 @@ __global__ __launch_bounds__(kThreads, 1) void paged_prefill_d256_kernel(const P
 }  // namespace
 
 hipError_t launch_prefill_d256(const PrefillArgs &a, hipStream_t s) {
-  const int n_items = a.q_tiles * a.q_heads * a.num_seqs;
-  const int grid = (n_items + 7) / 8 * 8;
+  const int grid = prefill_grid<BM>(a);
   if (a.pool.format == kF16)
     hipLaunchKernelGGL(paged_prefill_d256_kernel<kF16>, dim3(grid), dim3(kThreads), 0, s, a);
   else
     hipLaunchKernelGGL(paged_prefill_d256_kernel<kBf16>, dim3(grid), dim3(kThreads), 0, s, a);
-  return hipGetLastError();
+  const hipError_t e = hipGetLastError();
+  return e != hipSuccess || a.max_pieces <= 1 ? e : launch_prefill_merge<D, BM, BM>(a, s);
 }
 
 }  // namespace llh

@@ -188,3 +188,58 @@ def test_rows_decode_group_of_eight(ctx, fmt):
         out = run_decode(ctx, pool, batch, q, Hq, window, 0.088)
         assert_parity(out, ref, what=f"{fmt} W{window}")
     assert ctx.device_errors() == 0, ctx.last_error()
+
+
+@pytest.mark.parametrize("window", [0, 700])
+@pytest.mark.parametrize("D,Hq,Hkv,fmt,chunk,prefix", [
+    (128, 32, 4, "bf16", [300, 0, 130, 1], [1500, 10, 900, 2000]),   # all heads packed, cut; ragged
+    (128, 6, 2, "f16", [700], [800]),                                # odd group, cut
+    (128, 16, 2, "int8", [200, 200], [1300, 1300]),
+    (256, 16, 2, "bf16", [150, 90], [1500, 30]),                     # one sequence too short to cut
+    (256, 8, 4, "f16", [400], [1000]),
+])
+def test_prefill_cut_items(ctx, opts, D, Hq, Hkv, fmt, chunk, prefix, window):
+    """Prefill calls that fill less than half the chip cut their items' keys into pieces:
+    sampled rows against the oracle, and every row against the same call under capture,
+    where items stay whole."""
+    import torch
+
+    from helpers import assert_parity
+
+    opts(llm_hip.OPT_PREFILL_HEADS_PER_WG, 2)
+    lens = np.array([p + c for p, c in zip(prefix, chunk)], np.int32)
+    batch = workloads.paged_batch(lens, BT, 0.10, 71)
+    pool, _ = build_case(ctx, batch, Hq, Hkv, FMTS[fmt], 72, head_dim=D)
+    starts = np.concatenate([[0], np.cumsum(chunk)]).astype(np.int32)
+    T = int(starts[-1])
+    q = oracle.normal_bf16(75, T * Hq * D)
+    scale = 1.0 / math.sqrt(D)
+    keep = [to_dev(a) for a in (starts, batch.seq_lens, batch.tables, q)]
+    out = torch.zeros(T * Hq * D, dtype=torch.int16, device="cuda")
+    desc = ctx.prefill_desc(keep[0], keep[1], keep[2], Hq, max(chunk), window, total_q_rows=T)
+    stream = torch.cuda.Stream()
+    ctx.paged_prefill(pool, desc, keep[3], out, scale, stream=stream)
+    stream.synchronize()
+    cut = from_dev_bf16(out)
+    assert ctx.metrics()["workspace_bytes"] > 0
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        ctx.paged_prefill(pool, desc, keep[3], out, scale, stream=torch.cuda.current_stream())
+    out.zero_()
+    graph.replay()
+    torch.cuda.synchronize()
+    whole = from_dev_bf16(out)
+    assert_parity(cut, oracle.bf16_to_f32(whole), what="cut against whole")
+    assert not np.array_equal(cut, whole), "nothing was cut"
+    k = {b: oracle.Pool.from_raw(FMTS[fmt], BT, Hkv, D, batch.n_blocks, pool.raw()) for b in (0,)}[0]
+    qr = q.reshape(T, Hq * D)
+    rows = sorted({r for b in range(len(chunk)) for r in (starts[b], starts[b] + 17, starts[b + 1] - 1)
+                   if starts[b] <= r < starts[b + 1]})
+    for r in rows:
+        b = int(np.searchsorted(starts, r, side="right") - 1)
+        n = np.array([prefix[b] + r - starts[b] + 1], np.int32)
+        st, ref = k.decode(Hq, n, batch.tables[b:b + 1], window, qr[r], scale, threads=16)
+        assert st == oracle.OK
+        assert_parity(cut.reshape(T, Hq * D)[r], ref, what=f"row {r}")
+    assert ctx.device_errors() == 0, ctx.last_error()
+    ctx.release_stream(stream)
