@@ -71,6 +71,19 @@ void read_env_options(llh_ctx *ctx) {
 constexpr int kMaxDecodeSplits = 1024;  // partials one merge workgroup combines
 constexpr int kD256MaxSplits = 64;      // partials the head_dim-256 merge combines
 
+// Whether a head_dim-128 split-K step merges in its own launch (the last workgroup of each
+// (sequence, kv head); at most 64 splits) instead of a second one.  That saves the second
+// launch, but the last workgroup reads the partials alone and past its L2, and every workgroup
+// waits for its stores: it pays for few splits and small steps.  Measured on MI355X, two
+// launches / one (us): Hq16 / Hkv8, 1 x 512 10.2 / 7.5, 1 x 1000 10.9 / 7.9, 16 x U[50, 500]
+// 10.4 / 8.5, 1 x 4000 11.8 / 14.1, 4 x 4096 in the window 15.9 / 21.1; Hq32 / Hkv8, 1 x 1000
+// 10.7 / 9.5, 4 x U[500, 1000] 11.2 / 12.3.
+bool one_launch(int group, long long pairs, int splits) {
+  if (splits < 2 || splits > 16 || pairs > kArrivalCounters) return false;
+  if (group <= 2) return pairs <= 256;
+  return pairs * splits <= (group == 4 ? 256 : 128);
+}
+
 struct SplitPlan {
   int split_blocks;
   int max_splits;
@@ -864,7 +877,7 @@ int llh::plan_decode(llh_ctx *ctx, const llh_kv_pool *pool, const llh_decode_des
 int llh::launch_planned_decode(llh_ctx *ctx, const llh_kv_pool *pool, const llh_decode_desc *desc,
                                const DecodePlan &plan, const void *d_q, void *d_out, float score_scale,
                                hipStream_t s, char *ws, int32_t *err, bool timed, const uint16_t *k_new,
-                               const uint16_t *v_new) {
+                               const uint16_t *v_new, int32_t *counters) {
   const PoolView &pv = pool->view;
   ctx->decode_calls++;
   struct TimingHook {
@@ -896,6 +909,9 @@ int llh::launch_planned_decode(llh_ctx *ctx, const llh_kv_pool *pool, const llh_
     a.max_splits = plan.max_splits;
     a.stream_wgs = plan.stream_wgs;
     a.max_seq_len = desc->max_seq_len;
+    if (!plan.d256 && !plan.stream_wgs &&
+        one_launch(plan.group, (long long)desc->num_seqs * pv.kv_heads, plan.max_splits))
+      a.counters = counters;
     a.seg_desc = plan.stream_wgs ? reinterpret_cast<int32_t *>(ws + plan.desc_off) : nullptr;
     if (plan.stream_wgs) ctx->stream_decode_calls++;
     if (plan.d256) ctx->d256_decode_calls++;
@@ -979,7 +995,8 @@ static int paged_decode_impl(llh_ctx *ctx, const llh_kv_pool *pool, const llh_de
   char *ws = lease.base();
   if (extra_ptr) *extra_ptr = ws + plan.bytes;
   if (!d_out) d_out = ws + plan.bytes;
-  return launch_planned_decode(ctx, pool, desc, plan, d_q, d_out, score_scale, s, ws, lease.err());
+  return launch_planned_decode(ctx, pool, desc, plan, d_q, d_out, score_scale, s, ws, lease.err(), true, nullptr,
+                               nullptr, lease.counters());
 }
 
 static bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -1079,13 +1096,15 @@ int llh_paged_decode_append(llh_ctx *ctx, llh_kv_pool *pool, const llh_decode_de
   if (fused) {
     ctx->fused_append_calls++;
     return launch_planned_decode(ctx, pool, desc, plan, d_q, d_out, score_scale, s, ws, lease.err(), true,
-                                 static_cast<const uint16_t *>(d_k_new), static_cast<const uint16_t *>(d_v_new));
+                                 static_cast<const uint16_t *>(d_k_new), static_cast<const uint16_t *>(d_v_new),
+                                 lease.counters());
   }
   // the append kernel finds each new token's slot through the descriptor's table rows
   st = kv_append(ctx, pool, nullptr, d_k_new, d_v_new, desc->num_seqs, 0, stream, desc->d_seq_lens,
                  desc->d_block_tables, desc->max_blocks_per_seq);
   if (st != LLH_OK) return st;
-  return launch_planned_decode(ctx, pool, desc, plan, d_q, d_out, score_scale, s, ws, lease.err());
+  return launch_planned_decode(ctx, pool, desc, plan, d_q, d_out, score_scale, s, ws, lease.err(), true, nullptr,
+                               nullptr, lease.counters());
 }
 
 int llh_matvec_bf16_f32(llh_ctx *ctx, const void *d_w, int32_t rows, int32_t cols, const void *d_x, int32_t x_f32,

@@ -969,6 +969,76 @@ __device__ __forceinline__ void load_nt(const DecodeArgs &a, int b, int kvh, int
   load_new_token_q(a, b, kvh, lane, nt, blk);
 }
 
+// One-launch split-K: the workgroup that finishes last among the n_splits of a (sequence, kv
+// head) merges them.  The partials cross XCDs, whose L2s are not coherent with each other, so
+// they are stored and loaded at agent scope (written through, and read past, the L2).  A
+// wavefront waits until its stores have completed before its workgroup counts itself in, so
+// whoever counts n_splits finds every partial in memory; no release or acquire fence is
+// needed beyond that (a release at agent scope writes the whole L2 back, ~0.45 us each, one
+// after the other on an XCD).  The last workgroup sets the counter back for the next launch.
+__device__ __forceinline__ void st_agent(float *p, float v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void st_agent(float2 *p, float2 v) {
+  __hip_atomic_store(reinterpret_cast<uint64_t *>(p), __builtin_bit_cast(uint64_t, v), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float ld_agent(const float *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float2 ld_agent(const float2 *p) {
+  return __builtin_bit_cast(float2, __hip_atomic_load(reinterpret_cast<const uint64_t *>(p), __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_AGENT));
+}
+__device__ __forceinline__ bool last_to_arrive(int32_t *counter, int n) {
+  __shared__ int s_last;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's partials have reached memory
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const int seen = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s_last = seen == n - 1;
+    if (seen == n - 1) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  return s_last != 0;
+}
+
+// decode_merge_kernel's merge of up to 64 splits (the same sums in the same order), one dim per
+// lane, on partials read at agent scope.
+__device__ __forceinline__ void merge_arrived(const DecodeArgs &a, size_t row0, int last, int d, size_t orow) {
+  const int li = d & 63;
+  const float2 ml = ld_agent(&a.ws_ml[row0 + min(li, last)]);
+  const float mx = li <= last ? ml.x : -INFINITY;
+  constexpr int N = 16;  // partial rows in flight
+  float o_sp[N];
+#pragma unroll
+  for (int i = 0; i < N; i++) o_sp[i] = ld_agent(&a.ws_o[(row0 + min(i, last)) * D + d]);
+  float mm = fmaxf(mx, dpp<0xB1>(mx));  // quad_perm [1,0,3,2]
+  mm = fmaxf(mm, dpp<0x4E>(mm));        // quad_perm [2,3,0,1]
+  mm = fmaxf(mm, dpp<0x141>(mm));       // row_half_mirror
+  mm = fmaxf(mm, dpp<0x140>(mm));       // row_mirror
+  mm = fmaxf(mm, xor16_other(mm, li));
+  mm = fmaxf(mm, xor32_other(mm, li));
+  const float mref = (mm == -INFINITY) ? 0.0f : mm;
+  const float f = li <= last ? fast_exp2(mx - mref) : 0.0f;
+  float ll = row_sum16(ml.y * f);
+  ll += xor16_other(ll, li);
+  ll += xor32_other(ll, li);
+  float oo = 0.0f;
+  for (int i0 = 0;;) {
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+      const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), (i0 + i) & 63));
+      oo += o_sp[i] * (i0 + i <= last ? w : 0.0f);
+    }
+    i0 += N;
+    if (i0 > last) break;
+#pragma unroll
+    for (int i = 0; i < N; i++) o_sp[i] = ld_agent(&a.ws_o[(row0 + min(i0 + i, last)) * D + d]);
+  }
+  a.out[orow * D + d] = f32_to_bf16_rne(gated(oo / ll, a.gate, orow * D + d));
+}
+
 template <int G, int FMT, bool FUSED = false>
 __global__ __launch_bounds__(kDecodeThreads) void paged_decode_kernel(const DecodeArgs a) {
   // consecutive workgroups are consecutive splits of one (kv head, sequence):
@@ -1123,9 +1193,19 @@ __global__ __launch_bounds__(kDecodeThreads) void paged_decode_kernel(const Deco
       a.out[(qrow0 + gi) * D + d] = f32_to_bf16_rne(gated(oo / ll, a.gate, (qrow0 + gi) * D + d));
     } else {
       const size_t row = (qrow0 + gi) * a.max_splits + split;
-      a.ws_o[row * D + d] = oo;
-      if (d == 0) a.ws_ml[row] = make_float2(mm, ll);
+      if (a.counters) {
+        st_agent(&a.ws_o[row * D + d], oo);
+        if (d == 0) st_agent(&a.ws_ml[row], make_float2(mm, ll));
+      } else {
+        a.ws_o[row * D + d] = oo;
+        if (d == 0) a.ws_ml[row] = make_float2(mm, ll);
+      }
     }
+  }
+  if (n_splits > 1 && a.counters && last_to_arrive(&a.counters[(size_t)b * a.pool.kv_heads + kvh], n_splits)) {
+    // a wavefront per 64 dims of a query head; n_splits <= 64
+    for (int it = wave; it < 2 * G; it += 4)
+      merge_arrived(a, (qrow0 + it / 2) * a.max_splits, n_splits - 1, 64 * (it % 2) + lane, qrow0 + it / 2);
   }
 }
 
@@ -1707,7 +1787,7 @@ hipError_t launch_decode_t(const DecodeArgs &a, int max_seq_len, hipStream_t s, 
   hipLaunchKernelGGL((paged_decode_kernel<G, FMT, FUSED>), grid, dim3(kDecodeThreads), 0, s, a);
   hipError_t e = hipGetLastError();
   if (hook) hook(hu, 1, s);
-  if (e != hipSuccess || a.max_splits <= 1) return e;
+  if (e != hipSuccess || a.max_splits <= 1 || a.counters) return e;
   hipLaunchKernelGGL(decode_merge_kernel, dim3(a.q_heads, a.num_seqs), dim3(D), 0, s, a);
   return hipGetLastError();
 }

@@ -40,6 +40,11 @@ struct StreamWorkspace {
   void *ptr = nullptr;
   size_t bytes = 0;
   int32_t *err = nullptr;
+  // arrival counters of the one-launch split-K decode, in err's allocation: zero between
+  // launches (the launches of a stream run one after the other; each leaves them zero)
+  int32_t *counters() const { return err + kCountersOffset; }
+  static constexpr size_t kCountersOffset = 64;
+  static constexpr size_t kErrBytes = (kCountersOffset + kArrivalCounters) * sizeof(int32_t);
   std::mutex mu;
 };
 
@@ -119,9 +124,9 @@ struct llh_ctx {
     auto w = std::make_shared<llh::StreamWorkspace>();
     w->stream = s;
     hipError_t e = hipSetDevice(device);
-    if (e == hipSuccess) e = hipMalloc(&w->err, sizeof(int32_t));
+    if (e == hipSuccess) e = hipMalloc(&w->err, llh::StreamWorkspace::kErrBytes);
     // zeroed on the slot's own stream, so it lands before the stream's first kernel
-    if (e == hipSuccess) e = hipMemsetAsync(w->err, 0, sizeof(int32_t), s);
+    if (e == hipSuccess) e = hipMemsetAsync(w->err, 0, llh::StreamWorkspace::kErrBytes, s);
     if (e != hipSuccess) {
       if (w->err) (void)hipFree(w->err);
       return nullptr;
@@ -204,6 +209,7 @@ struct WsLease {
     return false;
   }
   int32_t *err() const { return w->err; }
+  int32_t *counters() const { return w->counters(); }
   char *base() const { return static_cast<char *>(w->ptr); }
 };
 
@@ -237,10 +243,12 @@ int plan_decode(llh_ctx *ctx, const llh_kv_pool *pool, const llh_decode_desc *de
                 bool keep_fused = false);
 // err: the device error word the kernels raise flags in; timed = false leaves out
 // the kernel-timing events (no event is created or recorded); k_new / v_new
-// (tuned kernels): fused append of each sequence's new token
+// (tuned kernels): fused append of each sequence's new token; counters: the stream's arrival
+// counters (null: split-K always merges in a second launch)
 int launch_planned_decode(llh_ctx *ctx, const llh_kv_pool *pool, const llh_decode_desc *desc, const DecodePlan &plan,
                           const void *d_q, void *d_out, float score_scale, hipStream_t s, char *ws, int32_t *err,
-                          bool timed = true, const uint16_t *k_new = nullptr, const uint16_t *v_new = nullptr);
+                          bool timed = true, const uint16_t *k_new = nullptr, const uint16_t *v_new = nullptr,
+                          int32_t *counters = nullptr);
 // Resolves this device's address of the no-allocation scratch (device current).
 int noalloc_init(int device);
 

@@ -57,6 +57,9 @@ struct PoolView {
   const void *v_scales;
 };
 
+// (sequence, kv head) pairs a stream's arrival counters serve (one-launch split-K)
+constexpr int kArrivalCounters = 4096;
+
 // Split-K decode over the tuned shape (head_dim 128, 16-token blocks).
 struct DecodeArgs {
   PoolView pool;
@@ -75,6 +78,7 @@ struct DecodeArgs {
   int32_t max_splits;
   int32_t stream_wgs;       // >0: persistent stream kernel over this many workgroups (split fields unused)
   int32_t max_seq_len;      // host bound on seq_lens (stream kernel: longer lengths raise kErrTooManySplits)
+  int32_t *counters;        // split-K, head_dim 128: null, or a zero per (sequence, kv head): one launch
   int32_t *seg_desc;        // stream kernel: [B][Hkv][2] (first partial slot, partial count; 0 = written)
   float scale_log2e;        // score_scale * log2(e)
   // fused append (bf16 pools): each sequence's new token (position len - 1), [B][Hkv][128]

@@ -628,3 +628,50 @@ def test_stream_segment_cut_into_hundreds_of_pieces(ctx, opts, fmt):
     opts(llm_hip.OPT_DECODE_KERNEL, "stream")
     batch = workloads.paged_batch([32768], BT, 0.0, 63)
     check(ctx, batch, 16, 8, fmt, seed=63, what=f"1 x 32768 stream fmt={fmt}")
+
+
+@pytest.mark.parametrize("Hq,Hkv,lens", [(16, 8, [512]), (8, 8, [70, 0, 1000, 33]), (16, 4, [900]), (64, 8, [250])])
+def test_decode_one_launch_merge_equals_two(ctx, Hq, Hkv, lens):
+    """Small split-K steps are merged by the last workgroup of each (sequence, kv head); the
+    no-allocation entry merges in a second launch: the same bits, call after call (the arrival
+    counters are left zero), eager and replayed from a graph between eager calls, and on two
+    streams at once."""
+    import torch
+
+    lens = np.array(lens, np.int32)
+    batch = workloads.paged_batch(lens, BT, 0.10, 81)
+    pool, q = build_case(ctx, batch, Hq, Hkv, llm_hip.KV_BF16, 82)
+    d_lens, d_tab, d_q = to_dev(lens), to_dev(batch.tables), to_dev(q)
+    desc = ctx.decode_desc(d_lens, d_tab, Hq, int(lens.max()))
+    two = torch.zeros(q.size, dtype=torch.int16, device="cuda")
+    ctx.paged_decode_noalloc(pool, desc, d_q, two, 0.088)
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    outs = [torch.zeros_like(two) for _ in range(2)]
+    torch.cuda.synchronize()
+    for _ in range(20):
+        for s, o in zip(streams, outs):
+            with torch.cuda.stream(s):
+                o.zero_()
+            ctx.paged_decode(pool, desc, d_q, o, 0.088, stream=s)
+        torch.cuda.synchronize()
+        for o in outs:
+            assert torch.equal(o, two)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=streams[0]):
+        for _ in range(3):
+            ctx.paged_decode(pool, desc, d_q, outs[0], 0.088, stream=torch.cuda.current_stream())
+    for _ in range(4):
+        outs[0].zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(streams[0]):
+            graph.replay()
+        streams[0].synchronize()
+        assert torch.equal(outs[0], two)
+        ctx.paged_decode(pool, desc, d_q, outs[0], 0.088, stream=streams[0])
+        streams[0].synchronize()
+        assert torch.equal(outs[0], two)
+    ref = oracle_decode(pool, batch, llm_hip.KV_BF16, Hq, Hkv, 0, q, 0.088)
+    assert_parity(from_dev_bf16(two), ref, what="one launch")
+    assert ctx.device_errors() == 0, ctx.last_error()
+    for s in streams:
+        ctx.release_stream(s)
