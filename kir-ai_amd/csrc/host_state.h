@@ -41,8 +41,15 @@ struct StreamWorkspace {
   size_t bytes = 0;
   int32_t *err = nullptr;
   // arrival counters of the one-launch split-K decode, in err's allocation: zero between
-  // launches (the launches of a stream run one after the other; each leaves them zero)
-  int32_t *counters() const { return err + kCountersOffset; }
+  // launches (the launches of a stream run one after the other; each leaves them zero).
+  // None to a call under capture, whose graph may be replayed on another stream beside this
+  // one's calls, or where the slot was made under capture (the clearing waits for a replay).
+  int32_t *counters() const { return counters_zeroed && !capturing(stream) ? err + kCountersOffset : nullptr; }
+  static bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
+  }
+  bool counters_zeroed = false;
   static constexpr size_t kCountersOffset = 64;
   static constexpr size_t kErrBytes = (kCountersOffset + kArrivalCounters) * sizeof(int32_t);
   std::mutex mu;
@@ -126,7 +133,9 @@ struct llh_ctx {
     hipError_t e = hipSetDevice(device);
     if (e == hipSuccess) e = hipMalloc(&w->err, llh::StreamWorkspace::kErrBytes);
     // zeroed on the slot's own stream, so it lands before the stream's first kernel
-    if (e == hipSuccess) e = hipMemsetAsync(w->err, 0, llh::StreamWorkspace::kErrBytes, s);
+    w->counters_zeroed = !llh::StreamWorkspace::capturing(s);
+    if (e == hipSuccess)
+      e = hipMemsetAsync(w->err, 0, w->counters_zeroed ? llh::StreamWorkspace::kErrBytes : sizeof(int32_t), s);
     if (e != hipSuccess) {
       if (w->err) (void)hipFree(w->err);
       return nullptr;
@@ -198,8 +207,7 @@ struct WsLease {
   // captured (a captured launch would keep a pointer that a later call may free) and when
   // the memory cannot be had; the caller then takes a path without scratch.
   bool try_acquire(llh_ctx *ctx, hipStream_t s, size_t bytes) {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return false;
+    if (llh::StreamWorkspace::capturing(s)) return false;
     w = ctx->slot(s);
     if (!w) return false;
     lock = std::unique_lock<std::mutex>(w->mu);
