@@ -108,6 +108,13 @@ __device__ __forceinline__ SeqSplit seq_split(const RowsArgs &a, int b) {
   return s;
 }
 
+// 1 / (weight sum).  No weight at all (every key masked, or every score -inf) gives the zero
+// row of the tile prefill and the reference-order decode, and the NaN (0 / 0) of the vector
+// decode kernels in the calls that are theirs too.
+__device__ __forceinline__ float row_inv(const RowsArgs &a, float ll) {
+  return ll == 0.0f && (a.chunk_starts || a.zero_bad) ? 0.0f : 1.0f / ll;
+}
+
 // keys per unit: K and V of a unit take 64 operand registers each in 16-bit formats (32 in
 // 8-bit ones)
 template <int D>
@@ -478,7 +485,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 && is16(FMT) ? 1 : 2) void pag
     const int pr = row0 + r;
     const size_t orow = (size_t)(sq.c0 + pr / G) * a.q_heads + kvh * G + pr % G;
     if (sq.n_splits == 1) {
-      const float inv = ll > 0.0f ? 1.0f / ll : (ll == 0.0f ? 0.0f : ll);
+      const float inv = row_inv(a, ll);
       const size_t o = orow * D + d;
 #pragma unroll
       for (int x = 0; x < 4; x++) a.out[o + x] = f32_to_bf16_rne(gated(oo[x] * inv, a.gate, o + x));
@@ -515,7 +522,7 @@ __device__ __forceinline__ void rows_merge(const RowsArgs &a, size_t orow, int l
   float oo = 0.0f;
 #pragma unroll
   for (int i = 0; i < N; i++) oo += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), i)) * o_sp[i];
-  const float inv = ll > 0.0f ? 1.0f / ll : (ll == 0.0f ? 0.0f : ll);
+  const float inv = row_inv(a, ll);
   a.out[orow * D + d] = f32_to_bf16_rne(gated(oo * inv, a.gate, orow * D + d));
 }
 

@@ -190,6 +190,37 @@ def test_rows_decode_group_of_eight(ctx, fmt):
     assert ctx.device_errors() == 0, ctx.last_error()
 
 
+def test_rows_decode_no_weight_as_the_vector_kernels(ctx, opts):
+    """Every score of a group of eight -inf (q . k overflows), or +inf: NaN rows from the
+    packed-row kernel and the vector kernel alike, split or not; the other heads' rows stay."""
+    import torch
+
+    Hq, Hkv, D = 32, 4, 128
+    lens = np.array([20, 700, 3000, 90, 40], np.int32)
+    batch = workloads.paged_batch(lens, BT, 0.0, 71)
+    pool = ctx.pool(llm_hip.KV_BF16, BT, Hkv, D, batch.n_blocks)
+    ids = torch.arange(batch.n_blocks, dtype=torch.int32, device="cuda")
+    k = torch.ones(batch.n_blocks, BT, Hkv, D, dtype=torch.bfloat16, device="cuda")
+    ctx.write_blocks(pool, ids, k.view(torch.int16), k.view(torch.int16))
+    q = torch.full((lens.size, Hq, D), 0.5, dtype=torch.bfloat16, device="cuda")
+    q[:, 3] = -3e38  # 128 of them: beyond f32
+    q[:, 17] = 3e38
+    outs = {}
+    desc = ctx.decode_desc(to_dev(lens), to_dev(batch.tables), Hq, int(lens.max()))
+    for kernel in ("auto", "split"):
+        opts(llm_hip.OPT_DECODE_KERNEL, kernel)
+        out = torch.zeros(lens.size, Hq, D, dtype=torch.bfloat16, device="cuda")
+        ctx.paged_decode(pool, desc, q.view(torch.int16), out.view(torch.int16), 0.088)
+        torch.cuda.synchronize()
+        outs[kernel] = out.cpu()
+    nan = torch.zeros(lens.size, Hq, D, dtype=torch.bool)
+    nan[:, [3, 17]] = True
+    for kernel, out in outs.items():
+        assert torch.equal(out.isnan(), nan), kernel
+        assert (out[~nan] == 1).all(), kernel
+    assert ctx.device_errors() == 0, ctx.last_error()
+
+
 @pytest.mark.parametrize("window", [0, 700])
 @pytest.mark.parametrize("D,Hq,Hkv,fmt,chunk,prefix", [
     (128, 32, 4, "bf16", [300, 0, 130, 1], [1500, 10, 900, 2000]),   # all heads packed, cut; ragged
