@@ -1509,16 +1509,17 @@ struct llh_layer_cache {
   std::mutex mu;
 
   size_t vector_len() const { return kv_heads * head_dim; }
-  // Brings d_table up to date on the cache's stream, through pinned memory of the table's
-  // size that is not touched before the stream has run; no copy when no block changed since.
-  hipError_t upload_table(void *pinned) {
+  // Brings d_table up to date on the cache's stream, through host memory of the table's
+  // size (or the table itself) that is not changed before the stream has run; no copy when no
+  // block changed since.
+  hipError_t upload_table(void *from) {
     if (d_table && table_sent == table) return hipSuccess;
     hipError_t e = hipSuccess;
     if (!d_table) e = hipMalloc(&d_table, std::max<size_t>(1, table.size()) * sizeof(int32_t));
     if (e != hipSuccess) return e;
-    std::memcpy(pinned, table.data(), table.size() * sizeof(int32_t));
+    if (from != table.data()) std::memcpy(from, table.data(), table.size() * sizeof(int32_t));
     table_sent.clear();
-    e = hipMemcpyAsync(d_table, pinned, table.size() * sizeof(int32_t), hipMemcpyHostToDevice, stream);
+    e = hipMemcpyAsync(d_table, from, table.size() * sizeof(int32_t), hipMemcpyHostToDevice, stream);
     if (e == hipSuccess) table_sent = table;
     return e;
   }
@@ -1563,6 +1564,9 @@ int llh_layer_cache_create(llh_ctx *ctx, size_t max_tokens, size_t kv_heads, siz
     c->table.push_back(idx);
     c->ids.push_back(next_block_id());
   }
+  // the table's first upload, here rather than on the cache's first attention call
+  if (e == hipSuccess) e = c->upload_table(c->table.data());
+  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   if (e != hipSuccess) {
     delete c;
     return ctx->hip_fail(e, "layer cache allocation");
@@ -1888,12 +1892,15 @@ static int cache_mix_tuned(llh_ctx *ctx, llh_layer_cache *cache, const float *h_
   const size_t nb = cache->table.size();
   // The kernels read the length and q from, and write their output to, pinned host memory:
   // a few KB each way, cheaper over the bus than as two copies (a call on 500 cached tokens
-  // 27.6 -> 24.9 us).  The block table stays on the device between calls.
+  // 27.2 -> 24.3 us).  Every workgroup reads q, so the many of a long context take it from a
+  // copy: int8, Hq32, copied / read over the bus (us): 4096 tokens 35.5 / 35.7, 8192 42.6 /
+  // 44.7, 16384 60.0 / 64.8.  The block table stays on the device between calls.
+  const bool copy_q = row_count > 4096;
   const size_t off_q = kAlign;  // header: seq_len
   const size_t off_out = off_q + align_up(qdim * sizeof(uint16_t));
   const size_t out_bytes = d_w ? out_len * sizeof(float) : qdim * sizeof(uint16_t);
   const size_t off_table = off_out + align_up(out_bytes);
-  hipError_t e = cache->scratch.ensure(0, off_table + nb * sizeof(int32_t));
+  hipError_t e = cache->scratch.ensure(copy_q ? off_out : 0, off_table + nb * sizeof(int32_t));
   if (e != hipSuccess) return ctx->hip_fail(e, "scratch allocation");
   char *hb = static_cast<char *>(cache->scratch.host);
   e = cache->upload_table(hb + off_table);
@@ -1909,6 +1916,12 @@ static int cache_mix_tuned(llh_ctx *ctx, llh_layer_cache *cache, const float *h_
   std::memcpy(hb, &len, sizeof(len));
   auto *qh = reinterpret_cast<uint16_t *>(hb + off_q);
   for (size_t i = 0; i < qdim; i++) qh[i] = host_f32_to_bf16(h_query[i]);
+  const char *in = sb;
+  if (copy_q) {
+    in = static_cast<char *>(cache->scratch.dev);
+    e = hipMemcpyAsync(cache->scratch.dev, hb, off_out, hipMemcpyHostToDevice, cache->stream);
+    if (e != hipSuccess) return ctx->hip_fail(e, "attention upload");
+  }
   llh_kv_pool pool{};
   pool.ctx = ctx;
   pool.view = bs.view();
@@ -1919,15 +1932,15 @@ static int cache_mix_tuned(llh_ctx *ctx, llh_layer_cache *cache, const float *h_
   desc.max_seq_len = len;
   desc.window = (int32_t)row_count;  // attends [len - row_count, len): the first row_count logical rows
   desc.total_tokens_hint = (int32_t)row_count;
-  desc.d_seq_lens = reinterpret_cast<const int32_t *>(sb);
+  desc.d_seq_lens = reinterpret_cast<const int32_t *>(in);
   desc.d_block_tables = cache->d_table;
   int st;
   if (d_w) {
-    st = decode_projection_impl(ctx, &pool, &desc, sb + off_q, d_w, w_rows, reinterpret_cast<float *>(sb + off_out),
+    st = decode_projection_impl(ctx, &pool, &desc, in + off_q, d_w, w_rows, reinterpret_cast<float *>(sb + off_out),
                                 score_scale, cache->stream);
   } else {
     WsLease lease;
-    st = paged_decode_impl(ctx, &pool, &desc, sb + off_q, sb + off_out, score_scale, cache->stream, 0, nullptr, lease);
+    st = paged_decode_impl(ctx, &pool, &desc, in + off_q, sb + off_out, score_scale, cache->stream, 0, nullptr, lease);
   }
   if (st != LLH_OK) return st;
   e = hipStreamSynchronize(cache->stream);

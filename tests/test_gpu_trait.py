@@ -337,3 +337,46 @@ def test_trait_mix_non_finite_scores_still_error_on_the_tuned_shape(ctx, opts):
                                                                           11, 16, 8, 128, 1.0, out)
     assert e.value.status == llm_hip.ERR_NON_FINITE
     cache.close()
+
+
+@pytest.mark.parametrize("fmt", [llm_hip.KV_BF16, llm_hip.KV_INT8])
+@pytest.mark.parametrize("n,counts", [(4112, (4096, 4097, 4112)), (32, (32, 7))])
+def test_trait_mix_table_and_query_follow_the_cache(ctx, opts, fmt, n, counts):
+    """The block table stays on the device between calls and q is read over the bus up to 4096
+    rows, from a copy beyond: both sides of that, another query each call, and a clone whose
+    appends give it blocks of its own while the original keeps its rows.  Rows are N(0,1), for
+    which the bar allows the tuned path's rounding of q to bf16."""
+    opts(llm_hip.OPT_TRAIT_REFERENCE_ORDER, 0)
+    hkv = 1
+    rng = np.random.default_rng(17 + fmt)
+    rows = [oracle.bf16_to_f32(oracle.f32_to_bf16(rng.standard_normal((n, hkv * 128)).astype(np.float32)))
+            for _ in range(2)]
+    backend = HipNativeMatvecBackend(ctx)
+
+    def worst(c):
+        keys, vals = c.keys(), c.values()
+        bar = []
+        for count in counts:
+            q = rng.standard_normal(2 * 128).astype(np.float32)
+            out = np.zeros_like(q)
+            before = ctx.metrics()["trait_tuned_calls"]
+            assert backend.full_attention_cache_mix_f32_in_place(c, q, count, 2, hkv, 128, 0.0883883, out)
+            assert ctx.metrics()["trait_tuned_calls"] == before + 1
+            st, ref = oracle.attention_mix(q, keys, vals, count, 2, hkv, 128, 0.0883883)
+            assert st == oracle.OK
+            d = np.abs(out - ref)
+            bar += [d.max() / 2e-2, d.mean() / 2e-3]
+        return max(bar)
+
+    cache = LayerKvCache.from_rows(ctx, n, hkv, 128, *rows, revision=n, tokens_seen=n, fmt=fmt)
+    other = cache.clone()
+    try:
+        results = [worst(cache)]
+        for _ in range(20):  # wraps: the oldest rows' blocks are copied on write
+            k, v = (rng.standard_normal(hkv * 128).astype(np.float32) for _ in range(2))
+            backend.append_kv_cache_sliding_f32(other, k, v)
+        results += [worst(other), worst(cache)]
+    finally:  # before their context, whatever happens
+        other.close()
+        cache.close()
+    assert max(results) <= 1.0, results
