@@ -713,17 +713,17 @@ static int check_span(llh_ctx *ctx, const llh_kv_pool *pool, int32_t max_seq_len
 // Eight query heads per kv head fill half a matrix tile, and its MFMAs take the place of the
 // dot products that bound the vector kernels at this group size.  Measured on MI355X, Hq32 /
 // Hkv4, vector against packed rows (us): bf16 1 x 2000 12.0 / 12.0, 1 x 16000 41.4 / 14.6,
-// 4 x 4096 22.4 / 17.0, 32 x U[50, 500] 25.9 / 13.0, 32 x U[256, 4096] 54.9 / 38.8; int8
+// 4 x 4096 21.0 / 12.4, 32 x U[50, 500] 25.0 / 12.2, 32 x U[256, 4096] 53.9 / 44.3; int8
 // 1 x 16000 41.7 / 13.2, 32 x U[256, 4096] 58.5 / 35.7.  A few short sequences stay: bf16
 // 4 x U[500, 1000] 11.6 / 12.6.  At four heads per kv head it is faster where the sequences
 // are short enough for a unit or two per wavefront and fill the chip unsplit: Hq32 / Hkv8,
-// 32 x U[50, 500] bf16 16.6 / 14.1, int8 24.0 / 12.0, but 4 x U[500, 1000] 11.7 / 19.7 and
+// 32 x U[50, 500] bf16 15.7 / 12.9 (16 x U[50, 300] 10.4 / 11.8), int8 24.0 / 12.0, but 4 x U[500, 1000] 11.7 / 19.7 and
 // long ones 35.8 / 45.7 (16 x U[1000, 4000]); at two it is not (Hq16 / Hkv8, 32 x U[50, 500]
 // 12.3 / 14.0).
 static bool decode_prefers_rows(const PoolView &pv, int group, int num_seqs, int est_blocks) {
   const long long tiles = (long long)num_seqs * pv.kv_heads;
   if (group == 8) return tiles > 16 || est_blocks > 1024 / kFastBlockTokens + 1;
-  if (group == 4) return est_blocks <= 512 / kFastBlockTokens + 1 && tiles >= (is16(pv.format) ? 128 : 64);
+  if (group == 4) return est_blocks <= 512 / kFastBlockTokens + 1 && tiles >= (is16(pv.format) ? 256 : 64);
   return false;
 }
 

@@ -28,8 +28,8 @@
 //
 // int8 / fp8 codes enter the MFMA exactly (as bf16); their scales multiply the scores
 // and the weights in f32.  PARTS = 3 splits every f32 weight into three 16-bit terms
-// (24 bits, the whole f32 significand) for three P V products; PARTS = 1 rounds the
-// weights once, as the tuned 16-bit prefill does.
+// (24 bits, the whole f32 significand) for three P V products, PARTS = 2 into two; PARTS = 1
+// rounds the weights once, as the tuned 16-bit prefill does.
 //
 // Bound: the chain lengths -> table entry -> K / V at the start of a workgroup and, in long
 // splits, the latency of one unit's loads (one unit in flight per wavefront); HBM traffic
@@ -559,7 +559,12 @@ template <int D>
 hipError_t launch_rows_d(const RowsArgs &a, int max_rows, bool exact_weights, hipStream_t s, void *hu, LaunchHook hook) {
   switch (a.pool.format) {
     case kBf16:
-      return exact_weights ? launch_rows_t<D, kBf16, 3>(a, max_rows, s, hu, hook) : launch_rows_t<D, kBf16, 1>(a, max_rows, s, hu, hook);
+      if (exact_weights) return launch_rows_t<D, kBf16, 3>(a, max_rows, s, hu, hook);
+      // The vector decode kernels keep a maximum per four tokens, whose weights are exact more
+      // often than under this kernel's one per unit: two terms keep a decode step's error below
+      // theirs (short contexts, against f64: vector 0.00174, one term 0.00184).
+      if (D == kFastHeadDim && !a.chunk_starts) return launch_rows_t<D, kBf16, D == kFastHeadDim ? 2 : 1>(a, max_rows, s, hu, hook);
+      return launch_rows_t<D, kBf16, 1>(a, max_rows, s, hu, hook);
     case kF16:
       return exact_weights ? launch_rows_t<D, kF16, 3>(a, max_rows, s, hu, hook) : launch_rows_t<D, kF16, 1>(a, max_rows, s, hu, hook);
     case kInt8:
