@@ -72,14 +72,14 @@ constexpr int kMaxDecodeSplits = 1024;  // partials one merge workgroup combines
 constexpr int kD256MaxSplits = 64;      // partials the head_dim-256 merge combines
 
 // Whether a head_dim-128 split-K step merges in its own launch (the last workgroup of each
-// (sequence, kv head); at most 64 splits) instead of a second one.  That saves the second
-// launch, but the last workgroup reads the partials alone and past its L2, and every workgroup
-// waits for its stores: it pays for few splits and small steps.  Measured on MI355X, two
+// (sequence, kv head)) instead of a second one.  That saves the second launch, but the last
+// workgroup reads the partials alone and past its L2, and every workgroup waits for its stores:
+// it pays for few splits and small steps.  Measured on MI355X, two
 // launches / one (us): Hq16 / Hkv8, 1 x 512 10.2 / 7.5, 1 x 1000 10.9 / 7.9, 16 x U[50, 500]
 // 10.4 / 8.5, 1 x 4000 11.8 / 14.1, 4 x 4096 in the window 15.9 / 21.1; Hq32 / Hkv8, 1 x 1000
 // 10.7 / 9.5, 4 x U[500, 1000] 11.2 / 12.3.
 bool one_launch(int group, long long pairs, int splits) {
-  if (splits < 2 || splits > 16 || pairs > kArrivalCounters) return false;
+  if (splits < 2 || splits > kOneLaunchSplits || pairs > kArrivalCounters) return false;
   if (group <= 2) return pairs <= 256;
   return pairs * splits <= (group == 4 ? 256 : 128);
 }

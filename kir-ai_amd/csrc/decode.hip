@@ -1003,39 +1003,22 @@ __device__ __forceinline__ bool last_to_arrive(int32_t *counter, int n) {
   return s_last != 0;
 }
 
-// decode_merge_kernel's merge of up to 64 splits (the same sums in the same order), one dim per
-// lane, on partials read at agent scope.
+// merge_in_registers' merge (the same sums in the same order, so the same bits) of at most
+// kOneLaunchSplits splits, one dim per lane, on partials read at agent scope.
 __device__ __forceinline__ void merge_arrived(const DecodeArgs &a, size_t row0, int last, int d, size_t orow) {
   const int li = d & 63;
+  constexpr int N = kOneLaunchSplits;  // every partial row in flight
   const float2 ml = ld_agent(&a.ws_ml[row0 + min(li, last)]);
-  const float mx = li <= last ? ml.x : -INFINITY;
-  constexpr int N = 16;  // partial rows in flight
   float o_sp[N];
 #pragma unroll
   for (int i = 0; i < N; i++) o_sp[i] = ld_agent(&a.ws_o[(row0 + min(i, last)) * D + d]);
-  float mm = fmaxf(mx, dpp<0xB1>(mx));  // quad_perm [1,0,3,2]
-  mm = fmaxf(mm, dpp<0x4E>(mm));        // quad_perm [2,3,0,1]
-  mm = fmaxf(mm, dpp<0x141>(mm));       // row_half_mirror
-  mm = fmaxf(mm, dpp<0x140>(mm));       // row_mirror
-  mm = fmaxf(mm, xor16_other(mm, li));
-  mm = fmaxf(mm, xor32_other(mm, li));
-  const float mref = (mm == -INFINITY) ? 0.0f : mm;
-  const float f = li <= last ? fast_exp2(mx - mref) : 0.0f;
-  float ll = row_sum16(ml.y * f);
-  ll += xor16_other(ll, li);
-  ll += xor32_other(ll, li);
+  const float mx[1] = {li <= last ? ml.x : -INFINITY}, ly[1] = {ml.y};
+  float f[1];
+  const float ll = merge_weights<1>(mx, ly, li, f);
   float oo = 0.0f;
-  for (int i0 = 0;;) {
 #pragma unroll
-    for (int i = 0; i < N; i++) {
-      const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), (i0 + i) & 63));
-      oo += o_sp[i] * (i0 + i <= last ? w : 0.0f);
-    }
-    i0 += N;
-    if (i0 > last) break;
-#pragma unroll
-    for (int i = 0; i < N; i++) o_sp[i] = ld_agent(&a.ws_o[(row0 + min(i0 + i, last)) * D + d]);
-  }
+  for (int i = 0; i < N; i++)
+    oo += o_sp[i] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f[0]), i));
   a.out[orow * D + d] = f32_to_bf16_rne(gated(oo / ll, a.gate, orow * D + d));
 }
 
@@ -1203,7 +1186,7 @@ __global__ __launch_bounds__(kDecodeThreads) void paged_decode_kernel(const Deco
     }
   }
   if (n_splits > 1 && a.counters && last_to_arrive(&a.counters[(size_t)b * a.pool.kv_heads + kvh], n_splits)) {
-    // a wavefront per 64 dims of a query head; n_splits <= 64
+    // a wavefront per 64 dims of a query head
     for (int it = wave; it < 2 * G; it += 4)
       merge_arrived(a, (qrow0 + it / 2) * a.max_splits, n_splits - 1, 64 * (it % 2) + lane, qrow0 + it / 2);
   }
@@ -1541,27 +1524,8 @@ __device__ __forceinline__ void merge_in_registers(const DecodeArgs &a, size_t r
     mx[p] = 64 * p + li <= last ? ml.x : -INFINITY;
     ly[p] = ml.y;
   }
-  // wavefront max and sum: DPP within rows of 16, then row exchanges (no LDS)
-  float mm = mx[0];
-#pragma unroll
-  for (int p = 1; p < P; p++) mm = fmaxf(mm, mx[p]);
-  mm = fmaxf(mm, dpp<0xB1>(mm));   // quad_perm [1,0,3,2]
-  mm = fmaxf(mm, dpp<0x4E>(mm));   // quad_perm [2,3,0,1]
-  mm = fmaxf(mm, dpp<0x141>(mm));  // row_half_mirror
-  mm = fmaxf(mm, dpp<0x140>(mm));  // row_mirror
-  mm = fmaxf(mm, xor16_other(mm, li));
-  mm = fmaxf(mm, xor32_other(mm, li));
-  const float mref = (mm == -INFINITY) ? 0.0f : mm;
-  float f[P];
-  float lsum = 0.0f;
-#pragma unroll
-  for (int p = 0; p < P; p++) {
-    f[p] = 64 * p + li <= last ? fast_exp2(mx[p] - mref) : 0.0f;
-    lsum += ly[p] * f[p];
-  }
-  float ll = row_sum16(lsum);
-  ll += xor16_other(ll, li);
-  ll += xor32_other(ll, li);
+  float f[P];  // wavefront max and sum: DPP within rows of 16, then row exchanges (no LDS)
+  const float ll = merge_weights<P>(mx, ly, li, f);
   // the weights to every lane through LDS (broadcast reads)
   __shared__ __attribute__((aligned(16))) float s_w[N];
   if (d < 64) {

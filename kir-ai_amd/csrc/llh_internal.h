@@ -59,6 +59,7 @@ struct PoolView {
 
 // (sequence, kv head) pairs a stream's arrival counters serve (one-launch split-K)
 constexpr int kArrivalCounters = 4096;
+constexpr int kOneLaunchSplits = 16;  // and the most splits one of them merges
 
 // Split-K decode over the tuned shape (head_dim 128, 16-token blocks).
 struct DecodeArgs {

@@ -507,21 +507,12 @@ __device__ __forceinline__ void rows_merge(const RowsArgs &a, size_t orow, int l
   for (int i = 0; i < N; i++) o_sp[i] = a.ws_o[(p0 + min(i, last)) * D + d];
   const int li = d & 63;
   const float2 ml = a.ws_ml[p0 + min(li, last)];
-  const float mx = li <= last ? ml.x : -INFINITY;
-  float mm = fmaxf(mx, dpp<0xB1>(mx));
-  mm = fmaxf(mm, dpp<0x4E>(mm));
-  mm = fmaxf(mm, dpp<0x141>(mm));
-  mm = fmaxf(mm, dpp<0x140>(mm));
-  mm = fmaxf(mm, xor16_other(mm, li));
-  mm = fmaxf(mm, xor32_other(mm, li));
-  const float mref = (mm == -INFINITY) ? 0.0f : mm;
-  const float f = li <= last ? fast_exp2(mx - mref) : 0.0f;
-  float ll = row_sum16(f * ml.y);
-  ll += xor16_other(ll, li);
-  ll += xor32_other(ll, li);
+  const float mx[1] = {li <= last ? ml.x : -INFINITY}, ly[1] = {ml.y};
+  float f[1];
+  const float ll = merge_weights<1>(mx, ly, li, f);
   float oo = 0.0f;
 #pragma unroll
-  for (int i = 0; i < N; i++) oo += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), i)) * o_sp[i];
+  for (int i = 0; i < N; i++) oo += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f[0]), i)) * o_sp[i];
   const float inv = row_inv(a, ll);
   a.out[orow * D + d] = f32_to_bf16_rne(gated(oo * inv, a.gate, orow * D + d));
 }

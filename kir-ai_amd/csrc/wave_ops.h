@@ -116,6 +116,40 @@ __device__ __forceinline__ float row_sum_stride4(float v) {
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// a * b rounded to f32, whatever it is added to.  A product that goes straight into an exchange
+// sum would be fused into its first addition: a lane then adds its own product unrounded to its
+// neighbour's rounded one, and the lanes of a row disagree about the sum.
+__device__ __forceinline__ float rounded_product(float a, float b) {
+#pragma clang fp contract(off)
+  return a * b;
+}
+
+// Log-sum-exp weights of up to 64 P partials, P (max, sum) pairs per lane (mx = -inf in the
+// places past the last): f = 2^(mx - largest), the same in every kernel that merges; returns the
+// sum of l f over the wavefront, the same bits in every lane.
+template <int P>
+__device__ __forceinline__ float merge_weights(const float (&mx)[P], const float (&l)[P], int lane, float (&f)[P]) {
+  float mm = mx[0];
+#pragma unroll
+  for (int p = 1; p < P; p++) mm = fmaxf(mm, mx[p]);
+  mm = fmaxf(mm, dpp<0xB1>(mm));   // quad_perm [1,0,3,2]
+  mm = fmaxf(mm, dpp<0x4E>(mm));   // quad_perm [2,3,0,1]
+  mm = fmaxf(mm, dpp<0x141>(mm));  // row_half_mirror
+  mm = fmaxf(mm, dpp<0x140>(mm));  // row_mirror
+  mm = fmaxf(mm, xor16_other(mm, lane));
+  mm = fmaxf(mm, xor32_other(mm, lane));
+  const float mref = mm == -INFINITY ? 0.0f : mm;
+  float sum = 0.0f;
+#pragma unroll
+  for (int p = 0; p < P; p++) {
+    f[p] = fast_exp2(mx[p] - mref);
+    sum = p ? __builtin_fmaf(l[p], f[p], sum) : rounded_product(l[p], f[p]);
+  }
+  sum = row_sum16(sum);
+  sum += xor16_other(sum, lane);
+  return sum + xor32_other(sum, lane);
+}
+
 __device__ __forceinline__ float f16_bits_to_f32(uint32_t h) {
   return (float)__builtin_bit_cast(_Float16, (uint16_t)h);
 }

@@ -675,3 +675,32 @@ def test_decode_one_launch_merge_equals_two(ctx, Hq, Hkv, lens):
     assert ctx.device_errors() == 0, ctx.last_error()
     for s in streams:
         ctx.release_stream(s)
+
+
+@pytest.mark.parametrize("fmt", [llm_hip.KV_BF16, llm_hip.KV_INT8])
+@pytest.mark.parametrize("Hq,Hkv,lens", [(16, 8, [512]), (8, 8, [70, 0, 1000, 33]), (64, 8, [250])])
+def test_decode_one_launch_merge_over_changing_inputs(ctx, Hq, Hkv, lens, fmt):
+    """One-launch steps over two pools in turn, a new query each, back to back on one stream: the
+    workspace always holds the other step's partials, and every step must still have the bits of
+    its two-launch merge (the no-allocation entry's).  200 steps: a denominator off by an ulp
+    changes about one bf16 output in 2^16."""
+    import torch
+
+    lens = np.array(lens, np.int32)
+    cases = []
+    for seed in (83, 84):
+        batch = workloads.paged_batch(lens, BT, 0.10, seed)
+        pool, _ = build_case(ctx, batch, Hq, Hkv, fmt, seed)
+        cases.append((pool, ctx.decode_desc(to_dev(lens), to_dev(batch.tables), Hq, int(lens.max()))))
+    g = torch.Generator(device="cuda")
+    g.manual_seed(85)
+    q = torch.randn(200, lens.size * Hq * D, generator=g, device="cuda").to(torch.bfloat16).view(torch.int16)
+    one, two = torch.zeros_like(q), torch.zeros_like(q)
+    for i in range(len(q)):
+        ctx.paged_decode(*cases[i % 2], q[i], one[i], 0.088)
+    for i in range(len(q)):
+        ctx.paged_decode_noalloc(*cases[i % 2], q[i], two[i], 0.088)
+    torch.cuda.synchronize()
+    diff = (one != two).sum(1)
+    assert not diff.any(), f"{int((diff > 0).sum())} of {len(q)} steps differ, {int(diff.sum())} outputs in all"
+    assert ctx.device_errors() == 0, ctx.last_error()
