@@ -440,7 +440,8 @@ __global__ __launch_bounds__(kPrefillThreads * HPW, 2 / HPW) void paged_prefill_
   }
 
   // ---- normalise and store: lane holds dims 32mt + 8(j/4) + 4h + (j%4) of its row ----
-  if (bad && tid == 0) atomicOr(a.err, kErrBadBlock);  // a needed block was missing: its keys read as zeros
+  // a needed block was missing (its keys read as zeros): each 256 threads know of the blocks they load
+  if (bad && ltid == 0) atomicOr(a.err, kErrBadBlock);
   const float l_tot = l_run + xor32_other(l_run, lane);
   if (!row_ok) return;
   if (it.pieces > 1) {  // this piece's unnormalised sums, for prefill_merge_kernel

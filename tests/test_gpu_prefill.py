@@ -289,3 +289,31 @@ def test_prefill_span_beyond_table_row_raises_flag(ctx, opts, generic):
     ctx.paged_prefill(pool, ctx.prefill_desc(starts, clens, tab, 8, 20, 40, total_q_rows=20), q, out, 0.1)
     torch.cuda.synchronize()
     assert ctx.device_errors() == 0
+
+
+@pytest.mark.parametrize("rows_per_wg", [1, 2])
+@pytest.mark.parametrize("head_dim,Hq,Hkv,fmt", [(128, 3, 3, llm_hip.KV_BF16), (128, 6, 2, llm_hip.KV_INT8),
+                                                 (128, 8, 2, llm_hip.KV_F16), (256, 8, 2, llm_hip.KV_BF16)])
+def test_prefill_bad_block_at_every_place_of_a_tile(ctx, opts, head_dim, Hq, Hkv, fmt, rows_per_wg):
+    """A table entry outside the pool at each of the four block places of a 64-key tile, in the
+    prefix and in the chunk, over contexts too short to be cut and long enough: flagged every
+    time by the tile kernels, and never without one."""
+    import torch
+
+    opts(llm_hip.OPT_PREFILL_HEADS_PER_WG, rows_per_wg)
+    chunk = 150
+    for prefix in (64, 2500):
+        batch = workloads.paged_batch([prefix + chunk], BT, 0.10, 91)
+        pool = ctx.pool(fmt, BT, Hkv, head_dim, batch.n_blocks)
+        q = to_dev(oracle.normal_bf16(92, chunk * Hq * head_dim))
+        out = torch.zeros_like(q)
+        starts, lens = to_dev(np.array([0, chunk], np.int32)), to_dev(batch.seq_lens)
+        for place in [None, *range(4), *range(prefix // BT, prefix // BT + 4)]:
+            tables = batch.tables.copy()
+            if place is not None:
+                tables[0, place] = batch.n_blocks + 3
+            desc = ctx.prefill_desc(starts, lens, to_dev(tables), Hq, chunk, total_q_rows=chunk)
+            ctx.paged_prefill(pool, desc, q, out, 0.1)
+            torch.cuda.synchronize()
+            want = 0 if place is None else llm_hip.ERR_FLAG_BAD_BLOCK
+            assert ctx.device_errors() == want, (prefix, place)
