@@ -144,7 +144,7 @@ typedef struct llh_metrics {
                                      head_dim 256 (packed rows), else the element-wise kernel */
   uint64_t fused_append_calls;    /* llh_paged_decode_append calls served by one launch */
   uint64_t stream_slots;          /* streams holding a workspace slot (scratch and error word) now */
-  uint64_t workspace_bytes;       /* device bytes of those slots' scratch now */
+  uint64_t workspace_bytes;       /* device bytes of those slots' scratch now, the prefill's included */
   uint64_t d256_decode_calls;     /* decode calls that ran the head_dim-256 kernel */
   uint64_t generic_decode_calls;  /* llh_paged_decode* calls outside the tuned kernels' shapes: the packed-row
                                      kernel at head_dim 128 / 256 over 16-token blocks, else the element-wise one */
@@ -332,8 +332,11 @@ typedef struct llh_prefill_desc {
  * blocks and 16-byte aligned rows run MFMA kernels: 128-row tiles (int8 / fp8 at
  * head_dim 128: codes * scale rounded to bf16 as the key/value tiles are staged),
  * or, for calls of few rows and for int8 / fp8 at head_dim 256, packed 16-row
- * tiles over split keys, whose partial results live in the stream's workspace (a
- * stream under capture gets none: its calls do not split).  Every other shape with
+ * tiles over split keys.  Calls that split keys keep partial results in scratch of
+ * the stream's slot that is the prefill's own: made on the first such call (at most
+ * 77 MB in two buffers on 256 compute units), never grown, moved or freed before the
+ * slot, and no part of the workspace that decode calls reserve.  A stream under capture
+ * and hipStreamPerThread get none: their calls do not split.  Every other shape with
  * head_dim <= 512 runs an element-wise kernel (sequential f32 dot products, online softmax in
  * f32); head_dim > 512 returns LLH_ERR_UNSUPPORTED. */
 int llh_paged_prefill(llh_ctx *ctx, const llh_kv_pool *pool, const llh_prefill_desc *desc, const void *d_q,

@@ -242,7 +242,8 @@ SplitRows split_prefill_rows(const llh_ctx *ctx, const PoolView &pv, const llh_p
   r.max_splits = (int)std::min<long long>({(long long)kRowsMaxSplits, std::max(1LL, slots / tiles), (units + 3) / 4});
   r.single_units = rows_single(ctx, tiles);
   if (units <= r.single_units) r.max_splits = 1;
-  const size_t rows = r.max_splits > 1 ? (size_t)d->total_q_rows * d->num_q_heads * r.max_splits : 0;
+  // at most 16 rows per workgroup: within the scratch wherever there is more than one split
+  const size_t rows = r.max_splits > 1 ? (size_t)d->num_seqs * d->max_chunk_len * d->num_q_heads * r.max_splits : 0;
   r.o_off = align_up(rows * sizeof(float2));
   r.bytes = align_up(r.o_off + rows * pv.head_dim * sizeof(float));
   return r;
@@ -315,6 +316,8 @@ int llh_ctx_destroy(llh_ctx *ctx) {
   for (hipEvent_t e : ctx->event_pool) (void)hipEventDestroy(e);
   for (auto &w : ctx->workspaces) {
     if (w->ptr) (void)hipFree(w->ptr);
+    for (void *p : w->prefill)
+      if (p) (void)hipFree(p);
     if (w->err) (void)hipFree(w->err);
   }
   if (ctx->d_err) (void)hipFree(ctx->d_err);
@@ -382,10 +385,14 @@ static int release_slot(llh_ctx *ctx, hipStream_t stream, bool stream_alive) {
     ctx->retired_flags |= flags;
   }
   if (w->ptr) (void)hipFree(w->ptr);
+  for (void *&p : w->prefill) {
+    if (p) (void)hipFree(p);
+    p = nullptr;
+  }
   if (w->err) (void)hipFree(w->err);
   w->ptr = nullptr;
   w->err = nullptr;
-  w->bytes = 0;
+  w->bytes = w->prefill_bytes = 0;
   return LLH_OK;
 }
 
@@ -452,7 +459,7 @@ int llh_ctx_metrics(const llh_ctx *ctx, llh_metrics *out) {
   std::lock_guard<std::mutex> g(const_cast<llh_ctx *>(ctx)->ws_mu);
   out->stream_slots = ctx->workspaces.size();
   out->workspace_bytes = 0;
-  for (auto &w : ctx->workspaces) out->workspace_bytes += w->bytes;
+  for (auto &w : ctx->workspaces) out->workspace_bytes += w->bytes + w->prefill_bytes;
   return LLH_OK;
 }
 
@@ -950,7 +957,8 @@ int llh::launch_planned_decode(llh_ctx *ctx, const llh_kv_pool *pool, const llh_
     r.scale = score_scale;
     r.scale_log2e = score_scale * 1.4426950408889634f;
     r.gate = static_cast<const uint16_t *>(desc->d_gate);
-    const hipError_t e = launch_rows(r, 1, plan.exact, s, timed ? &th : nullptr, timed ? hook : nullptr);
+    r.max_rows = 1;
+    const hipError_t e = launch_rows(r, plan.exact, s, timed ? &th : nullptr, timed ? hook : nullptr);
     if (e != hipSuccess) return ctx->hip_fail(e, "decode launch");
     return LLH_OK;
   }
@@ -1191,6 +1199,7 @@ int llh_paged_prefill(llh_ctx *ctx, const llh_kv_pool *pool, const llh_prefill_d
   auto ev = ctx->timing_begin(static_cast<hipStream_t>(stream));
   hipError_t e;
   WsLease lease;
+  char *scratch = nullptr;
   SplitRows sr{};
   // int8 / fp8 blocks at head_dim 256 always run the packed-row kernel, unsplit where no
   // scratch may be taken
@@ -1199,7 +1208,9 @@ int llh_paged_prefill(llh_ctx *ctx, const llh_kv_pool *pool, const llh_prefill_d
   bool rows = rows_only || ((fast || fast256) && prefill_takes_rows(ctx, pv, desc));
   if (rows) {
     sr = split_prefill_rows(ctx, pv, desc);
-    if (!lease.try_acquire(ctx, static_cast<hipStream_t>(stream), sr.bytes)) {
+    if (sr.max_splits > 1 && sr.bytes <= prefill_scratch_bytes(ctx->cus, kRowsScratch))
+      scratch = lease.prefill_scratch(ctx, static_cast<hipStream_t>(stream), kRowsScratch);
+    if (sr.max_splits > 1 && !scratch) {
       rows = rows_only;
       sr.max_splits = 1;
     }
@@ -1208,7 +1219,7 @@ int llh_paged_prefill(llh_ctx *ctx, const llh_kv_pool *pool, const llh_prefill_d
   // Items of `bm` rows, all heads of a kv head packed.  Where they make at most half as many
   // groups of `cut` rows as there are compute units and the contexts may be long enough, they
   // are cut into as many pieces as still give one workgroup per compute unit (more than that is
-  // a second round), with the partial sums in the stream's workspace (none under capture).
+  // a second round), with the partial sums in the stream's scratch (none under capture).
   // Else, where they do not fill the compute units, only `least` heads are packed.  Measured on
   // MI355X, least heads packed / all / all, cut (us): head_dim 128, Hq32 / Hkv4, 1 x (4096 + 512)
   // 132 / 103 / 58, 8 x (1024 + 64) 38 / - / 33, 8 x (256 + 64) 17.3 / 19.7 / 29.6,
@@ -1217,7 +1228,6 @@ int llh_paged_prefill(llh_ctx *ctx, const llh_kv_pool *pool, const llh_prefill_d
   auto plan_pieces = [&](int bm, int cut, int least) {
     const int G = desc->num_q_heads / pv.kv_heads;
     const long long groups = (long long)pv.kv_heads * desc->num_seqs;
-    const long long tiles = std::max(1LL, ((long long)desc->max_chunk_len * G + bm - 1) / bm);
     // every sequence's last group may be partial; a uniform batch is counted exactly
     const long long cuts = std::max<long long>(
         1, (long long)desc->total_q_rows == (long long)desc->max_chunk_len * desc->num_seqs
@@ -1232,15 +1242,13 @@ int llh_paged_prefill(llh_ctx *ctx, const llh_kv_pool *pool, const llh_prefill_d
     };
     if (pieces < 2 || desc->num_seqs > 64 || keys / 64 < prefill_cut_tiles((int)pieces, pv.head_dim))
       return whole(cuts >= ctx->cus ? G : least);
-    a.pack = G;
-    a.q_tiles = (int32_t)tiles;
-    const size_t rows = (size_t)(tiles * groups * pieces * bm);
-    const size_t o_off = align_up(rows * sizeof(float2));
-    if (!lease.try_acquire(ctx, static_cast<hipStream_t>(stream), o_off + rows * pv.head_dim * sizeof(float)))
-      return whole(least);
+    scratch = lease.prefill_scratch(ctx, static_cast<hipStream_t>(stream), kCutScratch);
+    if (!scratch) return whole(least);
+    whole(G);
     a.max_pieces = (int32_t)pieces;
-    a.ws_ml = reinterpret_cast<float2 *>(lease.base());
-    a.ws_o = reinterpret_cast<float *>(lease.base() + o_off);
+    a.ws_pieces = 2 * ctx->cus;
+    a.ws_ml = reinterpret_cast<float2 *>(scratch);
+    a.ws_o = reinterpret_cast<float *>(scratch + align_up((size_t)a.ws_pieces * cut * sizeof(float2)));
   };
   if (rows) {
     RowsArgs r{};
@@ -1251,8 +1259,8 @@ int llh_paged_prefill(llh_ctx *ctx, const llh_kv_pool *pool, const llh_prefill_d
     r.context_lens = a.context_lens;
     r.tables = a.tables;
     if (sr.max_splits > 1) {
-      r.ws_o = reinterpret_cast<float *>(lease.base() + sr.o_off);
-      r.ws_ml = reinterpret_cast<float2 *>(lease.base());
+      r.ws_o = reinterpret_cast<float *>(scratch + sr.o_off);
+      r.ws_ml = reinterpret_cast<float2 *>(scratch);
     }
     r.err = a.err;
     r.num_seqs = a.num_seqs;
@@ -1265,7 +1273,8 @@ int llh_paged_prefill(llh_ctx *ctx, const llh_kv_pool *pool, const llh_prefill_d
     r.scale = score_scale;
     r.scale_log2e = a.scale_log2e;
     r.gate = a.gate;
-    e = launch_rows(r, desc->max_chunk_len, /*exact_weights=*/false, static_cast<hipStream_t>(stream));
+    r.max_rows = desc->max_chunk_len;
+    e = launch_rows(r, /*exact_weights=*/false, static_cast<hipStream_t>(stream));
   } else if (fast) {
     const bool narrow = ctx->opt(LLH_OPT_PREFILL_HEADS_PER_WG) == 1;
     // both workgroup sizes pack and cut alike, and give the same bits

@@ -27,6 +27,18 @@ inline size_t align_up(size_t x) { return (x + kAlign - 1) / kAlign * kAlign; }
 // crates/llm-kv-cache/src/block_id.rs:11-41).
 uint64_t next_block_id();
 
+// The prefill kernels' scratch of a stream, two buffers: partial rows of the packed-row kernel,
+// partial sums of the tile kernels' cut items.  Both are bounded by the compute units, whatever
+// the call's sizes: splits and cuts serve calls that do not fill the chip.
+enum PrefillScratch { kRowsScratch, kCutScratch, kPrefillScratches };
+inline size_t prefill_scratch_bytes(int cus, PrefillScratch which) {
+  // rows of D floats and (max, sum).  Rows kernel: at most two workgroups of 16 rows per compute
+  // unit are split.  Tile kernels: as many cut pieces as compute units, by an estimate of the
+  // items that is at most half of them short (pieces of 256 rows at head_dim 128, 128 at 256).
+  return which == kRowsScratch ? align_up((size_t)2 * cus * 16 * (kD256HeadDim + 2) * sizeof(float))
+                               : align_up((size_t)2 * cus * 256 * (kFastHeadDim + 2) * sizeof(float));
+}
+
 // Device scratch of one stream: split partials, merge descriptors and the
 // fused projection's staging, plus the stream's own device error word (the
 // sticky flags the kernels of this stream's calls raise).  A call holds `mu`
@@ -40,6 +52,11 @@ struct StreamWorkspace {
   void *ptr = nullptr;
   size_t bytes = 0;
   int32_t *err = nullptr;
+  // Scratch of the prefill kernels that split their keys, apart from `ptr`, which a captured
+  // decode may hold: made on the first call that splits, of a size that every such call keeps to,
+  // and never moved or freed before the slot is.
+  void *prefill[kPrefillScratches] = {};
+  size_t prefill_bytes = 0;
   // arrival counters of the one-launch split-K decode, in err's allocation: zero between
   // launches (the launches of a stream run one after the other; each leaves them zero).
   // None to a call under capture, whose graph may be replayed on another stream beside this
@@ -203,18 +220,25 @@ struct WsLease {
     lock = std::unique_lock<std::mutex>(w->mu);
     return ctx->grow_locked(*w, bytes);
   }
-  // The stream's workspace grown to `bytes`, or nothing: false while the stream is being
-  // captured (a captured launch would keep a pointer that a later call may free) and when
-  // the memory cannot be had; the caller then takes a path without scratch.
-  bool try_acquire(llh_ctx *ctx, hipStream_t s, size_t bytes) {
-    if (llh::StreamWorkspace::capturing(s)) return false;
+  // The stream's prefill scratch, or null: while the stream is being captured (the graph may be
+  // replayed beside this stream's calls), on the handle that stands for another stream in each
+  // thread, and when the memory cannot be had; the caller then takes a path without scratch.
+  char *prefill_scratch(llh_ctx *ctx, hipStream_t s, llh::PrefillScratch which) {
+    if (s == hipStreamPerThread || llh::StreamWorkspace::capturing(s)) return nullptr;
     w = ctx->slot(s);
-    if (!w) return false;
+    if (!w) return nullptr;
     lock = std::unique_lock<std::mutex>(w->mu);
-    if (ctx->grow_locked(*w, bytes) == LLH_OK) return true;
-    (void)hipGetLastError();
-    lock.unlock();
-    return false;
+    void *&p = w->prefill[which];
+    if (p) return static_cast<char *>(p);
+    const size_t bytes = llh::prefill_scratch_bytes(ctx->cus, which);
+    if (hipSetDevice(ctx->device) != hipSuccess || hipMalloc(&p, bytes) != hipSuccess) {
+      p = nullptr;
+      (void)hipGetLastError();
+      lock.unlock();
+      return nullptr;
+    }
+    w->prefill_bytes += bytes;
+    return static_cast<char *>(p);
   }
   int32_t *err() const { return w->err; }
   int32_t *counters() const { return w->counters(); }

@@ -131,15 +131,16 @@ struct PrefillArgs {
   int32_t q_tiles;          // row tiles per (sequence, head group) in the grid
   int32_t pack;             // query heads of a kv head packed into an item's rows
   int32_t max_pieces;       // > 1: items may be cut into at most this many pieces (prefill_items.h)
-  float *ws_o;              // max_pieces > 1: [items][max_pieces][rows][D] partial outputs
-  float2 *ws_ml;            // [items][max_pieces][rows] (max in log2 units, sum)
+  int32_t ws_pieces;        // max_pieces > 1: pieces (of a group's rows) that ws_o and ws_ml hold
+  float *ws_o;              // [cut groups][max_pieces][rows][D] partial outputs
+  float2 *ws_ml;            // [cut groups][max_pieces][rows] (max in log2 units, sum)
   float scale_log2e;
   float scale;              // score_scale (generic kernel)
   const uint16_t *gate;     // null, or [T][Hq][D] bf16: out = attention * sigmoid(gate)
 };
 
 // Packed query rows over split keys (rows.hip): decode steps outside the tuned shapes
-// and prefill calls of few rows.  Workspace: partial rows [T][Hq][max_splits].
+// and prefill calls of few rows.  Workspace: partial rows [num_seqs][max_rows][Hq][max_splits].
 constexpr int kRowsMaxSplits = 64;
 struct RowsArgs {
   PoolView pool;            // head_dim 128 or 256, 16-token blocks, any format but int8 rows
@@ -148,10 +149,11 @@ struct RowsArgs {
   const int32_t *chunk_starts;  // [num_seqs + 1], or null: decode, one row per sequence
   const int32_t *context_lens;  // [num_seqs]
   const int32_t *tables;
-  float *ws_o;              // [T][Hq][max_splits][D]
-  float2 *ws_ml;            // [T][Hq][max_splits]  (max in log2 units, sum)
+  float *ws_o;              // [num_seqs][max_rows][Hq][max_splits][D]
+  float2 *ws_ml;            // [num_seqs][max_rows][Hq][max_splits]  (max in log2 units, sum)
   int32_t *err;
   int32_t num_seqs;
+  int32_t max_rows;         // host bound on a sequence's query rows: further ones are not computed
   int32_t q_heads;
   int32_t max_blocks;
   int32_t window;
@@ -244,9 +246,8 @@ int matvec_ksplit(int rows, int cols, int n, int cus);
 // `hook(user, 0, s)` runs just before and `hook(user, 1, s)` just after the main
 // decode kernel is enqueued (before the merge): kernel timing records events there.
 typedef void (*LaunchHook)(void *user, int phase, hipStream_t s);
-// max_rows: host bound on a sequence's query rows; exact_weights: softmax weights keep
-// f32 precision in p . v (always so for int8 / fp8 blocks)
-hipError_t launch_rows(const RowsArgs &a, int max_rows, bool exact_weights, hipStream_t s, void *hook_user = nullptr,
+// exact_weights: softmax weights keep f32 precision in p . v (always so for int8 / fp8 blocks)
+hipError_t launch_rows(const RowsArgs &a, bool exact_weights, hipStream_t s, void *hook_user = nullptr,
                        LaunchHook hook = nullptr);
 hipError_t launch_decode(const DecodeArgs &a, int group, int max_seq_len, hipStream_t s, void *hook_user = nullptr,
                          LaunchHook hook = nullptr);

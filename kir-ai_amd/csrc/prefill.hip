@@ -445,7 +445,7 @@ __global__ __launch_bounds__(kPrefillThreads * HPW, 2 / HPW) void paged_prefill_
   const float l_tot = l_run + xor32_other(l_run, lane);
   if (!row_ok) return;
   if (it.pieces > 1) {  // this piece's unnormalised sums, for prefill_merge_kernel
-    const size_t p = (size_t)it.slot * BM + wave * 32 + col;
+    const size_t p = (size_t)it.slot + wave * 32 + col;
     if (h == 0) a.ws_ml[p] = make_float2(m_run, l_tot);
 #pragma unroll
     for (int mt = 0; mt < 4; mt++)
@@ -590,7 +590,7 @@ __global__ __launch_bounds__(256) void prefill_generic_kernel(const PrefillArgs 
 
 hipError_t launch_prefill(const PrefillArgs &a, int variant, hipStream_t s) {
   const bool wide = variant == kPrefillRows256;
-  const int grid = wide ? prefill_grid<256>(a) : prefill_grid<128>(a);
+  const int grid = wide ? prefill_grid<256, 256>(a) : prefill_grid<128, 256>(a);
   switch (a.pool.format) {
     case kBf16:
       launch_prefill_fmt<kBf16>(a, variant, grid, s);

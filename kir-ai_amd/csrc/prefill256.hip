@@ -379,7 +379,7 @@ __global__ __launch_bounds__(kThreads, 1) void paged_prefill_d256_kernel(const P
   const float l_tot = row_sum4(l_run);
   if (!row_ok) return;
   if (it.pieces > 1) {  // this piece's unnormalised sums, for prefill_merge_kernel
-    const size_t p = (size_t)it.slot * BM + wave * ROWS + r;
+    const size_t p = (size_t)it.slot + wave * ROWS + r;
     if (g == 0) a.ws_ml[p] = make_float2(m_run, l_tot);
 #pragma unroll
     for (int db = 0; db < 16; db++) *reinterpret_cast<f32x4_t *>(&a.ws_o[p * D + db * 16 + 4 * g]) = oacc[db];
@@ -401,7 +401,7 @@ __global__ __launch_bounds__(kThreads, 1) void paged_prefill_d256_kernel(const P
 }  // namespace
 
 hipError_t launch_prefill_d256(const PrefillArgs &a, hipStream_t s) {
-  const int grid = prefill_grid<BM>(a);
+  const int grid = prefill_grid<BM, BM>(a);
   if (a.pool.format == kF16)
     hipLaunchKernelGGL(paged_prefill_d256_kernel<kF16>, dim3(grid), dim3(kThreads), 0, s, a);
   else

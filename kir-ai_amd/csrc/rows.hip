@@ -149,7 +149,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 && is16(FMT) ? 1 : 2) void pag
     if (sq.flags && tid == 0) atomicOr(a.err, sq.flags);
     return;
   }
-  const int rows = sq.chunk * G;
+  const int rows = min(sq.chunk, a.max_rows) * G;
   const int row0 = tile * TILE;
   if (row0 >= rows || split >= max(sq.n_splits, 1)) return;
   if (sq.units == 0) {  // empty context: zero output (weighted sum of nothing)
@@ -482,15 +482,15 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 && is16(FMT) ? 1 : 2) void pag
       ll += s_l[w][r] * f;
       oo += *reinterpret_cast<const f32x4_t *>(&s_o[w][r][d]) * f;
     }
-    const int pr = row0 + r;
-    const size_t orow = (size_t)(sq.c0 + pr / G) * a.q_heads + kvh * G + pr % G;
+    const int tok = (row0 + r) / G;
+    const int head = kvh * G + (row0 + r) % G;
     if (sq.n_splits == 1) {
       const float inv = row_inv(a, ll);
-      const size_t o = orow * D + d;
+      const size_t o = ((size_t)(sq.c0 + tok) * a.q_heads + head) * D + d;
 #pragma unroll
       for (int x = 0; x < 4; x++) a.out[o + x] = f32_to_bf16_rne(gated(oo[x] * inv, a.gate, o + x));
     } else {
-      const size_t p = orow * a.max_splits + split;
+      const size_t p = (((size_t)b * a.max_rows + tok) * a.q_heads + head) * a.max_splits + split;
       *reinterpret_cast<f32x4_t *>(&a.ws_o[p * D + d]) = oo;
       if (d == 0) a.ws_ml[p] = make_float2(mm, ll);
     }
@@ -500,8 +500,8 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 && is16(FMT) ? 1 : 2) void pag
 // Merge of the n <= N splits of one (query row, head): every partial row in flight at
 // once, the (max, sum) pairs one per lane, split weights through v_readlane.
 template <int D, int N>
-__device__ __forceinline__ void rows_merge(const RowsArgs &a, size_t orow, int last, int d) {
-  const size_t p0 = orow * a.max_splits;
+__device__ __forceinline__ void rows_merge(const RowsArgs &a, size_t prow, size_t orow, int last, int d) {
+  const size_t p0 = prow * a.max_splits;
   float o_sp[N];
 #pragma unroll
   for (int i = 0; i < N; i++) o_sp[i] = a.ws_o[(p0 + min(i, last)) * D + d];
@@ -523,45 +523,46 @@ __global__ __launch_bounds__(D) void paged_rows_merge_kernel(const RowsArgs a) {
   const SeqSplit sq = seq_split<UK>(a, b);
   const int tok = blockIdx.x / a.q_heads;
   if (sq.skip || tok >= sq.chunk || sq.n_splits <= 1) return;
-  const size_t orow = (size_t)sq.c0 * a.q_heads + blockIdx.x;
+  const size_t prow = (size_t)b * a.max_rows * a.q_heads + blockIdx.x;  // row of the partials
+  const size_t orow = (size_t)sq.c0 * a.q_heads + blockIdx.x;           // and of the output
   const int last = sq.n_splits - 1;
   const int d = threadIdx.x;
-  if (last < 8) return rows_merge<D, 8>(a, orow, last, d);
-  if (last < 16) return rows_merge<D, 16>(a, orow, last, d);
-  if (last < 32) return rows_merge<D, 32>(a, orow, last, d);
-  return rows_merge<D, kRowsMaxSplits>(a, orow, last, d);
+  if (last < 8) return rows_merge<D, 8>(a, prow, orow, last, d);
+  if (last < 16) return rows_merge<D, 16>(a, prow, orow, last, d);
+  if (last < 32) return rows_merge<D, 32>(a, prow, orow, last, d);
+  return rows_merge<D, kRowsMaxSplits>(a, prow, orow, last, d);
 }
 
 template <int D, int FMT, int PARTS>
-hipError_t launch_rows_t(const RowsArgs &a, int max_rows, hipStream_t s, void *hu, LaunchHook hook) {
-  const int tiles = (max_rows * (a.q_heads / a.pool.kv_heads) + TILE - 1) / TILE;
+hipError_t launch_rows_t(const RowsArgs &a, hipStream_t s, void *hu, LaunchHook hook) {
+  const int tiles = (a.max_rows * (a.q_heads / a.pool.kv_heads) + TILE - 1) / TILE;
   if (hook) hook(hu, 0, s);
   hipLaunchKernelGGL((paged_rows_kernel<D, FMT, PARTS>), dim3(a.max_splits * a.pool.kv_heads * tiles, a.num_seqs),
                      dim3(64 * WAVES), 0, s, a);
   hipError_t e = hipGetLastError();
   if (hook) hook(hu, 1, s);
   if (e != hipSuccess || a.max_splits <= 1) return e;
-  hipLaunchKernelGGL((paged_rows_merge_kernel<D, kUnitKeys<D>>), dim3(max_rows * a.q_heads, a.num_seqs), dim3(D), 0, s,
+  hipLaunchKernelGGL((paged_rows_merge_kernel<D, kUnitKeys<D>>), dim3(a.max_rows * a.q_heads, a.num_seqs), dim3(D), 0, s,
                      a);
   return hipGetLastError();
 }
 
 template <int D>
-hipError_t launch_rows_d(const RowsArgs &a, int max_rows, bool exact_weights, hipStream_t s, void *hu, LaunchHook hook) {
+hipError_t launch_rows_d(const RowsArgs &a, bool exact_weights, hipStream_t s, void *hu, LaunchHook hook) {
   switch (a.pool.format) {
     case kBf16:
-      if (exact_weights) return launch_rows_t<D, kBf16, 3>(a, max_rows, s, hu, hook);
+      if (exact_weights) return launch_rows_t<D, kBf16, 3>(a, s, hu, hook);
       // The vector decode kernels keep a maximum per four tokens, whose weights are exact more
       // often than under this kernel's one per unit: two terms keep a decode step's error below
       // theirs (short contexts, against f64: vector 0.00174, one term 0.00184).
-      if (D == kFastHeadDim && !a.chunk_starts) return launch_rows_t<D, kBf16, D == kFastHeadDim ? 2 : 1>(a, max_rows, s, hu, hook);
-      return launch_rows_t<D, kBf16, 1>(a, max_rows, s, hu, hook);
+      if (D == kFastHeadDim && !a.chunk_starts) return launch_rows_t<D, kBf16, D == kFastHeadDim ? 2 : 1>(a, s, hu, hook);
+      return launch_rows_t<D, kBf16, 1>(a, s, hu, hook);
     case kF16:
-      return exact_weights ? launch_rows_t<D, kF16, 3>(a, max_rows, s, hu, hook) : launch_rows_t<D, kF16, 1>(a, max_rows, s, hu, hook);
+      return exact_weights ? launch_rows_t<D, kF16, 3>(a, s, hu, hook) : launch_rows_t<D, kF16, 1>(a, s, hu, hook);
     case kInt8:
-      return launch_rows_t<D, kInt8, 3>(a, max_rows, s, hu, hook);
+      return launch_rows_t<D, kInt8, 3>(a, s, hu, hook);
     case kFp8:
-      return launch_rows_t<D, kFp8, 3>(a, max_rows, s, hu, hook);
+      return launch_rows_t<D, kFp8, 3>(a, s, hu, hook);
   }
   return hipErrorInvalidValue;
 }
@@ -570,10 +571,10 @@ hipError_t launch_rows_d(const RowsArgs &a, int max_rows, bool exact_weights, hi
 
 int rows_unit_keys(int head_dim) { return head_dim == 256 ? 32 : 64; }
 
-hipError_t launch_rows(const RowsArgs &a, int max_rows, bool exact_weights, hipStream_t s, void *hu, LaunchHook hook) {
-  if (a.max_splits < 1 || a.max_splits > kRowsMaxSplits || max_rows < 1) return hipErrorInvalidValue;
-  return a.pool.head_dim == 256 ? launch_rows_d<256>(a, max_rows, exact_weights, s, hu, hook)
-                                : launch_rows_d<128>(a, max_rows, exact_weights, s, hu, hook);
+hipError_t launch_rows(const RowsArgs &a, bool exact_weights, hipStream_t s, void *hu, LaunchHook hook) {
+  if (a.max_splits < 1 || a.max_splits > kRowsMaxSplits || a.max_rows < 1) return hipErrorInvalidValue;
+  return a.pool.head_dim == 256 ? launch_rows_d<256>(a, exact_weights, s, hu, hook)
+                                : launch_rows_d<128>(a, exact_weights, s, hu, hook);
 }
 
 }  // namespace llh

@@ -274,3 +274,85 @@ def test_prefill_cut_items(ctx, opts, D, Hq, Hkv, fmt, chunk, prefix, window):
         assert_parity(cut.reshape(T, Hq * D)[r], ref, what=f"row {r}")
     assert ctx.device_errors() == 0, ctx.last_error()
     ctx.release_stream(stream)
+
+
+def prefill_call(ctx, fmt, D, Hq, Hkv, chunk, prefix, seed, max_chunk=None, table_blocks=None):
+    """(batch, pool, q, out, desc) of a ragged prefill call on the device; table_blocks: row
+    width of the block tables (default: the longest context's)."""
+    import torch
+
+    lens = np.array([p + c for p, c in zip(prefix, chunk)], np.int32)
+    batch = workloads.paged_batch(lens, BT, 0.10, seed)
+    pool, _ = build_case(ctx, batch, Hq, Hkv, fmt, seed + 1, head_dim=D)
+    tables = batch.tables
+    if table_blocks is not None:
+        tables = np.full((lens.size, table_blocks), -1, np.int32)
+        tables[:, :batch.tables.shape[1]] = batch.tables
+    starts = np.concatenate([[0], np.cumsum(chunk)]).astype(np.int32)
+    T = int(starts[-1])
+    q = to_dev(oracle.normal_bf16(seed + 2, T * Hq * D))
+    desc = ctx.prefill_desc(to_dev(starts), to_dev(batch.seq_lens), to_dev(tables), Hq, max_chunk or max(chunk),
+                            total_q_rows=T)
+    return batch, pool, q, torch.zeros_like(q), desc
+
+
+@pytest.mark.parametrize("D,Hq,Hkv,n,chunk", [(128, 32, 4, 32, 481), (256, 16, 2, 64, 449)])
+def test_prefill_scratch_is_bounded_and_its_own(ctx, opts, D, Hq, Hkv, n, chunk):
+    """One long chunk beside many single tokens, cut into pieces, with a tight and a loose bound on
+    the chunks, between replays of a decode captured on the same stream: the decode's workspace stays
+    where it is, and the prefill's scratch is made once, a fixed number of rows per compute unit."""
+    import torch
+
+    from helpers import assert_parity
+
+    stream = torch.cuda.Stream()
+    lens = np.array([3000, 70, 900], np.int32)
+    batch = workloads.paged_batch(lens, BT, 0.10, 101)
+    pool, q = build_case(ctx, batch, 16, 8, llm_hip.KV_BF16, 102)
+    d_q = to_dev(q)
+    d_out = torch.zeros_like(d_q)
+    desc = ctx.decode_desc(to_dev(lens), to_dev(batch.tables), 16, 3000)
+    ctx.paged_decode(pool, desc, d_q, d_out, 0.088, stream=stream)
+    stream.synchronize()
+    want = d_out.clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        ctx.paged_decode(pool, desc, d_q, d_out, 0.088, stream=torch.cuda.current_stream())
+
+    def replay():
+        d_out.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            graph.replay()
+        stream.synchronize()
+        assert torch.equal(d_out, want)
+
+    replay()
+    m0 = ctx.metrics()
+    chunks = [1] * n
+    chunks[n // 2] = chunk
+    outs, used = [], []
+    for max_chunk in (chunk, 4096):
+        _, ppool, pq, pout, pdesc = prefill_call(ctx, llm_hip.KV_BF16, D, Hq, Hkv, chunks, [1300] * n, 103, max_chunk)
+        ctx.paged_prefill(ppool, pdesc, pq, pout, 0.088, stream=stream)
+        stream.synchronize()
+        replay()
+        outs.append(pout.clone())
+        used.append(ctx.metrics()["workspace_bytes"] - m0["workspace_bytes"])
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert 0 < used[0] <= cus * (2 * 256 * 130 * 4 + 2 * 16 * 258 * 4) and used[1] == used[0], used
+    assert torch.equal(*outs)
+    g2 = torch.cuda.CUDAGraph()  # under capture the items stay whole
+    with torch.cuda.graph(g2, stream=stream):
+        ctx.paged_prefill(ppool, pdesc, pq, pout, 0.088, stream=torch.cuda.current_stream())
+    pout.zero_()
+    g2.replay()
+    torch.cuda.synchronize()
+    assert_parity(from_dev_bf16(outs[0]), oracle.bf16_to_f32(from_dev_bf16(pout)), what="cut against whole")
+    assert not torch.equal(outs[0], pout), "nothing was cut"
+    replay()
+    m1 = ctx.metrics()
+    assert m1["device_errors"] == m0["device_errors"] and ctx.device_errors() == 0, ctx.last_error()
+    ctx.release_stream(stream)
+    assert ctx.metrics()["workspace_bytes"] < m1["workspace_bytes"] - used[0] + 1
+
