@@ -150,6 +150,15 @@ typedef struct llh_metrics {
                                      kernel at head_dim 128 / 256 over 16-token blocks, else the element-wise one */
 } llh_metrics;
 int llh_ctx_metrics(const llh_ctx *ctx, llh_metrics *out);
+/* Calls that took a path chosen by size (tests of the choice; llh_metrics keeps its layout). */
+typedef enum llh_route {
+  LLH_ROUTE_ROWS_DECODE = 0,  /* decode steps on the packed-row kernel */
+  LLH_ROUTE_ROWS_PREFILL = 1, /* prefill calls on it */
+  LLH_ROUTE_ONE_LAUNCH = 2,   /* split-K decode steps merged in their own launch */
+  LLH_ROUTE_CUT_PREFILL = 3,  /* prefill calls whose long items may be cut into pieces */
+  LLH_ROUTE_COUNT = 4
+} llh_route;
+int llh_debug_route_calls(const llh_ctx *ctx, int32_t route, uint64_t *calls);
 /* Sticky error flags the batched kernels raise instead of faulting: 1 = a
  * block table entry outside the pool, 2 = a sequence longer than the call's
  * max_seq_len allows, 4 = a non-finite value (score, or a row given to an

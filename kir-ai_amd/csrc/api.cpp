@@ -463,6 +463,13 @@ int llh_ctx_metrics(const llh_ctx *ctx, llh_metrics *out) {
   return LLH_OK;
 }
 
+int llh_debug_route_calls(const llh_ctx *ctx, int32_t route, uint64_t *calls) {
+  if (!ctx || !calls) return LLH_ERR_NULL;
+  if (route < 0 || route >= LLH_ROUTE_COUNT) return LLH_ERR_INVALID_SHAPE;
+  *calls = ctx->routes[route].load();
+  return LLH_OK;
+}
+
 int llh_ctx_device_errors(llh_ctx *ctx, int32_t *flags, int32_t reset) {
   if (!ctx || !flags) return LLH_ERR_NULL;
   *flags = 0;
@@ -919,6 +926,7 @@ int llh::launch_planned_decode(llh_ctx *ctx, const llh_kv_pool *pool, const llh_
     if (!plan.d256 && !plan.stream_wgs &&
         one_launch(plan.group, (long long)desc->num_seqs * pv.kv_heads, plan.max_splits))
       a.counters = counters;
+    if (a.counters) ctx->routes[LLH_ROUTE_ONE_LAUNCH]++;
     a.seg_desc = plan.stream_wgs ? reinterpret_cast<int32_t *>(ws + plan.desc_off) : nullptr;
     if (plan.stream_wgs) ctx->stream_decode_calls++;
     if (plan.d256) ctx->d256_decode_calls++;
@@ -934,6 +942,7 @@ int llh::launch_planned_decode(llh_ctx *ctx, const llh_kv_pool *pool, const llh_
   }
   if (plan.rows) {
     if (plan.exact) ctx->generic_decode_calls++;
+    ctx->routes[LLH_ROUTE_ROWS_DECODE]++;
     RowsArgs r{};
     r.pool = pv;
     r.q = static_cast<const uint16_t *>(d_q);
@@ -1245,12 +1254,14 @@ int llh_paged_prefill(llh_ctx *ctx, const llh_kv_pool *pool, const llh_prefill_d
     scratch = lease.prefill_scratch(ctx, static_cast<hipStream_t>(stream), kCutScratch);
     if (!scratch) return whole(least);
     whole(G);
+    ctx->routes[LLH_ROUTE_CUT_PREFILL]++;
     a.max_pieces = (int32_t)pieces;
     a.ws_pieces = 2 * ctx->cus;
     a.ws_ml = reinterpret_cast<float2 *>(scratch);
     a.ws_o = reinterpret_cast<float *>(scratch + align_up((size_t)a.ws_pieces * cut * sizeof(float2)));
   };
   if (rows) {
+    ctx->routes[LLH_ROUTE_ROWS_PREFILL]++;
     RowsArgs r{};
     r.pool = pv;
     r.q = a.q;

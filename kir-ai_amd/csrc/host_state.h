@@ -81,6 +81,7 @@ struct llh_ctx {
   std::atomic<uint64_t> decode_calls{0}, prefill_calls{0}, append_calls{0}, not_handled{0}, device_errors{0},
       shape_errors{0}, stream_decode_calls{0}, trait_tuned_calls{0}, generic_prefill_calls{0}, fused_append_calls{0},
       d256_decode_calls{0}, generic_decode_calls{0};
+  std::atomic<uint64_t> routes[LLH_ROUTE_COUNT] = {};
   std::atomic<int32_t> options[LLH_OPT_COUNT] = {};
 
   // per-stream workspaces; ws_mu guards the list, ws_min_bytes and retired_flags

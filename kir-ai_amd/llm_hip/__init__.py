@@ -55,6 +55,7 @@ OPT_FORCE_GENERIC = 3
 OPT_PREFILL_HEADS_PER_WG = 4
 OPT_TRAIT_REFERENCE_ORDER = 5
 DECODE_KERNELS = {"auto": 0, "split": 1, "stream": 2}
+ROUTES = ("rows_decode", "rows_prefill", "one_launch", "cut_prefill")  # llh_route
 
 _STATUS_NAMES = {
     NOT_HANDLED: "not handled",
@@ -301,6 +302,7 @@ SIGNATURES = {
     "llh_ctx_get_option": (ctypes.c_int, [_P, _I32, ctypes.POINTER(_I32)]),
     "llh_decode_workspace_bytes": (_SZ, [_I32, _I32, _I32]),
     "llh_ctx_metrics": (ctypes.c_int, [_P, ctypes.POINTER(Metrics)]),
+    "llh_debug_route_calls": (ctypes.c_int, [_P, _I32, ctypes.POINTER(_U64)]),
     "llh_ctx_device_errors": (ctypes.c_int, [_P, ctypes.POINTER(_I32), _I32]),
     "llh_ctx_stream_device_errors": (ctypes.c_int, [_P, _P, ctypes.POINTER(_I32), _I32]),
     "llh_ctx_set_kernel_timing": (ctypes.c_int, [_P, _I32]),
@@ -480,6 +482,14 @@ class Context:
         m = Metrics()
         self.check(self.lib.llh_ctx_metrics(self.handle, ctypes.byref(m)))
         return {f: getattr(m, f) for f, _ in Metrics._fields_}
+
+    def route_calls(self) -> dict[str, int]:
+        """Calls that took each path chosen by size (llh_route)."""
+        n, out = _U64(), {}
+        for i, name in enumerate(ROUTES):
+            self.check(self.lib.llh_debug_route_calls(self.handle, i, ctypes.byref(n)))
+            out[name] = n.value
+        return out
 
     def device_errors(self, reset: bool = True) -> int:
         """OR of every stream's sticky device flags (waits for the device)."""

@@ -648,6 +648,7 @@ def test_decode_one_launch_merge_equals_two(ctx, Hq, Hkv, lens):
     streams = [torch.cuda.Stream() for _ in range(2)]
     outs = [torch.zeros_like(two) for _ in range(2)]
     torch.cuda.synchronize()
+    before = ctx.route_calls()["one_launch"]
     for _ in range(20):
         for s, o in zip(streams, outs):
             with torch.cuda.stream(s):
@@ -656,10 +657,12 @@ def test_decode_one_launch_merge_equals_two(ctx, Hq, Hkv, lens):
         torch.cuda.synchronize()
         for o in outs:
             assert torch.equal(o, two)
+    assert ctx.route_calls()["one_launch"] == before + 40
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph, stream=streams[0]):
         for _ in range(3):
             ctx.paged_decode(pool, desc, d_q, outs[0], 0.088, stream=torch.cuda.current_stream())
+    assert ctx.route_calls()["one_launch"] == before + 40
     for _ in range(4):
         outs[0].zero_()
         torch.cuda.synchronize()
@@ -696,11 +699,13 @@ def test_decode_one_launch_merge_over_changing_inputs(ctx, Hq, Hkv, lens, fmt):
     g.manual_seed(85)
     q = torch.randn(200, lens.size * Hq * D, generator=g, device="cuda").to(torch.bfloat16).view(torch.int16)
     one, two = torch.zeros_like(q), torch.zeros_like(q)
+    before = ctx.route_calls()["one_launch"]
     for i in range(len(q)):
         ctx.paged_decode(*cases[i % 2], q[i], one[i], 0.088)
     for i in range(len(q)):
         ctx.paged_decode_noalloc(*cases[i % 2], q[i], two[i], 0.088)
     torch.cuda.synchronize()
+    assert ctx.route_calls()["one_launch"] == before + len(q)
     diff = (one != two).sum(1)
     assert not diff.any(), f"{int((diff > 0).sum())} of {len(q)} steps differ, {int(diff.sum())} outputs in all"
     assert ctx.device_errors() == 0, ctx.last_error()

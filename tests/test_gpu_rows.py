@@ -125,7 +125,8 @@ def test_rows_prefill(ctx, opts, D, Hq, Hkv, fmt, window):
 
     from helpers import assert_parity
 
-    chunk = [8, 0, 1, 13, 5]
+    # few keys (a window of 33) at head_dim 256: packed rows only below 32 row tiles
+    chunk = [3, 0, 1, 2, 5] if D == 256 and window else [8, 0, 1, 13, 5]
     prefix = [0, 40, 2100, 243, 507]
     lens = np.array([p + c for p, c in zip(prefix, chunk)], np.int32)
     batch = workloads.paged_batch(lens, BT, 0.10, 31)
@@ -143,9 +144,11 @@ def test_rows_prefill(ctx, opts, D, Hq, Hkv, fmt, window):
     assert st == oracle.OK
     ref = ref.ravel() / (1.0 + np.exp(-oracle.bf16_to_f32(gate).astype(np.float64)))
     stream = torch.cuda.Stream()
+    before = ctx.route_calls()["rows_prefill"]
     with torch.cuda.stream(stream):
         ctx.paged_prefill(pool, desc, keep[3], out, scale, stream=stream)
     stream.synchronize()
+    assert ctx.route_calls()["rows_prefill"] == before + 1
     rows = from_dev_bf16(out)
     assert_parity(rows, ref.astype(np.float32), what="packed rows")
     if D == 256 and fmt in ("int8", "fp8"):  # no tile kernel: packed rows always, f32 weights
@@ -154,6 +157,8 @@ def test_rows_prefill(ctx, opts, D, Hq, Hkv, fmt, window):
     out.zero_()
     ctx.paged_prefill(pool, desc, keep[3], out, scale)
     torch.cuda.synchronize()
+    rows_only = D == 256 and fmt in ("int8", "fp8")
+    assert ctx.route_calls()["rows_prefill"] == before + 1 + rows_only
     tiles = from_dev_bf16(out)
     assert_parity(tiles, ref.astype(np.float32), what="128-row tiles")
     opts(llm_hip.OPT_PREFILL_HEADS_PER_WG, 0)
@@ -172,7 +177,7 @@ def test_rows_prefill(ctx, opts, D, Hq, Hkv, fmt, window):
 
 
 @pytest.mark.parametrize("fmt", FMTS)
-def test_rows_decode_group_of_eight(ctx, fmt):
+def test_rows_decode_group_of_eight(ctx, opts, fmt):
     """Groups of eight at head_dim 128, which the planner gives to the packed-row kernel,
     against the vector kernels (forced) and the oracle: edge lengths, one long sequence,
     a window."""
@@ -185,8 +190,38 @@ def test_rows_decode_group_of_eight(ctx, fmt):
     pool, q = build_case(ctx, batch, Hq, Hkv, FMTS[fmt], 62, head_dim=D)
     for window in (0, 100):
         ref = oracle_decode(pool, batch, FMTS[fmt], Hq, Hkv, window, q, 0.088, head_dim=D)
+        outs = {}
+        for kernel in ("auto", "split", "stream"):
+            opts(llm_hip.OPT_DECODE_KERNEL, kernel)
+            before = ctx.route_calls()["rows_decode"]
+            outs[kernel] = run_decode(ctx, pool, batch, q, Hq, window, 0.088)
+            assert ctx.route_calls()["rows_decode"] - before == (kernel == "auto"), kernel
+            assert_parity(outs[kernel], ref, what=f"{fmt} W{window} {kernel}")
+            assert_parity(outs["auto"], oracle.bf16_to_f32(outs[kernel]), what=f"{fmt} W{window} rows, {kernel}")
+    assert ctx.device_errors() == 0, ctx.last_error()
+
+
+@pytest.mark.parametrize("fmt,tiles", [("bf16", 256), ("f16", 256), ("int8", 64), ("fp8", 64)])
+def test_rows_decode_group_of_four_rule(ctx, fmt, tiles):
+    """Groups of four at head_dim 128 take the packed-row kernel from `tiles` (sequence, kv head)
+    pairs up and up to 512 attended tokens: one below and at either line, and a window of that
+    length over longer contexts; each against the oracle."""
+    from helpers import assert_parity
+    from test_gpu_decode import run_decode
+
+    Hq, Hkv, D = 32, 8, 128
+    n = tiles // Hkv
+    for seqs, longest, window, rows in ((n, 512, 0, 1), (n - 1, 512, 0, 0), (n, 513, 0, 0), (n, 800, 512, 1),
+                                        (n, 800, 513, 0)):
+        lens = np.resize(np.array(EDGES[:-2] + [longest], np.int32), seqs)
+        lens[0] = longest
+        batch = workloads.paged_batch(lens, BT, 0.10, 65)
+        pool, q = build_case(ctx, batch, Hq, Hkv, FMTS[fmt], 66, head_dim=D)
+        before = ctx.route_calls()["rows_decode"]
         out = run_decode(ctx, pool, batch, q, Hq, window, 0.088)
-        assert_parity(out, ref, what=f"{fmt} W{window}")
+        what = f"{fmt} {seqs} x {longest} W{window}"
+        assert ctx.route_calls()["rows_decode"] - before == rows, what
+        assert_parity(out, oracle_decode(pool, batch, FMTS[fmt], Hq, Hkv, window, q, 0.088, head_dim=D), what=what)
     assert ctx.device_errors() == 0, ctx.last_error()
 
 
@@ -249,8 +284,10 @@ def test_prefill_cut_items(ctx, opts, D, Hq, Hkv, fmt, chunk, prefix, window):
     out = torch.zeros(T * Hq * D, dtype=torch.int16, device="cuda")
     desc = ctx.prefill_desc(keep[0], keep[1], keep[2], Hq, max(chunk), window, total_q_rows=T)
     stream = torch.cuda.Stream()
+    before = ctx.route_calls()["cut_prefill"]
     ctx.paged_prefill(pool, desc, keep[3], out, scale, stream=stream)
     stream.synchronize()
+    assert ctx.route_calls()["cut_prefill"] == before + 1
     cut = from_dev_bf16(out)
     assert ctx.metrics()["workspace_bytes"] > 0
     graph = torch.cuda.CUDAGraph()
@@ -262,14 +299,14 @@ def test_prefill_cut_items(ctx, opts, D, Hq, Hkv, fmt, chunk, prefix, window):
     whole = from_dev_bf16(out)
     assert_parity(cut, oracle.bf16_to_f32(whole), what="cut against whole")
     assert not np.array_equal(cut, whole), "nothing was cut"
-    k = {b: oracle.Pool.from_raw(FMTS[fmt], BT, Hkv, D, batch.n_blocks, pool.raw()) for b in (0,)}[0]
+    opool = oracle.Pool.from_raw(FMTS[fmt], BT, Hkv, D, batch.n_blocks, pool.raw())
     qr = q.reshape(T, Hq * D)
     rows = sorted({r for b in range(len(chunk)) for r in (starts[b], starts[b] + 17, starts[b + 1] - 1)
                    if starts[b] <= r < starts[b + 1]})
     for r in rows:
         b = int(np.searchsorted(starts, r, side="right") - 1)
         n = np.array([prefix[b] + r - starts[b] + 1], np.int32)
-        st, ref = k.decode(Hq, n, batch.tables[b:b + 1], window, qr[r], scale, threads=16)
+        st, ref = opool.decode(Hq, n, batch.tables[b:b + 1], window, qr[r], scale, threads=16)
         assert st == oracle.OK
         assert_parity(cut.reshape(T, Hq * D)[r], ref, what=f"row {r}")
     assert ctx.device_errors() == 0, ctx.last_error()
