@@ -60,8 +60,11 @@ struct StreamWorkspace {
   // arrival counters of the one-launch split-K decode, in err's allocation: zero between
   // launches (the launches of a stream run one after the other; each leaves them zero).
   // None to a call under capture, whose graph may be replayed on another stream beside this
-  // one's calls, or where the slot was made under capture (the clearing waits for a replay).
-  int32_t *counters() const { return counters_zeroed && !capturing(stream) ? err + kCountersOffset : nullptr; }
+  // one's calls, or where the slot was made under capture (the clearing waits for a replay), or
+  // on hipStreamPerThread, the one handle that is another stream in every thread.
+  int32_t *counters() const {
+    return counters_zeroed && stream != hipStreamPerThread && !capturing(stream) ? err + kCountersOffset : nullptr;
+  }
   static bool capturing(hipStream_t s) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     return hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;

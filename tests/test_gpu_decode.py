@@ -709,3 +709,33 @@ def test_decode_one_launch_merge_over_changing_inputs(ctx, Hq, Hkv, lens, fmt):
     diff = (one != two).sum(1)
     assert not diff.any(), f"{int((diff > 0).sum())} of {len(q)} steps differ, {int(diff.sum())} outputs in all"
     assert ctx.device_errors() == 0, ctx.last_error()
+
+
+def test_per_thread_stream_handle_shares_no_counters(ctx):
+    """hipStreamPerThread is one handle and another stream in every thread: a counter that two
+    threads' steps both raised would end every later step's merge early or never.  Steps on it
+    merge in a second launch, and short prefill chunks are not split."""
+    import torch
+
+    per_thread = 2  # hipStreamPerThread
+    lens = np.array([512], np.int32)
+    batch = workloads.paged_batch(lens, BT, 0.10, 86)
+    pool, q = build_case(ctx, batch, 16, 8, llm_hip.KV_BF16, 86)
+    d_q = to_dev(q)
+    one, two = torch.zeros_like(d_q), torch.zeros_like(d_q)
+    desc = ctx.decode_desc(to_dev(lens), to_dev(batch.tables), 16, 512)
+    ctx.paged_decode(pool, desc, d_q, one, 0.088)
+    before = ctx.route_calls()
+    for _ in range(3):
+        two.zero_()
+        torch.cuda.synchronize()
+        ctx.paged_decode(pool, desc, d_q, two, 0.088, stream=per_thread)
+        torch.cuda.synchronize()
+        assert torch.equal(one, two)
+    pdesc = ctx.prefill_desc(to_dev(np.array([0, 1], np.int32)), to_dev(lens), to_dev(batch.tables), 16, 1)
+    ctx.paged_prefill(pool, pdesc, d_q, two, 0.088, stream=per_thread)
+    torch.cuda.synchronize()
+    assert_parity(from_dev_bf16(two), oracle.bf16_to_f32(from_dev_bf16(one)), what="prefill")
+    assert ctx.route_calls() == before
+    assert ctx.device_errors() == 0, ctx.last_error()
+    ctx.release_stream(per_thread)
