@@ -78,7 +78,8 @@ typedef enum llh_kv_format {
                           conversion does).  The tuned decode and prefill kernels compute q . k on
                           fp16 with each query head (prefill: each query row) scaled into fp16 by a
                           power of two: elements within 2^-28 of the largest |q| are exact, smaller
-                          ones err by under 2^-38 of it; softmax weights enter p . v as fp16.  Device
+                          ones err by under 2^-38 of it; softmax weights enter p . v as fp16.  The
+                          packed-row decode outside their shapes keeps q and f32 weights.  Device
                           pools only: a layer cache of this format is UNSUPPORTED, as
                           LayerKvCache::new_with_config refuses it (layer.rs:399-403) */
 } llh_kv_format;

@@ -3,10 +3,10 @@
 // The query rows that share a kv head -- the G heads of a decode token, or the heads of
 // a short prefill chunk -- are packed sixteen to a tile (row r = token * G + head), and
 // the keys of a sequence are split over workgroups and, inside one, over its four
-// wavefronts.  A wavefront walks units of 64 keys (32 at head_dim 256): it loads the unit's K and V straight into MFMA operand registers (every
-// byte is used by one wavefront, so LDS would only add a copy), and the next unit's
-// loads are in flight behind the current unit's math.  Wavefronts merge in LDS, splits
-// in paged_rows_merge_kernel.
+// wavefronts.  A wavefront walks units of 64 keys (32 at head_dim 256): it loads the unit's
+// K and V straight into MFMA operand registers (every byte is used by one wavefront, so LDS
+// would only add a copy), and the next unit's loads are in flight behind the current unit's
+// math.  Wavefronts merge in LDS, splits in paged_rows_merge_kernel.
 //
 // It serves
 //  * decode steps outside the tuned kernels' shapes (head_dim 128 or 256, 16-token
@@ -27,9 +27,11 @@
 // operand without leaving its lane.
 //
 // int8 / fp8 codes enter the MFMA exactly (as bf16); their scales multiply the scores
-// and the weights in f32.  PARTS = 3 splits every f32 weight into three 16-bit terms
-// (24 bits, the whole f32 significand) for three P V products, PARTS = 2 into two; PARTS = 1
-// rounds the weights once, as the tuned 16-bit prefill does.
+// and the weights in f32.  PARTS = 3 splits every f32 weight into three bf16 terms
+// (24 bits, the whole f32 significand) for three P V products, PARTS = 2 into two (16 bits);
+// PARTS = 1 rounds the weights once, as the tuned 16-bit prefill does.  Beside three terms an
+// fp16 element enters as two bf16 terms (8 + 3 bits, exact), so that q stays as it is and small
+// weights keep their bits, which fp16 terms would lose below 2^-14.
 //
 // Bound: the chain lengths -> table entry -> K / V at the start of a workgroup and, in long
 // splits, the latency of one unit's loads (one unit in flight per wavefront); HBM traffic
@@ -75,6 +77,23 @@ __device__ __forceinline__ u32x4_t codes8(uint32_t lo, uint32_t hi) {
   else
     return u32x4_t{fp8x2_to_bf16<false>(lo), fp8x2_to_bf16<true>(lo), fp8x2_to_bf16<false>(hi),
                    fp8x2_to_bf16<true>(hi)};
+}
+
+// Eight fp16 elements as eight bf16 terms and the rest, both exact; an infinity or a NaN is all
+// in the first.
+__device__ __forceinline__ void f16x8_to_bf16(const u32x4_t &w, u32x4_t &hi, u32x4_t &lo) {
+#pragma unroll
+  for (int x = 0; x < 4; x++) {
+    uint32_t h[2], l[2];
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+      const float v = f16_bits_to_f32(w[x] >> (16 * e) & 0xffffu);
+      h[e] = __float_as_uint(v) & 0xffff0000u;
+      l[e] = (h[e] & 0x7f800000u) == 0x7f800000u ? 0u : __float_as_uint(v - __uint_as_float(h[e]));
+    }
+    hi[x] = h[0] >> 16 | h[1];
+    lo[x] = l[0] >> 16 | l[1];
+  }
 }
 
 // The keys of a sequence and their split, the same in every kernel of a call.
@@ -123,7 +142,8 @@ constexpr int kUnitKeys = D == 256 ? 32 : 64;
 template <int D, int FMT, int PARTS>
 __global__ __launch_bounds__(64 * WAVES, D == 256 && is16(FMT) ? 1 : 2) void paged_rows_kernel(const RowsArgs a) {
   constexpr bool Q8 = !is16(FMT);
-  constexpr int OP = FMT == kF16 ? kF16 : kBf16;
+  constexpr bool WIDE16 = FMT == kF16 && PARTS == 3;  // fp16 elements as two bf16 terms
+  constexpr int OP = FMT == kF16 && !WIDE16 ? kF16 : kBf16;
   constexpr int UK = kUnitKeys<D>;
   constexpr int NT = UK / 16;          // score tiles of 16 keys
   constexpr int NS = UK / 32;          // P V steps of 32 keys
@@ -187,7 +207,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 && is16(FMT) ? 1 : 2) void pag
       qb[ks] = *reinterpret_cast<const u32x4_t *>(qr + (Q8 ? 64 * (ks >> 1) + 16 * g + 8 * (ks & 1) : 32 * ks + 8 * g));
   }
   float c = a.scale_log2e, c_nat = a.scale;
-  if constexpr (FMT == kF16) {  // the row's q scaled into fp16 (lanes col + 16 g hold its dims)
+  if constexpr (OP == kF16) {  // the row's q scaled into fp16 (lanes col + 16 g hold its dims)
     uint32_t w[4 * KS];
 #pragma unroll
     for (int ks = 0; ks < KS; ks++)
@@ -293,6 +313,11 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 && is16(FMT) ? 1 : 2) void pag
         if constexpr (Q8) {
           acc[j] = mfma16<OP>(codes8<FMT>(kr[j][x][0], kr[j][x][1]), qb[2 * x], acc[j]);
           acc[j] = mfma16<OP>(codes8<FMT>(kr[j][x][2], kr[j][x][3]), qb[2 * x + 1], acc[j]);
+        } else if constexpr (WIDE16) {
+          u32x4_t hi, lo;
+          f16x8_to_bf16(kr[j][x], hi, lo);
+          acc[j] = mfma16<OP>(hi, qb[x], acc[j]);
+          acc[j] = mfma16<OP>(lo, qb[x], acc[j]);
         } else {
           acc[j] = mfma16<OP>(kr[j][x], qb[x], acc[j]);
         }
@@ -357,7 +382,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 && is16(FMT) ? 1 : 2) void pag
         if constexpr (PARTS > 1 || Q8) l_run += p[x];
         // the scale of a slot that is not attended may be anything
         if constexpr (Q8)
-          p[x] = (sc[8 * s + x] == -INFINITY) | ((vmiss >> s & 1u) != 0) ? 0.0f : p[x] * scale_of(8 * s + x, 1);
+          p[x] = ((sc[8 * s + x] == -INFINITY) | ((vmiss >> s & 1u) != 0)) ? 0.0f : p[x] * scale_of(8 * s + x, 1);
       }
 #pragma unroll
       for (int q = 0; q < PARTS; q++) {
@@ -367,13 +392,8 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 && is16(FMT) ? 1 : 2) void pag
           pb[s][q][x] = w;
           if constexpr (PARTS == 1 && !Q8) l_run = dot2_ones_16<OP>(w, l_run);
           if (q + 1 < PARTS) {  // the rest of the weight, exactly
-            if constexpr (OP == kF16) {
-              p[2 * x] -= f16_bits_to_f32(w & 0xffffu);
-              p[2 * x + 1] -= f16_bits_to_f32(w >> 16);
-            } else {
-              p[2 * x] -= bf16_lo(w);
-              p[2 * x + 1] -= bf16_hi(w);
-            }
+            p[2 * x] -= bf16_lo(w);
+            p[2 * x + 1] -= bf16_hi(w);
           }
         }
       }
@@ -394,27 +414,34 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 && is16(FMT) ? 1 : 2) void pag
 #pragma unroll
         for (int e = 0; e < PW; e++) {
           const int p = p0 + PW * w + e;
-          mask |= !miss & (p >= tile_lo0) & (p < sq.ctx) ? (Q8 ? 0xffu : 0xffffu) << (32 / PW * e) : 0u;
+          mask |= (!miss & (p >= tile_lo0) & (p < sq.ctx)) ? (Q8 ? 0xffu : 0xffffu) << (32 / PW * e) : 0u;
         }
         vmask[i][w] = mask;
       }
     }
 #pragma unroll
     for (int s = 0; s < NS; s++) {
-      constexpr int GRP = 4;  // output tiles whose independent products hide each other's latency
+      // output tiles whose independent products hide each other's latency
+      constexpr int GRP = WIDE16 ? 2 : 4;
 #pragma unroll
       for (int d0 = 0; d0 < ND; d0 += GRP) {
-        u32x4_t va[GRP];
+        u32x4_t va[GRP], vl[GRP];
 #pragma unroll
         for (int d = 0; d < GRP; d++) {
           const vword_t v = vr[s][d0 + d] & vmask[s];
           if constexpr (Q8) va[d] = codes8<FMT>(v[0], v[1]);
+          else if constexpr (WIDE16) f16x8_to_bf16(v, va[d], vl[d]);
           else va[d] = v;
         }
 #pragma unroll
-        for (int q = 0; q < PARTS; q++)
+        for (int q = 0; q < PARTS; q++) {
 #pragma unroll
           for (int d = 0; d < GRP; d++) oacc[d0 + d] = mfma16<OP>(va[d], pb[s][q], oacc[d0 + d]);
+          if constexpr (WIDE16) {
+#pragma unroll
+            for (int d = 0; d < GRP; d++) oacc[d0 + d] = mfma16<OP>(vl[d], pb[s][q], oacc[d0 + d]);
+          }
+        }
       }
     }
   };
@@ -542,23 +569,30 @@ hipError_t launch_rows_t(const RowsArgs &a, hipStream_t s, void *hu, LaunchHook 
   hipError_t e = hipGetLastError();
   if (hook) hook(hu, 1, s);
   if (e != hipSuccess || a.max_splits <= 1) return e;
-  hipLaunchKernelGGL((paged_rows_merge_kernel<D, kUnitKeys<D>>), dim3(a.max_rows * a.q_heads, a.num_seqs), dim3(D), 0, s,
-                     a);
+  hipLaunchKernelGGL((paged_rows_merge_kernel<D, kUnitKeys<D>>), dim3(a.max_rows * a.q_heads, a.num_seqs), dim3(D), 0,
+                     s, a);
   return hipGetLastError();
+}
+
+// 16-bit pools: PARTS by the caller's need.  The vector decode kernels keep a maximum per four
+// tokens, whose weights are exact more often than under this kernel's one per unit: two terms
+// keep a decode step's error below theirs (short contexts, against f64: bf16, vector 0.00174, one
+// term 0.00184).
+template <int D, int FMT>
+hipError_t launch_rows_16(const RowsArgs &a, bool exact_weights, hipStream_t s, void *hu, LaunchHook hook) {
+  if (exact_weights) return launch_rows_t<D, FMT, 3>(a, s, hu, hook);
+  if constexpr (D == kFastHeadDim && FMT == kBf16)
+    if (!a.chunk_starts) return launch_rows_t<D, FMT, 2>(a, s, hu, hook);
+  return launch_rows_t<D, FMT, 1>(a, s, hu, hook);
 }
 
 template <int D>
 hipError_t launch_rows_d(const RowsArgs &a, bool exact_weights, hipStream_t s, void *hu, LaunchHook hook) {
   switch (a.pool.format) {
     case kBf16:
-      if (exact_weights) return launch_rows_t<D, kBf16, 3>(a, s, hu, hook);
-      // The vector decode kernels keep a maximum per four tokens, whose weights are exact more
-      // often than under this kernel's one per unit: two terms keep a decode step's error below
-      // theirs (short contexts, against f64: vector 0.00174, one term 0.00184).
-      if (D == kFastHeadDim && !a.chunk_starts) return launch_rows_t<D, kBf16, D == kFastHeadDim ? 2 : 1>(a, s, hu, hook);
-      return launch_rows_t<D, kBf16, 1>(a, s, hu, hook);
+      return launch_rows_16<D, kBf16>(a, exact_weights, s, hu, hook);
     case kF16:
-      return exact_weights ? launch_rows_t<D, kF16, 3>(a, s, hu, hook) : launch_rows_t<D, kF16, 1>(a, s, hu, hook);
+      return launch_rows_16<D, kF16>(a, exact_weights, s, hu, hook);
     case kInt8:
       return launch_rows_t<D, kInt8, 3>(a, s, hu, hook);
     case kFp8:

@@ -393,3 +393,54 @@ def test_prefill_scratch_is_bounded_and_its_own(ctx, opts, D, Hq, Hkv, n, chunk)
     ctx.release_stream(stream)
     assert ctx.metrics()["workspace_bytes"] < m1["workspace_bytes"] - used[0] + 1
 
+
+# groups that the packed-row kernel serves in place of the reference-order kernel (f32 weights),
+# and of the vector kernels (8 and 4 at head_dim 128); sequences enough for the rules
+ROW_GROUPS = [(256, 8, 4, 2), (128, 12, 4, 2), (128, 32, 4, 5), (128, 32, 8, 32)]
+
+
+def one_pool(ctx, fmt, D, Hkv, k, v):
+    """A pool whose blocks 0 .. hold the rows k, v ([n][Hkv][D] f32, exact in bf16), whole blocks."""
+    n = k.shape[0] // BT
+    pool = ctx.pool(fmt, BT, Hkv, D, n)
+    rows = [to_dev(oracle.f32_to_bf16(x.astype(np.float32).ravel())) for x in (k, v)]
+    ctx.write_blocks(pool, to_dev(np.arange(n, dtype=np.int32)), *rows)
+    return pool
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "f16"])
+@pytest.mark.parametrize("D,Hq,Hkv,seqs", ROW_GROUPS[:2])
+def test_rows_decode_small_weights_and_query_range(ctx, D, Hq, Hkv, seqs, fmt):
+    """One key of weight 1 and value 0 before a tail of weights near 2^-26 whose values are the
+    output, and a query whose deciding element is 2^-44 of its largest (which meets zeros): both
+    are far below fp16's smallest step, none of f32's.  Against f64: 2^-8 of the value (the
+    output's bf16 rounding is 2^-9, weights of 16 bits and f32 sums far less)."""
+    import torch
+
+    L = 496
+    k, v = np.zeros((L, Hkv, D)), np.ones((L, Hkv, D))
+    k[0, :, 0] = 1.0
+    k[2::2, :, 1] = 2.0**15
+    v[0] = 0.0
+    v[1::2, :, D // 2:] = 0.0  # the second half of the dims tells the even keys from the odd
+    q = np.zeros((seqs, Hq, D))
+    q[:, :, 0] = 18.0 * 2.0**-20
+    q[:, :, 1] = 2.0**-34 * 133 / 128
+    q[:, :, 2] = 2.0**10
+    pool = one_pool(ctx, FMTS[fmt], D, Hkv, k, v)
+    lens = np.full(seqs, L, np.int32)
+    tables = np.tile(np.arange(L // BT, dtype=np.int32), (seqs, 1))
+    out = torch.zeros(seqs * Hq * D, dtype=torch.int16, device="cuda")
+    desc = ctx.decode_desc(to_dev(lens), to_dev(tables), Hq, L)
+    before = ctx.route_calls()["rows_decode"]
+    ctx.paged_decode(pool, desc, to_dev(oracle.f32_to_bf16(q.astype(np.float32).ravel())), out, 2.0**20)
+    torch.cuda.synchronize()
+    assert ctx.route_calls()["rows_decode"] == before + 1
+    w = np.exp((k[:, 0] @ q[0, 0]) * 2.0**20 - 18.0)
+    ref = (w / w.sum()) @ v[:, 0]
+    got = oracle.bf16_to_f32(from_dev_bf16(out)).reshape(-1, D)
+    assert 0 < ref.min() < ref.max() < 1e-4
+    assert (np.abs(got - ref) <= ref * 2.0**-8).all(), (got[0, [0, -1]], ref[[0, -1]])
+    assert ctx.device_errors() == 0, ctx.last_error()
+
+
