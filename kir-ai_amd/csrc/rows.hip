@@ -28,7 +28,8 @@
 //
 // int8 / fp8 codes enter the MFMA exactly (as bf16); their scales multiply the scores
 // and the weights in f32.  PARTS = 3 splits every f32 weight into three bf16 terms
-// (24 bits, the whole f32 significand) for three P V products, PARTS = 2 into two (16 bits);
+// (24 bits, the whole f32 significand) for three P V products, PARTS = 2 into two terms of the
+// pool's own type (bf16: 16 bits; fp16: 22, and 2^-31 of the largest weight at the least);
 // PARTS = 1 rounds the weights once, as the tuned 16-bit prefill does.  Beside three terms an
 // fp16 element enters as two bf16 terms (8 + 3 bits, exact), so that q stays as it is and small
 // weights keep their bits, which fp16 terms would lose below 2^-14.
@@ -144,6 +145,8 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 && is16(FMT) ? 1 : 2) void pag
   constexpr bool Q8 = !is16(FMT);
   constexpr bool WIDE16 = FMT == kF16 && PARTS == 3;  // fp16 elements as two bf16 terms
   constexpr int OP = FMT == kF16 && !WIDE16 ? kF16 : kBf16;
+  // Two fp16 terms reach 2^-24 at the least: the weights, at most 2^8 (below), are held 2^7 larger.
+  constexpr float BIAS = OP == kF16 && PARTS == 2 ? 7.0f : 0.0f;
   constexpr int UK = kUnitKeys<D>;
   constexpr int NT = UK / 16;          // score tiles of 16 keys
   constexpr int NS = UK / 32;          // P V steps of 32 keys
@@ -372,7 +375,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 && is16(FMT) ? 1 : 2) void pag
 #pragma unroll
       for (int d = 0; d < ND; d++) oacc[d] *= alpha;
     }
-    const float mref = m_run == -INFINITY ? 0.0f : m_run;
+    const float mref = (m_run == -INFINITY ? 0.0f : m_run) - BIAS;
 #pragma unroll
     for (int s = 0; s < NS; s++) {
       float p[8];
@@ -392,8 +395,13 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 && is16(FMT) ? 1 : 2) void pag
           pb[s][q][x] = w;
           if constexpr (PARTS == 1 && !Q8) l_run = dot2_ones_16<OP>(w, l_run);
           if (q + 1 < PARTS) {  // the rest of the weight, exactly
-            p[2 * x] -= bf16_lo(w);
-            p[2 * x + 1] -= bf16_hi(w);
+            if constexpr (OP == kF16) {
+              p[2 * x] -= f16_bits_to_f32(w & 0xffffu);
+              p[2 * x + 1] -= f16_bits_to_f32(w >> 16);
+            } else {
+              p[2 * x] -= bf16_lo(w);
+              p[2 * x + 1] -= bf16_hi(w);
+            }
           }
         }
       }
@@ -487,7 +495,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 && is16(FMT) ? 1 : 2) void pag
   l_run += xor16_other(l_run, lane);
   l_run += xor32_other(l_run, lane);
   if (g == 0) {
-    s_m[wave][col] = m_run;
+    s_m[wave][col] = m_run - BIAS;
     s_l[wave][col] = l_run;
   }
 #pragma unroll
@@ -577,11 +585,11 @@ hipError_t launch_rows_t(const RowsArgs &a, hipStream_t s, void *hu, LaunchHook 
 // 16-bit pools: PARTS by the caller's need.  The vector decode kernels keep a maximum per four
 // tokens, whose weights are exact more often than under this kernel's one per unit: two terms
 // keep a decode step's error below theirs (short contexts, against f64: bf16, vector 0.00174, one
-// term 0.00184).
+// term 0.00184; fp16, 0.00165 and 0.00166).
 template <int D, int FMT>
 hipError_t launch_rows_16(const RowsArgs &a, bool exact_weights, hipStream_t s, void *hu, LaunchHook hook) {
   if (exact_weights) return launch_rows_t<D, FMT, 3>(a, s, hu, hook);
-  if constexpr (D == kFastHeadDim && FMT == kBf16)
+  if constexpr (D == kFastHeadDim)
     if (!a.chunk_starts) return launch_rows_t<D, FMT, 2>(a, s, hu, hook);
   return launch_rows_t<D, FMT, 1>(a, s, hu, hook);
 }

@@ -444,3 +444,30 @@ def test_rows_decode_small_weights_and_query_range(ctx, D, Hq, Hkv, seqs, fmt):
     assert ctx.device_errors() == 0, ctx.last_error()
 
 
+@pytest.mark.parametrize("fmt", ["bf16", "f16"])
+@pytest.mark.parametrize("D,Hq,Hkv,seqs", ROW_GROUPS[2:])
+def test_rows_decode_error_is_no_larger_than_the_vector_kernels(ctx, opts, D, Hq, Hkv, seqs, fmt):
+    """Groups of eight and four at head_dim 128: the distance from f64 over ragged short contexts,
+    on the packed-row kernel and on the vector kernel (forced) that it stands in for."""
+    from test_gpu_decode import run_decode
+
+    lens = np.random.default_rng(5).integers(50, 501, seqs).astype(np.int32)
+    batch = workloads.paged_batch(lens, BT, 0.10, 111)
+    pool, q = build_case(ctx, batch, Hq, Hkv, FMTS[fmt], 112, head_dim=D)
+    opool = oracle.Pool.from_raw(FMTS[fmt], BT, Hkv, D, batch.n_blocks, pool.raw())
+    qf = oracle.bf16_to_f32(q).reshape(seqs, Hkv, Hq // Hkv, D).astype(np.float64)
+    ref = np.empty_like(qf)
+    for b, n in enumerate(lens):
+        k, v = (x.reshape(n, Hkv, D).astype(np.float64) for x in opool.gather_f32(batch.tables[b], 0, n)[1:])
+        s = np.einsum("hgd,nhd->hgn", qf[b], k) * 0.088
+        w = np.exp(s - s.max(-1, keepdims=True))
+        ref[b] = np.einsum("hgn,nhd->hgd", w / w.sum(-1, keepdims=True), v)
+    err = {}
+    for kernel in ("auto", "split"):
+        opts(llm_hip.OPT_DECODE_KERNEL, kernel)
+        before = ctx.route_calls()["rows_decode"]
+        out = oracle.bf16_to_f32(run_decode(ctx, pool, batch, q, Hq, 0, 0.088)).reshape(ref.shape)
+        assert ctx.route_calls()["rows_decode"] - before == (kernel == "auto")
+        err[kernel] = np.linalg.norm(out - ref) / np.linalg.norm(ref)
+    print(err)
+    assert err["auto"] <= err["split"], err
