@@ -80,6 +80,15 @@ __device__ __forceinline__ u32x4_t codes8(uint32_t lo, uint32_t hi) {
                    fp8x2_to_bf16<true>(hi)};
 }
 
+// Two values cut (rounded towards zero) to OP's 16 bits.
+template <int OP>
+__device__ __forceinline__ uint32_t cut_16(float lo, float hi) {
+  if constexpr (OP == kF16)
+    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(lo, hi));
+  else
+    return __float_as_uint(lo) >> 16 | (__float_as_uint(hi) & 0xffff0000u);
+}
+
 // Eight fp16 elements as eight bf16 terms and the rest, both exact; an infinity or a NaN is all
 // in the first.
 __device__ __forceinline__ void f16x8_to_bf16(const u32x4_t &w, u32x4_t &hi, u32x4_t &lo) {
@@ -387,20 +396,29 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 && is16(FMT) ? 1 : 2) void pag
         if constexpr (Q8)
           p[x] = ((sc[8 * s + x] == -INFINITY) | ((vmiss >> s & 1u) != 0)) ? 0.0f : p[x] * scale_of(8 * s + x, 1);
       }
+      // 16-bit values may be infinite, and such a value times the terms of a positive weight has
+      // to be that infinity: the terms are cut, not rounded, so that none is negative, and none
+      // is zero where the weight is not.
+      constexpr bool CUT = PARTS > 1 && !Q8;
+      float least[CUT ? 8 : 1];
+      if constexpr (CUT) {
+#pragma unroll
+        for (int x = 0; x < 8; x++) least[x] = p[x] > 0.0f ? (OP == kF16 ? 0x1p-24f : 0x1p-120f) : 0.0f;
+      }
 #pragma unroll
       for (int q = 0; q < PARTS; q++) {
 #pragma unroll
         for (int x = 0; x < 4; x++) {
-          const uint32_t w = pack_16<OP>(p[2 * x], p[2 * x + 1]);
+          float &p0 = p[2 * x], &p1 = p[2 * x + 1];
+          const uint32_t w = CUT && q + 1 < PARTS ? cut_16<OP>(p0, p1) : pack_16<OP>(p0, p1);
           pb[s][q][x] = w;
           if constexpr (PARTS == 1 && !Q8) l_run = dot2_ones_16<OP>(w, l_run);
           if (q + 1 < PARTS) {  // the rest of the weight, exactly
-            if constexpr (OP == kF16) {
-              p[2 * x] -= f16_bits_to_f32(w & 0xffffu);
-              p[2 * x + 1] -= f16_bits_to_f32(w >> 16);
-            } else {
-              p[2 * x] -= bf16_lo(w);
-              p[2 * x + 1] -= bf16_hi(w);
+            p0 -= OP == kF16 ? f16_bits_to_f32(w & 0xffffu) : bf16_lo(w);
+            p1 -= OP == kF16 ? f16_bits_to_f32(w >> 16) : bf16_hi(w);
+            if constexpr (CUT) {
+              p0 = fmaxf(p0, least[2 * x]);
+              p1 = fmaxf(p1, least[2 * x + 1]);
             }
           }
         }

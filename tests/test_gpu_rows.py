@@ -471,3 +471,39 @@ def test_rows_decode_error_is_no_larger_than_the_vector_kernels(ctx, opts, D, Hq
         err[kernel] = np.linalg.norm(out - ref) / np.linalg.norm(ref)
     print(err)
     assert err["auto"] <= err["split"], err
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "f16"])
+@pytest.mark.parametrize("D,Hq,Hkv,seqs", ROW_GROUPS)
+def test_rows_decode_infinite_values(ctx, opts, D, Hq, Hkv, seqs, fmt):
+    """An infinite value row element gives that infinity in its dim, two of opposite signs NaN, and
+    the other dims their sums, as from the kernel that this one stands in for."""
+    import torch
+
+    L = 304
+    rng = np.random.default_rng(7)
+    k, v = (oracle.bf16_to_f32(oracle.f32_to_bf16(rng.standard_normal(L * Hkv * D).astype(np.float32)))
+            .reshape(L, Hkv, D) for _ in range(2))
+    v[70, :, 5], v[200, :, 9], v[30, :, 11], v[290, :, 11] = np.inf, -np.inf, np.inf, -np.inf
+    pool = one_pool(ctx, FMTS[fmt], D, Hkv, k, v)
+    lens = np.full(seqs, L, np.int32)
+    tables = np.tile(np.arange(L // BT, dtype=np.int32), (seqs, 1))
+    q = to_dev(oracle.f32_to_bf16(rng.standard_normal(seqs * Hq * D).astype(np.float32)))
+    desc = ctx.decode_desc(to_dev(lens), to_dev(tables), Hq, L)
+    outs = []
+    for option in (None, (llm_hip.OPT_FORCE_GENERIC, 1) if D == 256 or Hq == 12 else (llm_hip.OPT_DECODE_KERNEL, 1)):
+        if option:
+            opts(*option)
+        before = ctx.route_calls()["rows_decode"]
+        out = torch.zeros(seqs, Hq, D, dtype=torch.bfloat16, device="cuda")
+        ctx.paged_decode(pool, desc, q, out.view(torch.int16), 0.05)
+        torch.cuda.synchronize()
+        assert ctx.route_calls()["rows_decode"] - before == (option is None)
+        outs.append(out.float().cpu())
+    rows, other = outs
+    assert (rows[..., 5] == math.inf).all() and (rows[..., 9] == -math.inf).all() and rows[..., 11].isnan().all()
+    finite = [d for d in range(D) if d not in (5, 9, 11)]
+    assert (rows[..., finite] - other[..., finite]).abs().max() <= 2e-2
+    assert torch.equal(rows.isnan(), other.isnan()) and torch.equal(rows.isinf(), other.isinf())
+    assert ctx.device_errors() == 0, ctx.last_error()
+
