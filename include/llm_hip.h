@@ -293,11 +293,14 @@ int llh_paged_decode(llh_ctx *ctx, const llh_kv_pool *pool, const llh_decode_des
  * call: the same result as llh_kv_append of each sequence's new token, at position
  * d_seq_lens[b] - 1 through its block-table row, followed by llh_paged_decode.
  * d_k_new, d_v_new: [num_seqs][kv_heads][head_dim] bf16 (sequences with
- * d_seq_lens[b] == 0 have none).  bf16 pools on the tuned kernels run it as one
- * launch: the new token is attended from d_k_new / d_v_new and written to its slot
- * by the wavefront that computes the sequence's last block; other pools (the
- * quantised token must be attended as stored) and shapes run the append kernel,
- * then the decode.  The pool is written: unlike llh_paged_decode, concurrent calls
+ * d_seq_lens[b] == 0 have none).  The tuned kernels run it as one launch: the
+ * wavefront that computes the sequence's last block attends the new token (as stored, in
+ * quantised pools) and writes it to its slot.  fp8 pools on the stream kernel, fp16 pools at
+ * head_dim 128, other shapes and unaligned rows run the append kernel, then the decode of
+ * llh_paged_decode.  The pool's bytes are those of the two calls; so is the output where
+ * both run the same kernel.  One-launch steps keep to the vector kernels also where
+ * llh_paged_decode takes packed rows (groups of eight or four at head_dim 128): there, and for
+ * bf16 pools' new token, outputs agree within the rounding of the weights.  The pool is written: unlike llh_paged_decode, concurrent calls
  * must not share the sequences' last blocks. */
 int llh_paged_decode_append(llh_ctx *ctx, llh_kv_pool *pool, const llh_decode_desc *desc, const void *d_k_new,
                             const void *d_v_new, const void *d_q, void *d_out, float score_scale, void *stream);

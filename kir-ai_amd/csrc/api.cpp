@@ -1106,6 +1106,10 @@ int llh_paged_decode_append(llh_ctx *ctx, llh_kv_pool *pool, const llh_decode_de
   const bool fused = plan.fast && (pv.format != LLH_KV_F16 || plan.d256) && aligned16(d_k_new) &&
                      aligned16(d_v_new) &&
                      !(pv.format == LLH_KV_FP8_E4M3 && plan.stream_wgs > 0) && (!plan.d256 || plan.stream_wgs > 0);
+  if (!fused) {  // the step is llh_paged_decode's
+    st = plan_decode(ctx, pool, desc, d_q, d_out, score_scale, &plan);
+    if (st != LLH_OK) return st;
+  }
   WsLease lease;
   st = lease.acquire(ctx, s, plan.bytes);
   if (st != LLH_OK) return st;

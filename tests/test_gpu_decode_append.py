@@ -265,3 +265,21 @@ def test_fp8_append_over_a_window_ring_needs_one_block_more(ctx):
         st, ref = opool.decode(Hq, lens, tables, W, q, 0.09)
         assert st == oracle.OK
         assert_parity(from_dev_bf16(out), ref, what=f"fp8 window ring of {nb} blocks")
+
+
+@pytest.mark.parametrize("fmt,Hq,Hkv,lens", [
+    (llm_hip.KV_F16, 32, 4, [16, 300, 1024, 77, 2000]),         # no fused form at head_dim 128
+    (llm_hip.KV_F16, 32, 8, list(range(17, 500, 15))),          # groups of four, 33 sequences
+    (llm_hip.KV_FP8_E4M3, 32, 4, [4096, 3000] * 40),            # stream kernel: none for fp8
+])
+def test_decode_append_not_fused_decodes_as_the_plain_call(ctx, fmt, Hq, Hkv, lens):
+    """Where the append runs first, the decode that follows is llh_paged_decode's own choice:
+    packed rows for groups of eight and four, and the same bits."""
+    batch = workloads.paged_batch(np.array(lens, np.int32), BT, 0.10, 97)
+    before = ctx.route_calls()["rows_decode"], ctx.metrics()["fused_append_calls"]
+    one, two, raw_a, raw_b, ref = run_both(ctx, batch, Hq, Hkv, fmt, 0, 98)
+    assert (ctx.route_calls()["rows_decode"], ctx.metrics()["fused_append_calls"]) == (before[0] + 2, before[1])
+    assert_pools_equal(batch, raw_a, raw_b)
+    assert np.array_equal(one, two)
+    assert_parity(one, ref)
+
