@@ -565,7 +565,8 @@ __device__ __forceinline__ void rows_merge(const RowsArgs &a, size_t prow, size_
   const float ll = merge_weights<1>(mx, ly, li, f);
   float oo = 0.0f;
 #pragma unroll
-  for (int i = 0; i < N; i++) oo += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f[0]), i)) * o_sp[i];
+  for (int i = 0; i < N; i++)  // nothing of the places past the last (0 x infinity is NaN)
+    oo += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f[0]), i)) * (i <= last ? o_sp[i] : 0.0f);
   const float inv = row_inv(a, ll);
   a.out[orow * D + d] = f32_to_bf16_rne(gated(oo * inv, a.gate, orow * D + d));
 }
