@@ -228,7 +228,9 @@ SplitRows split_rows(const llh_ctx *ctx, const PoolView &pv, long long tiles, in
 
 // Split of a prefill call on the packed-row kernel: the context lengths are on the device,
 // so the bound is the table row's (or the window's), and a sequence spreads its own keys
-// over at most max_splits splits.
+// over at most max_splits splits.  Three rounds of units per wavefront stay whole: the splits'
+// merge, by the last workgroup of a tile, costs about as much as two rounds (head_dim 256, Hq16 /
+// Hkv2, 4 x (128 + 16) tokens: 11.1 us whole, 15.8 in two splits).
 SplitRows split_prefill_rows(const llh_ctx *ctx, const PoolView &pv, const llh_prefill_desc *d) {
   const int group = d->num_q_heads / pv.kv_heads;
   const int uk = rows_unit_keys(pv.head_dim);
@@ -240,7 +242,7 @@ SplitRows split_prefill_rows(const llh_ctx *ctx, const PoolView &pv, const llh_p
   SplitRows r{};
   r.split_units = 4;
   r.max_splits = (int)std::min<long long>({(long long)kRowsMaxSplits, std::max(1LL, slots / tiles), (units + 3) / 4});
-  r.single_units = rows_single(ctx, tiles);
+  r.single_units = tiles >= ctx->cus ? 16 : 12;
   if (units <= r.single_units) r.max_splits = 1;
   // at most 16 rows per workgroup: within the scratch wherever there is more than one split
   const size_t rows = r.max_splits > 1 ? (size_t)d->num_seqs * d->max_chunk_len * d->num_q_heads * r.max_splits : 0;
@@ -250,14 +252,16 @@ SplitRows split_prefill_rows(const llh_ctx *ctx, const PoolView &pv, const llh_p
 }
 
 // Whether a prefill call of the tuned shapes runs the packed-row kernel.  Its time grows with
-// its 16-row tiles times their keys; the tile kernels' has a floor (a second launch and
-// partial sums, or few workgroups).  Keys are bounded by the table rows (or the window).
-// Measured on MI355X, packed rows against tiles (us): head_dim 128, bf16, Hq16 / Hkv8,
-// 1 x (4096 + chunk): 64 row tiles 24.9 / 25.5, 128 36.4 / 34.9, 256 60.3 / 39.0; 1 x (1024 +
-// chunk): 256 25.7 / 26.8; 1 x (256 + chunk): 256 12.3 / 23.1; int8, 8 x (1024 + 32), 512 row
-// tiles 29.8 / 34.3; head_dim 256, Hq16 / Hkv2: 1 x 4096: 64 35.6 / 37.4, 128 63.1 / 40.4;
-// 8 x 1024: 128 28.9 / 29.4, and over 300 keys the tile kernel's single launch wins from 32 row
-// tiles on: 128 16.9 / 15.3.
+// its 16-row tiles times their keys; the tile kernels' has a floor (few workgroups, each walking
+// every key).  Up to 64 row tiles it serves every call: the host knows of the contexts only the
+// width of the table rows (or the window), which may be far more than they are, and here it is no
+// worse at any length.  Measured on MI355X under tables of 2048 blocks, tiles whole / packed rows
+// (us): head_dim 128, Hq16 / Hkv8, 1 x (0 + 8) 7.9 / 7.4, 1 x (256 + 64) 16.3 / 9.6, 8 x (1536 +
+// 16) 50.5 / 21.8; head_dim 256, Hq16 / Hkv2, 64 row tiles, 4 x (0 + 16) 7.7 / 7.5, 4 x (64 + 16)
+// 9.5 / 9.7, 8 x (256 + 8) 15.1 / 15.7, 1 x (256 + 64) 16.8 / 14.0, 1 x (1024 + 64) 40.0 / 19.5.
+// Beyond, it serves calls whose table rows bound tiles times keys: head_dim 128, Hq16 / Hkv8,
+// bf16, 1 x (256 + 256), 256 row tiles, 25.0 / 11.9; int8, Hq32 / Hkv8, 8 x (128 + 32), 512, 12.9 /
+// 10.9; head_dim 256, 8 x (1024 + 16), 128, 38.3 / 26.7, but over 320 keys 16.7 / 16.9.
 bool prefill_takes_rows(const llh_ctx *ctx, const PoolView &pv, const llh_prefill_desc *d) {
   if (d->max_chunk_len <= 0 || ctx->opt(LLH_OPT_PREFILL_HEADS_PER_WG)) return false;
   const int group = d->num_q_heads / pv.kv_heads;
@@ -265,8 +269,7 @@ bool prefill_takes_rows(const llh_ctx *ctx, const PoolView &pv, const llh_prefil
   long long keys = (long long)d->max_blocks_per_seq * kFastBlockTokens;
   if (d->window > 0) keys = std::min<long long>(keys, (long long)d->window + d->max_chunk_len);
   if (pv.head_dim == kD256HeadDim) {
-    if (keys <= 320) return tiles < 32;
-    return tiles <= 64 || (tiles <= 128 && tiles * keys <= 150000);
+    return tiles <= 64 || (keys > 320 && tiles <= 128 && tiles * keys <= 150000);
   }
   const long long budget = is16(pv.format) ? 400000 : 600000;
   return tiles <= 64 || (tiles <= 512 && tiles * keys <= budget);
@@ -1229,40 +1232,36 @@ int llh_paged_prefill(llh_ctx *ctx, const llh_kv_pool *pool, const llh_prefill_d
     }
   }
   if (rows_only) ctx->generic_prefill_calls++;
-  // Items of `bm` rows, all heads of a kv head packed.  Where they make at most half as many
-  // groups of `cut` rows as there are compute units and the contexts may be long enough, they
-  // are cut into as many pieces as still give one workgroup per compute unit (more than that is
-  // a second round), with the partial sums in the stream's scratch (none under capture).
-  // Else, where they do not fill the compute units, only `least` heads are packed.  Measured on
-  // MI355X, least heads packed / all / all, cut (us): head_dim 128, Hq32 / Hkv4, 1 x (4096 + 512)
-  // 132 / 103 / 58, 8 x (1024 + 64) 38 / - / 33, 8 x (256 + 64) 17.3 / 19.7 / 29.6,
-  // 8 x (1536 + 512) 142 / 138 / -; head_dim 256, Hq16 / Hkv2, 2 x (1024 + 256) 59.6 / - / 36.2,
-  // 8 x (256 + 64) 17.2 / 22.6 / 29.2.
-  auto plan_pieces = [&](int bm, int cut, int least) {
+  // The tile kernels' items: groups of `cut` rows, all heads of a kv head packed.  Where they make
+  // at most half as many groups as there are compute units, items of long sequences are cut into
+  // as many pieces (a power of two) as still give one workgroup per compute unit (more than that
+  // is a second round), with the partial sums in the stream's scratch (none under capture).  Where
+  // nothing is cut and the groups do not fill the compute units, only `least` heads are packed.
+  auto plan_items = [&](int cut, int least) {
     const int G = desc->num_q_heads / pv.kv_heads;
-    const long long groups = (long long)pv.kv_heads * desc->num_seqs;
     // every sequence's last group may be partial; a uniform batch is counted exactly
     const long long cuts = std::max<long long>(
         1, (long long)desc->total_q_rows == (long long)desc->max_chunk_len * desc->num_seqs
-               ? ((long long)desc->max_chunk_len * G + cut - 1) / cut * groups
+               ? ((long long)desc->max_chunk_len * G + cut - 1) / cut * pv.kv_heads * desc->num_seqs
                : pv.kv_heads * (((long long)desc->total_q_rows * G + cut - 1) / cut + (desc->num_seqs + 1) / 2));
     long long keys = (long long)desc->max_blocks_per_seq * kFastBlockTokens;
     if (desc->window > 0) keys = std::min<long long>(keys, (long long)desc->window + desc->max_chunk_len);
-    const long long pieces = std::min<long long>(kPrefillMaxPieces, ctx->cus / cuts);
-    auto whole = [&](int pack) {
-      a.pack = pack;
-      a.q_tiles = (int32_t)std::max(1LL, ((long long)desc->max_chunk_len * pack + bm - 1) / bm);
-    };
-    if (pieces < 2 || desc->num_seqs > 64 || keys / 64 < prefill_cut_tiles((int)pieces, pv.head_dim))
-      return whole(cuts >= ctx->cus ? G : least);
+    int pieces = kPrefillMaxPieces;
+    while (pieces > 1 && pieces > ctx->cus / cuts) pieces /= 2;
+    a.pack = cuts >= ctx->cus ? G : least;
+    a.cut_pack = G;
+    if (pieces < 2 || desc->num_seqs > 64 || keys / 64 < prefill_cut_tiles(pieces, pv.head_dim)) return;
     scratch = lease.prefill_scratch(ctx, static_cast<hipStream_t>(stream), kCutScratch);
-    if (!scratch) return whole(least);
-    whole(G);
+    if (!scratch) return;
     ctx->routes[LLH_ROUTE_CUT_PREFILL]++;
-    a.max_pieces = (int32_t)pieces;
+    a.max_pieces = pieces;
     a.ws_pieces = 2 * ctx->cus;
     a.ws_ml = reinterpret_cast<float2 *>(scratch);
     a.ws_o = reinterpret_cast<float *>(scratch + align_up((size_t)a.ws_pieces * cut * sizeof(float2)));
+    a.counters = lease.counters();
+  };
+  auto tiles_of = [&](int pack, int bm) {
+    return (int32_t)std::max(1LL, ((long long)desc->max_chunk_len * pack + bm - 1) / bm);
   };
   if (rows) {
     ctx->routes[LLH_ROUTE_ROWS_PREFILL]++;
@@ -1276,6 +1275,7 @@ int llh_paged_prefill(llh_ctx *ctx, const llh_kv_pool *pool, const llh_prefill_d
     if (sr.max_splits > 1) {
       r.ws_o = reinterpret_cast<float *>(scratch + sr.o_off);
       r.ws_ml = reinterpret_cast<float2 *>(scratch);
+      r.counters = lease.counters();
     }
     r.err = a.err;
     r.num_seqs = a.num_seqs;
@@ -1291,12 +1291,16 @@ int llh_paged_prefill(llh_ctx *ctx, const llh_kv_pool *pool, const llh_prefill_d
     r.max_rows = desc->max_chunk_len;
     e = launch_rows(r, /*exact_weights=*/false, static_cast<hipStream_t>(stream));
   } else if (fast) {
-    const bool narrow = ctx->opt(LLH_OPT_PREFILL_HEADS_PER_WG) == 1;
     // both workgroup sizes pack and cut alike, and give the same bits
-    plan_pieces(narrow ? 128 : 256, 256, desc->num_q_heads / pv.kv_heads % 2 ? 1 : 2);
+    const bool narrow = ctx->opt(LLH_OPT_PREFILL_HEADS_PER_WG) == 1;
+    plan_items(256, desc->num_q_heads / pv.kv_heads % 2 ? 1 : 2);
+    a.q_tiles = tiles_of(a.pack, narrow ? 128 : 256);
+    a.cut_tiles = tiles_of(a.cut_pack, narrow ? 128 : 256);
     e = launch_prefill(a, narrow ? kPrefillRows128 : kPrefillRows256, static_cast<hipStream_t>(stream));
   } else if (fast256) {
-    plan_pieces(128, 128, 1);
+    plan_items(128, 1);
+    a.q_tiles = tiles_of(a.pack, 128);
+    a.cut_tiles = tiles_of(a.cut_pack, 128);
     e = launch_prefill_d256(a, static_cast<hipStream_t>(stream));
   } else {
     ctx->generic_prefill_calls++;

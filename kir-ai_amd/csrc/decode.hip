@@ -36,9 +36,10 @@
 // Each group keeps its own online-softmax state (running max in log2 units,
 // sum, 8 output dims per lane per head); groups, wavefronts and splits are
 // merged by log-sum-exp.
+#include "arrival.h"
 #include "device_common.h"
-#include "wave_ops.h"
 #include "stream_partition.h"
+#include "wave_ops.h"
 
 namespace llh {
 
@@ -970,39 +971,8 @@ __device__ __forceinline__ void load_nt(const DecodeArgs &a, int b, int kvh, int
 }
 
 // One-launch split-K: the workgroup that finishes last among the n_splits of a (sequence, kv
-// head) merges them.  The partials cross XCDs, whose L2s are not coherent with each other, so
-// they are stored and loaded at agent scope (written through, and read past, the L2).  A
-// wavefront waits until its stores have completed before its workgroup counts itself in, so
-// whoever counts n_splits finds every partial in memory; no release or acquire fence is
-// needed beyond that (a release at agent scope writes the whole L2 back, ~0.45 us each, one
-// after the other on an XCD).  The last workgroup sets the counter back for the next launch.
-__device__ __forceinline__ void st_agent(float *p, float v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void st_agent(float2 *p, float2 v) {
-  __hip_atomic_store(reinterpret_cast<uint64_t *>(p), __builtin_bit_cast(uint64_t, v), __ATOMIC_RELAXED,
-                     __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ float ld_agent(const float *p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ float2 ld_agent(const float2 *p) {
-  return __builtin_bit_cast(float2, __hip_atomic_load(reinterpret_cast<const uint64_t *>(p), __ATOMIC_RELAXED,
-                                                      __HIP_MEMORY_SCOPE_AGENT));
-}
-__device__ __forceinline__ bool last_to_arrive(int32_t *counter, int n) {
-  __shared__ int s_last;
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's partials have reached memory
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const int seen = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    s_last = seen == n - 1;
-    if (seen == n - 1) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  __syncthreads();
-  return s_last != 0;
-}
-
+// head) merges them (arrival.h).
+//
 // merge_in_registers' merge (the same sums in the same order, so the same bits) of at most
 // kOneLaunchSplits splits, one dim per lane, on partials read at agent scope.
 __device__ __forceinline__ void merge_arrived(const DecodeArgs &a, size_t row0, int last, int d, size_t orow) {

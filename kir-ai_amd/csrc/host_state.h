@@ -57,7 +57,7 @@ struct StreamWorkspace {
   // and never moved or freed before the slot is.
   void *prefill[kPrefillScratches] = {};
   size_t prefill_bytes = 0;
-  // arrival counters of the one-launch split-K decode, in err's allocation: zero between
+  // arrival counters of the launches that merge their own partials, in err's allocation: zero between
   // launches (the launches of a stream run one after the other; each leaves them zero).
   // None to a call under capture, whose graph may be replayed on another stream beside this
   // one's calls, or where the slot was made under capture (the clearing waits for a replay), or
@@ -224,14 +224,18 @@ struct WsLease {
     lock = std::unique_lock<std::mutex>(w->mu);
     return ctx->grow_locked(*w, bytes);
   }
-  // The stream's prefill scratch, or null: while the stream is being captured (the graph may be
-  // replayed beside this stream's calls), on the handle that stands for another stream in each
-  // thread, and when the memory cannot be had; the caller then takes a path without scratch.
+  // The stream's prefill scratch, or null: where the stream has no arrival counters (it is being
+  // captured, or its handle stands for another stream in each thread), and when the memory cannot
+  // be had; the caller then takes a path without scratch.
   char *prefill_scratch(llh_ctx *ctx, hipStream_t s, llh::PrefillScratch which) {
     if (s == hipStreamPerThread || llh::StreamWorkspace::capturing(s)) return nullptr;
     w = ctx->slot(s);
     if (!w) return nullptr;
     lock = std::unique_lock<std::mutex>(w->mu);
+    if (!w->counters()) {
+      lock.unlock();
+      return nullptr;
+    }
     void *&p = w->prefill[which];
     if (p) return static_cast<char *>(p);
     const size_t bytes = llh::prefill_scratch_bytes(ctx->cus, which);

@@ -110,11 +110,16 @@ struct GenericDecodeArgs {
   const uint16_t *gate;     // null, or [B][Hq][D] bf16: out = attention * sigmoid(gate)
 };
 
-constexpr int kPrefillMaxPieces = 8;
-// 64-key tiles from which a sequence is cut into `pieces`: the tiles saved against the memory
-// traffic of the partial sums and the second launch (prefill_items.h)
+constexpr int kPrefillMaxPieces = 8;  // a power of two
+// 64-key tiles from which a sequence is cut into `pieces` = 2, 4 or 8.  A cut saves 1 - 1 / pieces
+// of an item's tiles, about 1.8 us each (2.3 at head_dim 256) where few items run, and costs about
+// 18 us + 1.6 a piece: the partial sums written past the L2, and their merge by one workgroup.
+// Measured on MI355X, whole / cut (us): head_dim 128, 2 pieces 33 tiles 67.6 / 64.8; 4 pieces
+// 17 tiles 31.0 / 40.6, 33 66.7 / 49.6; 8 pieces 24 tiles 54.9 / 43.9; head_dim 256, 4 pieces
+// 20 tiles 59.7 / 44.9; 8 pieces 13 tiles 30.1 / 40.3, 17 37.9 / 42.4, 34 95.3 / 48.8.
 __host__ __device__ constexpr int prefill_cut_tiles(int pieces, int head_dim) {
-  return 36 / pieces + (head_dim == kD256HeadDim ? 7 : 4);
+  return head_dim == kD256HeadDim ? (pieces == 2 ? 23 : pieces == 4 ? 17 : 21)
+                                  : (pieces == 2 ? 31 : 21);
 }
 struct PrefillArgs {
   PoolView pool;
@@ -130,10 +135,13 @@ struct PrefillArgs {
   int32_t window;
   int32_t q_tiles;          // row tiles per (sequence, head group) in the grid
   int32_t pack;             // query heads of a kv head packed into an item's rows
-  int32_t max_pieces;       // > 1: items may be cut into at most this many pieces (prefill_items.h)
-  int32_t ws_pieces;        // max_pieces > 1: pieces (of a group's rows) that ws_o and ws_ml hold
+  int32_t max_pieces;       // 2, 4 or 8: items of long sequences are cut into as many pieces (prefill_items.h)
+  int32_t cut_tiles;        // max_pieces > 1: q_tiles and pack of a call in which any sequence is cut
+  int32_t cut_pack;
+  int32_t ws_pieces;        // pieces (of a group's rows) that ws_o and ws_ml hold
   float *ws_o;              // [cut groups][max_pieces][rows][D] partial outputs
   float2 *ws_ml;            // [cut groups][max_pieces][rows] (max in log2 units, sum)
+  int32_t *counters;        // a zero per cut item
   float scale_log2e;
   float scale;              // score_scale (generic kernel)
   const uint16_t *gate;     // null, or [T][Hq][D] bf16: out = attention * sigmoid(gate)
@@ -164,6 +172,7 @@ struct RowsArgs {
   int32_t max_len;          // > 0: so does a longer context
   int32_t zero_bad;         // keys of a block outside the pool: 1 = score 0 and a zero value, 0 = masked
   int32_t flag_nonfinite;   // 1: a non-finite score raises kErrNonFinite
+  int32_t *counters;        // null: splits merge in a second launch; or nine zeros per (sequence, kv head, row tile)
   float scale;
   float scale_log2e;
   const uint16_t *gate;

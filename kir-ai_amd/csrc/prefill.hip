@@ -235,7 +235,7 @@ __global__ __launch_bounds__(kPrefillThreads * HPW, 2 / HPW) void paged_prefill_
     return;
   }
   const int Hq = a.q_heads;
-  const int G = a.pack;
+  const int G = it.pack;
   const int kvh = it.kvh, c0 = it.c0, chunk = it.chunk, ctx = it.ctx, i0 = it.row0;
   const int rows = chunk * G;
 
@@ -443,18 +443,22 @@ __global__ __launch_bounds__(kPrefillThreads * HPW, 2 / HPW) void paged_prefill_
   // a needed block was missing (its keys read as zeros): each 256 threads know of the blocks they load
   if (bad && ltid == 0) atomicOr(a.err, kErrBadBlock);
   const float l_tot = l_run + xor32_other(l_run, lane);
-  if (!row_ok) return;
-  if (it.pieces > 1) {  // this piece's unnormalised sums, for prefill_merge_kernel
-    const size_t p = (size_t)it.slot + wave * 32 + col;
-    if (h == 0) a.ws_ml[p] = make_float2(m_run, l_tot);
+  if (it.pieces > 1) {  // this piece's unnormalised sums
+    if (row_ok && h == 0) store_piece_sums<256>(a, it, wave * 32 + col, m_run, l_tot);
+    constexpr int LD = 32 + kPiecePad;
+    static_assert(sizeof(k_lds) >= sizeof(float) * 4 * HPW * 32 * LD, "the K tiles hold every wavefront's buffer");
+    float *buf = reinterpret_cast<float *>(k_lds) + wave * 32 * LD;
 #pragma unroll
-    for (int mt = 0; mt < 4; mt++)
+    for (int mt = 0; mt < 4; mt++) {
 #pragma unroll
-      for (int jq = 0; jq < 4; jq++)
-        *reinterpret_cast<float4 *>(&a.ws_o[p * D + mt * 32 + jq * 8 + 4 * h]) =
-            make_float4(oacc[mt][4 * jq], oacc[mt][4 * jq + 1], oacc[mt][4 * jq + 2], oacc[mt][4 * jq + 3]);
-    return;
+      for (int j = 0; j < 16; j += 2)
+        *reinterpret_cast<float2 *>(&buf[col * LD + 8 * (j >> 2) + 4 * h + (j & 3)]) =
+            make_float2(oacc[mt][j], oacc[mt][j + 1]);
+      store_piece<D, 256, 32, 32>(a, it, buf, wave * 32, rows - wrow0, mt * 32, lane);
+    }
+    return finish_piece<D, BM, 256>(a, it);
   }
+  if (!row_ok) return;
   const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
   const size_t obase = ((size_t)(c0 + my_tok) * Hq + my_head) * D;
   uint16_t *orow = a.out + obase;
@@ -607,9 +611,7 @@ hipError_t launch_prefill(const PrefillArgs &a, int variant, hipStream_t s) {
     default:
       return hipErrorInvalidValue;
   }
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess || a.max_pieces <= 1) return e;
-  return wide ? launch_prefill_merge<D, 256, 256>(a, s) : launch_prefill_merge<D, 128, 256>(a, s);
+  return hipGetLastError();
 }
 
 hipError_t launch_prefill_generic(const PrefillArgs &a, int total_rows, hipStream_t s) {

@@ -183,7 +183,7 @@ __global__ __launch_bounds__(kThreads, 1) void paged_prefill_d256_kernel(const P
     return;
   }
   const int Hq = a.q_heads;
-  const int G = a.pack;
+  const int G = it.pack;
   const int kvh = it.kvh, c0 = it.c0, chunk = it.chunk, ctx = it.ctx, i0 = it.row0;
   const int rows = chunk * G;
 
@@ -377,14 +377,24 @@ __global__ __launch_bounds__(kThreads, 1) void paged_prefill_d256_kernel(const P
   // ---- normalise and store: lane holds dims 16db + 4g .. +4 of its row ----
   if (bad && tid == 0) atomicOr(a.err, kErrBadBlock);  // a needed block was missing: its keys read as zeros
   const float l_tot = row_sum4(l_run);
-  if (!row_ok) return;
-  if (it.pieces > 1) {  // this piece's unnormalised sums, for prefill_merge_kernel
-    const size_t p = (size_t)it.slot + wave * ROWS + r;
-    if (g == 0) a.ws_ml[p] = make_float2(m_run, l_tot);
+  if (it.pieces > 1) {  // this piece's unnormalised sums
+    if (row_ok && g == 0) store_piece_sums<BM>(a, it, wave * ROWS + r, m_run, l_tot);
+    constexpr int LD = 64 + kPiecePad;
+    static_assert(sizeof(k_lds) >= sizeof(float) * (kThreads / 64) * ROWS * LD, "the K tiles hold every wavefront's buffer");
+    float *buf = reinterpret_cast<float *>(k_lds) + wave * ROWS * LD;
 #pragma unroll
-    for (int db = 0; db < 16; db++) *reinterpret_cast<f32x4_t *>(&a.ws_o[p * D + db * 16 + 4 * g]) = oacc[db];
-    return;
+    for (int d0 = 0; d0 < 16; d0 += 4) {
+#pragma unroll
+      for (int db = 0; db < 4; db++) {
+        float2 *p = reinterpret_cast<float2 *>(&buf[r * LD + db * 16 + 4 * g]);
+        p[0] = make_float2(oacc[d0 + db][0], oacc[d0 + db][1]);
+        p[1] = make_float2(oacc[d0 + db][2], oacc[d0 + db][3]);
+      }
+      store_piece<D, BM, ROWS, 64>(a, it, buf, wave * ROWS, rows - wrow0, d0 * 16, lane);
+    }
+    return finish_piece<D, BM, BM>(a, it);
   }
+  if (!row_ok) return;
   const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
   const size_t obase = ((size_t)(c0 + my_tok) * Hq + my_head) * D;
   uint16_t *orow = a.out + obase;
@@ -406,8 +416,7 @@ hipError_t launch_prefill_d256(const PrefillArgs &a, hipStream_t s) {
     hipLaunchKernelGGL(paged_prefill_d256_kernel<kF16>, dim3(grid), dim3(kThreads), 0, s, a);
   else
     hipLaunchKernelGGL(paged_prefill_d256_kernel<kBf16>, dim3(grid), dim3(kThreads), 0, s, a);
-  const hipError_t e = hipGetLastError();
-  return e != hipSuccess || a.max_pieces <= 1 ? e : launch_prefill_merge<D, BM, BM>(a, s);
+  return hipGetLastError();
 }
 
 }  // namespace llh

@@ -6,7 +6,9 @@
 // wavefronts.  A wavefront walks units of 64 keys (32 at head_dim 256): it loads the unit's
 // K and V straight into MFMA operand registers (every byte is used by one wavefront, so LDS
 // would only add a copy), and the next unit's loads are in flight behind the current unit's
-// math.  Wavefronts merge in LDS, splits in paged_rows_merge_kernel.
+// math.  Wavefronts merge in LDS; splits merge in a second launch (decode, whose host knows the
+// longest context and so whether there are any) or, where only the block-table width is known, by
+// the last workgroup of a tile to arrive, so that short contexts pay for no launch.
 //
 // It serves
 //  * decode steps outside the tuned kernels' shapes (head_dim 128 or 256, 16-token
@@ -39,10 +41,12 @@
 // is each K / V byte once per 16-row tile.  Measured on MI355X: decode, 16 x U[256, 4096]
 // tokens, Hq16 / Hkv2, head_dim 256, fp8: 3139 us on the element-wise kernel, 19.7 us here
 // (32 MB, 1.6 TB/s); a chunk of 8 tokens over 4099 cached ones, Hq16 / Hkv8, head_dim 128,
-// bf16: 119.5 us on 128-row tiles, 12.6 us here (17 MB, 1.3 TB/s); 2 x (1024 + 250) tokens,
+// bf16: 119.5 us on 128-row tiles, 14.8 us here (17 MB, 1.1 TB/s; the merge of 17 splits by one
+// workgroup takes half of it: with a second launch 12.2, but 8 tokens over none under a table of
+// 2048 blocks then 10.2 against 7.4); 2 x (1024 + 250) tokens,
 // Hq16 / Hkv2, head_dim 256, int8: 10.6 ms element-wise, 48 us here (197 TFLOP/s: the code
 // conversions, repeated by every 16-row tile, bound it).
-#include "wave_ops.h"
+#include "arrival.h"
 
 namespace llh {
 
@@ -149,6 +153,49 @@ __device__ __forceinline__ float row_inv(const RowsArgs &a, float ll) {
 template <int D>
 constexpr int kUnitKeys = D == 256 ? 32 : 64;
 
+// Of a tile's rows, `n` partials from split s0 on, every `stride`-th, by one workgroup at agent
+// scope (arrival.h): the output, or (PARTIAL) a partial in the place of split s0.
+constexpr int kSplitGroup = 8;
+constexpr int kFlatSplits = 24;  // splits merged at once
+template <int D, bool PARTIAL>
+__device__ __forceinline__ void merge_splits(const RowsArgs &a, const SeqSplit &sq, int b, int kvh, int G, int row0,
+                                             int live, int s0, int stride, int n) {
+  constexpr int HALVES = D / 128;             // row parts of 128 dims
+  constexpr int U = TILE * HALVES / WAVES;    // a wavefront's, all at once: each round is a trip to memory
+  const int lane = threadIdx.x & 63;
+  for (int u0 = (int)(threadIdx.x >> 6) * U; u0 < live * HALVES; u0 += WAVES * U) {
+    const float2 *ml[U];
+    const float *o[U];
+    size_t place[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int part = min(u0 + u, live * HALVES - 1);
+      const int r = row0 + part / HALVES;
+      place[u] = (((size_t)b * a.max_rows + r / G) * a.q_heads + kvh * G + r % G) * a.max_splits + s0;
+      ml[u] = a.ws_ml + place[u];
+      o[u] = a.ws_o + place[u] * D + part % HALVES * 128;
+    }
+    float2 out[U];
+    float mx[U], sum[U];
+    merge_parts<U, 8>(ml, stride, o, (size_t)stride * D, n, lane, out, mx, sum);
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (u0 + u >= live * HALVES) break;
+      const int half = (u0 + u) % HALVES;
+      if constexpr (PARTIAL) {
+        st_agent(reinterpret_cast<float2 *>(&a.ws_o[place[u] * D + half * 128]) + lane, out[u]);
+        if (half == HALVES - 1 && lane == 0) st_agent(&a.ws_ml[place[u]], make_float2(mx[u], sum[u]));
+      } else {
+        const int r = row0 + (u0 + u) / HALVES;
+        const float inv = row_inv(a, sum[u]);
+        const size_t at = ((size_t)(sq.c0 + r / G) * a.q_heads + kvh * G + r % G) * D + half * 128 + 2 * lane;
+        a.out[at] = f32_to_bf16_rne(gated(out[u].x * inv, a.gate, at));
+        a.out[at + 1] = f32_to_bf16_rne(gated(out[u].y * inv, a.gate, at + 1));
+      }
+    }
+  }
+}
+
 template <int D, int FMT, int PARTS>
 __global__ __launch_bounds__(64 * WAVES, D == 256 && is16(FMT) ? 1 : 2) void paged_rows_kernel(const RowsArgs a) {
   constexpr bool Q8 = !is16(FMT);
@@ -166,9 +213,15 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 && is16(FMT) ? 1 : 2) void pag
 
   const int Hkv = a.pool.kv_heads;
   const int G = a.q_heads / Hkv;
-  const int split = blockIdx.x % a.max_splits;
-  const int kvh = blockIdx.x / a.max_splits % Hkv;
-  const int tile = blockIdx.x / a.max_splits / Hkv;
+  // Splits of a tile are neighbours, or, where max_splits says little about how many there are (the
+  // bound is a block-table row), the slowest index: workgroups go round-robin over the 8 XCDs, and
+  // the first splits of unsplit sequences would all meet on one (8 x (384 + 8) tokens, Hq16 / Hkv8,
+  // under a table of 2048 blocks: 19.4 us, 11.5 under the exact one).
+  const int first = gridDim.x / a.max_splits;
+  const int split = a.counters ? blockIdx.x / first : blockIdx.x % a.max_splits;
+  const int item = a.counters ? blockIdx.x % first : blockIdx.x / a.max_splits;
+  const int kvh = item % Hkv;
+  const int tile = item / Hkv;
   const int b = blockIdx.y;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -544,10 +597,35 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 && is16(FMT) ? 1 : 2) void pag
       for (int x = 0; x < 4; x++) a.out[o + x] = f32_to_bf16_rne(gated(oo[x] * inv, a.gate, o + x));
     } else {
       const size_t p = (((size_t)b * a.max_rows + tok) * a.q_heads + head) * a.max_splits + split;
-      *reinterpret_cast<f32x4_t *>(&a.ws_o[p * D + d]) = oo;
-      if (d == 0) a.ws_ml[p] = make_float2(mm, ll);
+      if (a.counters) {
+        float2 *o = reinterpret_cast<float2 *>(&a.ws_o[p * D + d]);
+        st_agent(o, make_float2(oo[0], oo[1]));
+        st_agent(o + 1, make_float2(oo[2], oo[3]));
+        if (d == 0) st_agent(&a.ws_ml[p], make_float2(mm, ll));
+      } else {
+        *reinterpret_cast<f32x4_t *>(&a.ws_o[p * D + d]) = oo;
+        if (d == 0) a.ws_ml[p] = make_float2(mm, ll);
+      }
     }
   }
+  if (sq.n_splits <= 1 || !a.counters) return;
+  // The last workgroup of the tile merges the splits.  One compute unit takes about 32 GB/s past
+  // its L2, so many splits are first merged in groups, each by the last of its own workgroups,
+  // into the place of the group's first split (8 tokens over 16000, head_dim 128: 64 splits at
+  // once 31.4 us, in groups 22.7).
+  int32_t *counters = &a.counters[((size_t)b * first + item) * (1 + kRowsMaxSplits / kSplitGroup)];
+  if (sq.n_splits <= kFlatSplits) {
+    if (last_to_arrive(counters, sq.n_splits)) merge_splits<D, false>(a, sq, b, kvh, G, row0, live, 0, 1, sq.n_splits);
+    return;
+  }
+  const int group = split / kSplitGroup;
+  const int g0 = group * kSplitGroup;
+  const int in_group = min(kSplitGroup, sq.n_splits - g0);
+  if (!last_to_arrive(&counters[1 + group], in_group)) return;
+  if (in_group > 1) merge_splits<D, true>(a, sq, b, kvh, G, row0, live, g0, 1, in_group);
+  const int n_groups = (sq.n_splits + kSplitGroup - 1) / kSplitGroup;
+  if (!last_to_arrive(counters, n_groups)) return;
+  merge_splits<D, false>(a, sq, b, kvh, G, row0, live, 0, kSplitGroup, n_groups);
 }
 
 // Merge of the n <= N splits of one (query row, head): every partial row in flight at
@@ -595,7 +673,7 @@ hipError_t launch_rows_t(const RowsArgs &a, hipStream_t s, void *hu, LaunchHook 
                      dim3(64 * WAVES), 0, s, a);
   hipError_t e = hipGetLastError();
   if (hook) hook(hu, 1, s);
-  if (e != hipSuccess || a.max_splits <= 1) return e;
+  if (e != hipSuccess || a.max_splits <= 1 || a.counters) return e;
   hipLaunchKernelGGL((paged_rows_merge_kernel<D, kUnitKeys<D>>), dim3(a.max_rows * a.q_heads, a.num_seqs), dim3(D), 0,
                      s, a);
   return hipGetLastError();

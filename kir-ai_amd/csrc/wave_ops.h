@@ -126,9 +126,10 @@ __device__ __forceinline__ float rounded_product(float a, float b) {
 
 // Log-sum-exp weights of up to 64 P partials, P (max, sum) pairs per lane (mx = -inf in the
 // places past the last): f = 2^(mx - largest), the same in every kernel that merges; returns the
-// sum of l f over the wavefront, the same bits in every lane.
+// sum of l f over the wavefront, the same bits in every lane, and the largest in *top.
 template <int P>
-__device__ __forceinline__ float merge_weights(const float (&mx)[P], const float (&l)[P], int lane, float (&f)[P]) {
+__device__ __forceinline__ float merge_weights(const float (&mx)[P], const float (&l)[P], int lane, float (&f)[P],
+                                               float *top = nullptr) {
   float mm = mx[0];
 #pragma unroll
   for (int p = 1; p < P; p++) mm = fmaxf(mm, mx[p]);
@@ -138,6 +139,7 @@ __device__ __forceinline__ float merge_weights(const float (&mx)[P], const float
   mm = fmaxf(mm, dpp<0x140>(mm));  // row_mirror
   mm = fmaxf(mm, xor16_other(mm, lane));
   mm = fmaxf(mm, xor32_other(mm, lane));
+  if (top) *top = mm;
   const float mref = mm == -INFINITY ? 0.0f : mm;
   float sum = 0.0f;
 #pragma unroll

@@ -732,6 +732,13 @@ def test_per_thread_stream_handle_shares_no_counters(ctx):
         ctx.paged_decode(pool, desc, d_q, two, 0.088, stream=per_thread)
         torch.cuda.synchronize()
         assert torch.equal(one, two)
+    assert ctx.route_calls() == before
+    lens = np.array([2000], np.int32)  # splits, where there are counters
+    batch = workloads.paged_batch(lens, BT, 0.10, 87)
+    pool, _ = build_case(ctx, batch, 16, 8, llm_hip.KV_BF16, 87)
+    ctx.paged_decode(pool, ctx.decode_desc(to_dev(lens), to_dev(batch.tables), 16, 2000), d_q, one, 0.088)
+    torch.cuda.synchronize()
+    before = ctx.route_calls()
     pdesc = ctx.prefill_desc(to_dev(np.array([0, 1], np.int32)), to_dev(lens), to_dev(batch.tables), 16, 1)
     ctx.paged_prefill(pool, pdesc, d_q, two, 0.088, stream=per_thread)
     torch.cuda.synchronize()

@@ -256,7 +256,7 @@ def test_rows_decode_no_weight_as_the_vector_kernels(ctx, opts):
     assert ctx.device_errors() == 0, ctx.last_error()
 
 
-@pytest.mark.parametrize("window", [0, 700])
+@pytest.mark.parametrize("window", [0, 1500])
 @pytest.mark.parametrize("D,Hq,Hkv,fmt,chunk,prefix", [
     (128, 32, 4, "bf16", [300, 0, 130, 1], [1500, 10, 900, 2000]),   # all heads packed, cut; ragged
     (128, 6, 2, "f16", [700], [800]),                                # odd group, cut
@@ -370,7 +370,7 @@ def test_prefill_scratch_is_bounded_and_its_own(ctx, opts, D, Hq, Hkv, n, chunk)
     chunks[n // 2] = chunk
     outs, used = [], []
     for max_chunk in (chunk, 4096):
-        _, ppool, pq, pout, pdesc = prefill_call(ctx, llm_hip.KV_BF16, D, Hq, Hkv, chunks, [1300] * n, 103, max_chunk)
+        _, ppool, pq, pout, pdesc = prefill_call(ctx, llm_hip.KV_BF16, D, Hq, Hkv, chunks, [2100] * n, 103, max_chunk)
         ctx.paged_prefill(ppool, pdesc, pq, pout, 0.088, stream=stream)
         stream.synchronize()
         replay()
@@ -506,5 +506,72 @@ def test_rows_decode_infinite_values(ctx, opts, D, Hq, Hkv, seqs, L, fmt):
     assert (rows[..., finite] - other[..., finite]).abs().max() <= 2e-2
     if D == 256 or Hq == 12:
         assert torch.equal(rows.isnan(), other.isnan()) and torch.equal(rows.isinf(), other.isinf())
+    assert ctx.device_errors() == 0, ctx.last_error()
+
+
+@pytest.mark.parametrize("D,Hq,Hkv,chunk,prefix,route", [
+    (128, 16, 8, [8, 3], [2100, 40], "rows_prefill"),      # one sequence split, one not
+    (128, 16, 8, [8, 3], [7000, 1600], "rows_prefill"),    # 28 splits, merged in groups, and 7
+    (256, 8, 4, [5], [900], "rows_prefill"),
+    (256, 8, 4, [5], [4000], "rows_prefill"),              # 32 splits (int8: as many)
+    (256, 8, 4, [2], [3190], "rows_prefill"),              # 25 splits: a group of one
+    (128, 32, 4, [300, 20], [1500, 1700], "cut_prefill"),
+    (256, 16, 2, [150, 90], [1500, 30], "cut_prefill"),    # one sequence cut, one not
+])
+@pytest.mark.parametrize("fmt", ["bf16", "int8"])
+def test_prefill_merges_in_its_launch_over_changing_inputs(ctx, D, Hq, Hkv, chunk, prefix, route, fmt):
+    """Splits and pieces merged by the last workgroup to arrive: two pools in turn, a query each,
+    back to back on one stream, so that the scratch always holds another call's partials; then the
+    same calls in the opposite order.  Every output has the same bits both times, and the first
+    ones meet the whole items of a captured call."""
+    import torch
+
+    from helpers import assert_parity
+
+    if D == 256 and fmt == "int8":
+        route = "rows_prefill"
+    cases = [prefill_call(ctx, FMTS[fmt], D, Hq, Hkv, chunk, prefix, seed) for seed in (121, 131)]
+    g = torch.Generator(device="cuda")
+    g.manual_seed(122)
+    q = torch.randn(60, cases[0][2].numel(), generator=g, device="cuda").to(torch.bfloat16).view(torch.int16)
+    there, back = torch.zeros_like(q), torch.zeros_like(q)
+    before = ctx.route_calls()[route]
+    for out, order in ((there, range(len(q))), (back, reversed(range(len(q))))):
+        for i in order:
+            _, pool, _, _, desc = cases[i % 2]
+            ctx.paged_prefill(pool, desc, q[i], out[i], 0.088)
+    torch.cuda.synchronize()
+    assert ctx.route_calls()[route] == before + 2 * len(q)
+    assert torch.equal(there, back), int((there != back).sum())
+    stream = torch.cuda.Stream()
+    whole = torch.zeros_like(q[:2])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        for i in range(2):
+            ctx.paged_prefill(cases[i][1], cases[i][4], q[i], whole[i], 0.088, stream=torch.cuda.current_stream())
+    graph.replay()
+    torch.cuda.synchronize()
+    assert_parity(from_dev_bf16(there[:2]), oracle.bf16_to_f32(from_dev_bf16(whole)))
+    assert ctx.device_errors() == 0, ctx.last_error()
+    ctx.release_stream(stream)
+
+
+@pytest.mark.parametrize("D,Hq,Hkv,fmt", [(128, 32, 4, "bf16"), (128, 6, 2, "f16"), (256, 16, 2, "bf16")])
+@pytest.mark.parametrize("chunk,prefix", [([64] * 8, [256] * 8), ([300, 0, 130], [1900, 10, 900])])
+def test_prefill_table_wider_than_the_contexts(ctx, opts, D, Hq, Hkv, fmt, chunk, prefix):
+    """Block-table rows of 2048 blocks: whether items are cut, and how heads are packed where they
+    are not, follows the contexts, so the bits are those of the exact table."""
+    import torch
+
+    opts(llm_hip.OPT_PREFILL_HEADS_PER_WG, 2)  # the tile kernels
+    outs = []
+    for width in (None, 2048):
+        _, pool, q, out, desc = prefill_call(ctx, FMTS[fmt], D, Hq, Hkv, chunk, prefix, 141, table_blocks=width)
+        before = ctx.route_calls()["cut_prefill"]
+        ctx.paged_prefill(pool, desc, q, out, 0.088)
+        torch.cuda.synchronize()
+        assert ctx.route_calls()["cut_prefill"] - before == (width is not None or max(prefix) > 1000)
+        outs.append(out)
+    assert torch.equal(*outs)
     assert ctx.device_errors() == 0, ctx.last_error()
 
