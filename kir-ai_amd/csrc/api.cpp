@@ -1291,9 +1291,15 @@ int llh_paged_prefill(llh_ctx *ctx, const llh_kv_pool *pool, const llh_prefill_d
     r.max_rows = desc->max_chunk_len;
     e = launch_rows(r, /*exact_weights=*/false, static_cast<hipStream_t>(stream));
   } else if (fast) {
-    // both workgroup sizes pack and cut alike, and give the same bits
-    const bool narrow = ctx->opt(LLH_OPT_PREFILL_HEADS_PER_WG) == 1;
-    plan_items(256, desc->num_q_heads / pv.kv_heads % 2 ? 1 : 2);
+    // Both workgroup sizes pack and cut alike, and give the same bits.  Where one head is packed,
+    // 256 rows are 256 tokens, whose wavefronts need very different stretches of the keys and wait
+    // for each other: 128 rows, two workgroups a compute unit (us, 256 / 128 rows: Hq4 / Hkv4,
+    // 8 x (0 + 512) 25.0 / 20.8; Hq6 / Hkv2 25.2 / 20.9; Hq16 / Hkv16, 2 x (0 + 2048) 70.7 / 65.8).
+    const int group = desc->num_q_heads / pv.kv_heads;
+    plan_items(256, group % 2 ? 1 : 2);
+    if (a.max_pieces > 1 && a.pack == 1) a.pack = group;
+    const int wg_opt = ctx->opt(LLH_OPT_PREFILL_HEADS_PER_WG);
+    const bool narrow = wg_opt == 1 || (wg_opt == 0 && a.pack == 1);
     a.q_tiles = tiles_of(a.pack, narrow ? 128 : 256);
     a.cut_tiles = tiles_of(a.cut_pack, narrow ? 128 : 256);
     e = launch_prefill(a, narrow ? kPrefillRows128 : kPrefillRows256, static_cast<hipStream_t>(stream));

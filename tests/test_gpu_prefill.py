@@ -317,3 +317,19 @@ def test_prefill_bad_block_at_every_place_of_a_tile(ctx, opts, head_dim, Hq, Hkv
             torch.cuda.synchronize()
             want = 0 if place is None else llm_hip.ERR_FLAG_BAD_BLOCK
             assert ctx.device_errors() == want, (prefix, place)
+
+
+@pytest.mark.parametrize("Hq,Hkv", [(4, 4), (6, 2)])
+@pytest.mark.parametrize("prefix,chunk", [([0] * 8, [512] * 8), ([1700, 30], [500, 77])])
+def test_prefill_odd_groups_workgroup_sizes_match(ctx, opts, Hq, Hkv, prefix, chunk):
+    """One head or three, whole items and cut ones: workgroups of 128 rows, of 256, and the
+    automatic choice (128 where one head is packed) give the same bits."""
+    outs = []
+    for option in (1, 2, 0):
+        opts(llm_hip.OPT_PREFILL_HEADS_PER_WG, option)
+        before = ctx.route_calls()
+        outs.append(build(ctx, prefix, chunk, Hq, Hkv, 0, 151)[4])
+        after = ctx.route_calls()
+        assert after["cut_prefill"] - before["cut_prefill"] == (max(prefix) > 0)
+        assert after["rows_prefill"] == before["rows_prefill"]
+    assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])
