@@ -190,12 +190,12 @@ int rows_single(const llh_ctx *ctx, long long tiles) { return tiles >= ctx->cus 
 // Split of the packed-row kernel (rows.hip).  A split holds at least one unit for each of
 // its four wavefronts.  Small steps take the split that gives one workgroup per compute
 // unit (two at head_dim 128): a workgroup's start and its merge cost more than a unit.
-// Steps of more than kSplitUnits units per workgroup take two rounds of them, which
-// levels ragged lengths.  Measured on MI355X in blocks of 16 tokens per split (us):
-//   16 x U[256, 4096], Hq16 / Hkv2, head_dim 256, fp8: 8: 29.6, 16: 20.0, 24: 23.6, 32: 26.1
-//   32 x U[256, 4096], the same over int8:             8: 36.5, 16: 32.0, 32: 30.5, 64: 45.0
-//   32 x U[256, 4096], Hq8 / Hkv4, head_dim 256, bf16: 16: 73.4, 32: 70.4, 64: 80.5
-//   32 x U[256, 4096], Hq24 / Hkv8, head_dim 128:      16: 70.4, 32: 61.3, 64: 67.0
+// Steps of more than kTwoRounds units per workgroup take two rounds of them, which
+// levels ragged lengths.  Measured on MI355X in blocks of 16 tokens per split, and as planned (us):
+//   16 x U[256, 4096], Hq16 / Hkv2, head_dim 256, fp8: 8: 24.5, 16: 20.2, 24: 22.1, 32: 19.3; 22.0
+//   32 x U[256, 4096], the same over int8:             8: 34.9, 16: 34.0, 32: 30.5, 64: 30.3; 30.5
+//   32 x U[256, 4096], Hq8 / Hkv4, head_dim 256, bf16: 16: 74.5, 32: 73.5, 64: 83.8; 77.4
+//   32 x U[256, 4096], Hq24 / Hkv8, head_dim 128:      16: 60.6, 32: 59.2, 64: 64.1; 61.6
 // `units`: the longest sequence's; `total`: all workgroup rows' together; `out_rows`:
 // (query row, head) pairs.
 struct SplitRows {
@@ -209,13 +209,16 @@ SplitRows split_rows(const llh_ctx *ctx, const PoolView &pv, long long tiles, in
   SplitRows r{};
   const bool wide = pv.head_dim == kD256HeadDim;
   const long long slots = (long long)ctx->cus * (wide ? 1 : 2);
-  const long long two_rounds = wide ? 16 : 8;
+  const long long kTwoRounds = wide ? 16 : 8;
   long long per = (total + slots - 1) / slots;
-  if (per > two_rounds) per = std::max(two_rounds, (per + 1) / 2);
+  if (per > kTwoRounds) per = std::max(kTwoRounds, (per + 1) / 2);
   r.split_units = (int)std::min<long long>(1 << 20, std::max<long long>(4, (per + 3) / 4 * 4));
   const int opt = ctx->opt(LLH_OPT_DECODE_SPLIT_BLOCKS);
   if (opt > 0) r.split_units = std::max(1, opt * kFastBlockTokens / rows_unit_keys(pv.head_dim));
   r.max_splits = std::min(kRowsMaxSplits, std::max(1, (units + r.split_units - 1) / r.split_units));
+  // Workgroups of splits that no sequence has still have to be dispatched, and `units` may be a
+  // bound far above every length.
+  r.max_splits = (int)std::min<long long>(r.max_splits, std::max(1LL, 4 * slots / tiles));
   r.single_units = rows_single(ctx, tiles);
   if (units <= r.single_units) r.max_splits = 1;
   for (;; r.max_splits--) {
@@ -729,14 +732,14 @@ static int check_span(llh_ctx *ctx, const llh_kv_pool *pool, int32_t max_seq_len
 // Whether a head_dim-128 decode step of the vector kernels' shapes runs the packed-row kernel.
 // Eight query heads per kv head fill half a matrix tile, and its MFMAs take the place of the
 // dot products that bound the vector kernels at this group size.  Measured on MI355X, Hq32 /
-// Hkv4, vector against packed rows (us): bf16 1 x 2000 12.0 / 12.0, 1 x 16000 41.4 / 14.6,
-// 4 x 4096 21.0 / 12.4, 32 x U[50, 500] 25.0 / 12.2, 32 x U[256, 4096] 53.9 / 44.3; int8
-// 1 x 16000 41.7 / 13.2, 32 x U[256, 4096] 58.5 / 35.7.  A few short sequences stay: bf16
-// 4 x U[500, 1000] 11.6 / 12.6.  At four heads per kv head it is faster where the sequences
+// Hkv4, vector against packed rows (us): bf16 1 x 2000 10.8 / 11.1, 1 x 16000 39.6 / 13.3,
+// 4 x 4096 21.2 / 12.6, 32 x U[50, 500] 30.3 / 12.2, 32 x U[256, 4096] 54.8 / 37.0; int8
+// 1 x 16000 41.0 / 12.4, 32 x U[256, 4096] 59.4 / 31.9.  A few short sequences stay: bf16
+// 4 x U[500, 1000] 11.0 / 12.6.  At four heads per kv head it is faster where the sequences
 // are short enough for a unit or two per wavefront and fill the chip unsplit: Hq32 / Hkv8,
-// 32 x U[50, 500] bf16 15.7 / 12.9 (16 x U[50, 300] 10.4 / 11.8), int8 24.0 / 12.0, but 4 x U[500, 1000] 11.7 / 19.7 and
-// long ones 35.8 / 45.7 (16 x U[1000, 4000]); at two it is not (Hq16 / Hkv8, 32 x U[50, 500]
-// 12.3 / 14.0).
+// 32 x U[50, 500] bf16 17.2 / 13.0 (16 x U[50, 300] 10.5 / 11.8), int8 18.8 / 10.8, but
+// 4 x U[500, 1000] 10.4 / 19.7 and long ones 34.8 / 45.7 (16 x U[1000, 4000]); at two it is not
+// (Hq16 / Hkv8, 32 x U[50, 500] 12.3 / 14.0).
 static bool decode_prefers_rows(const PoolView &pv, int group, int num_seqs, int est_blocks) {
   const long long tiles = (long long)num_seqs * pv.kv_heads;
   if (group == 8) return tiles > 16 || est_blocks > 1024 / kFastBlockTokens + 1;
@@ -1220,7 +1223,7 @@ int llh_paged_prefill(llh_ctx *ctx, const llh_kv_pool *pool, const llh_prefill_d
   // int8 / fp8 blocks at head_dim 256 always run the packed-row kernel, unsplit where no
   // scratch may be taken
   const bool rows_only = tuned_shape && !fast && !fast256 && pv.format != LLH_KV_INT8_ROW &&
-                         pv.head_dim == kD256HeadDim && desc->max_chunk_len > 0;
+                         pv.head_dim == kD256HeadDim && desc->max_chunk_len > 0 && desc->num_seqs <= 65535;
   bool rows = rows_only || ((fast || fast256) && prefill_takes_rows(ctx, pv, desc));
   if (rows) {
     sr = split_prefill_rows(ctx, pv, desc);

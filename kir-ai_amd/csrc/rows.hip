@@ -213,16 +213,17 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 && is16(FMT) ? 1 : 2) void pag
 
   const int Hkv = a.pool.kv_heads;
   const int G = a.q_heads / Hkv;
-  // Splits of a tile are neighbours, or, where max_splits says little about how many there are (the
-  // bound is a block-table row), the slowest index: workgroups go round-robin over the 8 XCDs, and
-  // the first splits of unsplit sequences would all meet on one (8 x (384 + 8) tokens, Hq16 / Hkv8,
-  // under a table of 2048 blocks: 19.4 us, 11.5 under the exact one).
-  const int first = gridDim.x / a.max_splits;
-  const int split = a.counters ? blockIdx.x / first : blockIdx.x % a.max_splits;
-  const int item = a.counters ? blockIdx.x % first : blockIdx.x / a.max_splits;
-  const int kvh = item % Hkv;
-  const int tile = item / Hkv;
-  const int b = blockIdx.y;
+  // The split is the slowest index.  max_splits follows the longest context there may be, and
+  // workgroups go round-robin over the 8 XCDs: with the splits of a tile side by side, the first
+  // splits of sequences shorter than that would meet on a few XCDs, between workgroups that leave
+  // at once (8 x (384 + 8) tokens, Hq16 / Hkv8, under a table of 2048 blocks: 19.4 us, 11.5 now;
+  // decode of 16 x U[500, 2000] tokens, Hq32 / Hkv4, called with a bound of 32768: 96 us, 34.5 now).
+  // The sequences are turned by one from split to split, so that one long sequence beside short
+  // ones does not keep to half of the XCDs either.
+  const int split = blockIdx.z;
+  const int b = (blockIdx.y + blockIdx.z) % gridDim.y;
+  const int kvh = blockIdx.x % Hkv;
+  const int tile = blockIdx.x / Hkv;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -613,7 +614,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 && is16(FMT) ? 1 : 2) void pag
   // its L2, so many splits are first merged in groups, each by the last of its own workgroups,
   // into the place of the group's first split (8 tokens over 16000, head_dim 128: 64 splits at
   // once 31.4 us, in groups 22.7).
-  int32_t *counters = &a.counters[((size_t)b * first + item) * (1 + kRowsMaxSplits / kSplitGroup)];
+  int32_t *counters = &a.counters[((size_t)b * gridDim.x + blockIdx.x) * (1 + kRowsMaxSplits / kSplitGroup)];
   if (sq.n_splits <= kFlatSplits) {
     if (last_to_arrive(counters, sq.n_splits)) merge_splits<D, false>(a, sq, b, kvh, G, row0, live, 0, 1, sq.n_splits);
     return;
@@ -667,9 +668,9 @@ __global__ __launch_bounds__(D) void paged_rows_merge_kernel(const RowsArgs a) {
 
 template <int D, int FMT, int PARTS>
 hipError_t launch_rows_t(const RowsArgs &a, hipStream_t s, void *hu, LaunchHook hook) {
-  const int tiles = (a.max_rows * (a.q_heads / a.pool.kv_heads) + TILE - 1) / TILE;
+  const unsigned tiles = (unsigned)(((long long)a.max_rows * (a.q_heads / a.pool.kv_heads) + TILE - 1) / TILE);
   if (hook) hook(hu, 0, s);
-  hipLaunchKernelGGL((paged_rows_kernel<D, FMT, PARTS>), dim3(a.max_splits * a.pool.kv_heads * tiles, a.num_seqs),
+  hipLaunchKernelGGL((paged_rows_kernel<D, FMT, PARTS>), dim3(tiles * a.pool.kv_heads, a.num_seqs, a.max_splits),
                      dim3(64 * WAVES), 0, s, a);
   hipError_t e = hipGetLastError();
   if (hook) hook(hu, 1, s);

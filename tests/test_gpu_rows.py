@@ -575,3 +575,29 @@ def test_prefill_table_wider_than_the_contexts(ctx, opts, D, Hq, Hkv, fmt, chunk
     assert torch.equal(*outs)
     assert ctx.device_errors() == 0, ctx.last_error()
 
+
+@pytest.mark.parametrize("fmt", ["bf16", "int8"])
+@pytest.mark.parametrize("D,Hq,Hkv", [(128, 32, 4), (128, 12, 4), (256, 8, 4)])
+def test_rows_decode_bound_far_above_the_lengths(ctx, D, Hq, Hkv, fmt):
+    """A step called with the model's longest context as its bound (as a captured graph is), with and
+    without a hint of the tokens, one long sequence among short and empty ones: as the oracle."""
+    import torch
+
+    from helpers import assert_parity
+
+    lens = np.array(EDGES + [5000], np.int32)
+    batch = workloads.paged_batch(lens, BT, 0.10, 161)
+    pool, q = build_case(ctx, batch, Hq, Hkv, FMTS[fmt], 162, head_dim=D)
+    tables = np.full((lens.size, 2048), -1, np.int32)
+    tables[:, :batch.tables.shape[1]] = batch.tables
+    ref = oracle_decode(pool, batch, FMTS[fmt], Hq, Hkv, 0, q, 0.088, head_dim=D)
+    for hint in (0, int(lens.sum())):
+        out = torch.full((q.size,), 0x7FC0, dtype=torch.int16, device="cuda")
+        desc = ctx.decode_desc(to_dev(lens), to_dev(tables), Hq, 32768, total_tokens_hint=hint)
+        before = ctx.route_calls()["rows_decode"]
+        ctx.paged_decode(pool, desc, to_dev(q), out, 0.088)
+        torch.cuda.synchronize()
+        assert ctx.route_calls()["rows_decode"] == before + 1
+        assert_parity(from_dev_bf16(out), ref, what=f"hint {hint}")
+    assert ctx.device_errors() == 0, ctx.last_error()
+
