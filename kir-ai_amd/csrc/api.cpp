@@ -74,14 +74,17 @@ constexpr int kD256MaxSplits = 64;      // partials the head_dim-256 merge combi
 // Whether a head_dim-128 split-K step merges in its own launch (the last workgroup of each
 // (sequence, kv head)) instead of a second one.  That saves the second launch, but the last
 // workgroup reads the partials alone and past its L2, and every workgroup waits for its stores:
-// it pays for few splits and small steps.  Measured on MI355X, two
-// launches / one (us): Hq16 / Hkv8, 1 x 512 10.2 / 7.5, 1 x 1000 10.9 / 7.9, 16 x U[50, 500]
-// 10.4 / 8.5, 1 x 4000 11.8 / 14.1, 4 x 4096 in the window 15.9 / 21.1; Hq32 / Hkv8, 1 x 1000
-// 10.7 / 9.5, 4 x U[500, 1000] 11.2 / 12.3.
-bool one_launch(int group, long long pairs, int splits) {
+// it pays for few splits and small steps.  Measured on MI355X, two launches / one (us), pairs x
+// splits: Hq16 / Hkv8 bf16, 1 x 1000 (8 x 16) 10.3 / 7.2, 16 x 600 (128 x 5) 10.8 / 9.4, 32 x 300
+// (256 x 3) 10.6 / 9.3, 4 x 2000 (32 x 16) 10.0 / 9.9, 8 x 1500 (64 x 12) 11.2 / 11.3, 16 x 1000
+// (128 x 8) 13.9 / 15.2; int8, 8 x 600 (64 x 10) 10.2 / 9.8, 16 x 600 (128 x 10) 13.2 / 15.0; Hq32 /
+// Hkv8 bf16, 1 x 1000 10.3 / 8.5, 2 x 1000 10.3 / 9.9; int8, 4 x 300 (32 x 5) 10.0 / 9.3, 2 x 600
+// (16 x 10) 9.9 / 10.1; Hq32 / Hkv4, 1 x 130 10.5 / 10.7.
+bool one_launch(int group, int format, long long pairs, int splits) {
   if (splits < 2 || splits > kOneLaunchSplits || pairs > kArrivalCounters) return false;
-  if (group <= 2) return pairs <= 256;
-  return pairs * splits <= (group == 4 ? 256 : 128);
+  const long long cost = (pairs + 16) * splits;
+  if (group <= 2) return cost <= 832;
+  return group == 4 && pairs * splits <= 256 && (is16(format) || cost <= 300);
 }
 
 struct SplitPlan {
@@ -930,7 +933,7 @@ int llh::launch_planned_decode(llh_ctx *ctx, const llh_kv_pool *pool, const llh_
     a.stream_wgs = plan.stream_wgs;
     a.max_seq_len = desc->max_seq_len;
     if (!plan.d256 && !plan.stream_wgs &&
-        one_launch(plan.group, (long long)desc->num_seqs * pv.kv_heads, plan.max_splits))
+        one_launch(plan.group, pv.format, (long long)desc->num_seqs * pv.kv_heads, plan.max_splits))
       a.counters = counters;
     if (a.counters) ctx->routes[LLH_ROUTE_ONE_LAUNCH]++;
     a.seg_desc = plan.stream_wgs ? reinterpret_cast<int32_t *>(ws + plan.desc_off) : nullptr;

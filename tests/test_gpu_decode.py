@@ -657,12 +657,13 @@ def test_decode_one_launch_merge_equals_two(ctx, Hq, Hkv, lens):
         torch.cuda.synchronize()
         for o in outs:
             assert torch.equal(o, two)
-    assert ctx.route_calls()["one_launch"] == before + 40
+    taken = 40 if Hq // Hkv < 8 else 0  # groups of eight: the second launch is cheaper
+    assert ctx.route_calls()["one_launch"] == before + taken
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph, stream=streams[0]):
         for _ in range(3):
             ctx.paged_decode(pool, desc, d_q, outs[0], 0.088, stream=torch.cuda.current_stream())
-    assert ctx.route_calls()["one_launch"] == before + 40
+    assert ctx.route_calls()["one_launch"] == before + taken
     for _ in range(4):
         outs[0].zero_()
         torch.cuda.synchronize()
@@ -681,7 +682,7 @@ def test_decode_one_launch_merge_equals_two(ctx, Hq, Hkv, lens):
 
 
 @pytest.mark.parametrize("fmt", [llm_hip.KV_BF16, llm_hip.KV_INT8])
-@pytest.mark.parametrize("Hq,Hkv,lens", [(16, 8, [512]), (8, 8, [70, 0, 1000, 33]), (64, 8, [250])])
+@pytest.mark.parametrize("Hq,Hkv,lens", [(16, 8, [512]), (8, 8, [70, 0, 1000, 33]), (32, 8, [250]), (64, 8, [250])])
 def test_decode_one_launch_merge_over_changing_inputs(ctx, Hq, Hkv, lens, fmt):
     """One-launch steps over two pools in turn, a new query each, back to back on one stream: the
     workspace always holds the other step's partials, and every step must still have the bits of
@@ -705,7 +706,7 @@ def test_decode_one_launch_merge_over_changing_inputs(ctx, Hq, Hkv, lens, fmt):
     for i in range(len(q)):
         ctx.paged_decode_noalloc(*cases[i % 2], q[i], two[i], 0.088)
     torch.cuda.synchronize()
-    assert ctx.route_calls()["one_launch"] == before + len(q)
+    assert ctx.route_calls()["one_launch"] == before + (len(q) if Hq // Hkv < 8 else 0)
     diff = (one != two).sum(1)
     assert not diff.any(), f"{int((diff > 0).sum())} of {len(q)} steps differ, {int(diff.sum())} outputs in all"
     assert ctx.device_errors() == 0, ctx.last_error()
