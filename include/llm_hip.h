@@ -104,7 +104,8 @@ const char *llh_ctx_last_error(const llh_ctx *ctx);
  * ones grow now; a new stream's first call allocates at least this much). */
 int llh_ctx_reserve_workspace(llh_ctx *ctx, size_t bytes);
 /* Allocates (or grows) the workspace of one stream now, so that its batched
- * calls of at most this size allocate nothing. */
+ * calls of at most this size allocate nothing (prefill calls that split their keys
+ * have scratch of their own: llh_paged_prefill). */
 int llh_ctx_reserve_stream_workspace(llh_ctx *ctx, void *stream, size_t bytes);
 /* Frees one stream's workspace (after waiting for the device).  Call it before
  * destroying a stream that made batched calls on this context. */
