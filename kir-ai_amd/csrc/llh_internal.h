@@ -145,6 +145,7 @@ struct PrefillArgs {
   float scale_log2e;
   float scale;              // score_scale (generic kernel)
   const uint16_t *gate;     // null, or [T][Hq][D] bf16: out = attention * sigmoid(gate)
+  int32_t run;              // head_dim 256: tiles of a group that follow each other in the order of whole items
 };
 
 // Packed query rows over split keys (rows.hip): decode steps outside the tuned shapes

@@ -229,7 +229,7 @@ __device__ __forceinline__ void store_tile(uint16_t *k_lds, uint16_t *v_lds, int
 template <int HPW, int FMT>
 __global__ __launch_bounds__(kPrefillThreads * HPW, 2 / HPW) void paged_prefill_kernel(const PrefillArgs a) {
   constexpr int BM = 128 * HPW;  // packed query rows per workgroup
-  const PrefillItem it = prefill_item<D, BM, 256>(a);
+  const PrefillItem it = prefill_item<BM, 256>(a);
   if (it.skip) {
     if (it.flags && threadIdx.x == 0) atomicOr(a.err, it.flags);
     return;

@@ -177,7 +177,7 @@ __device__ __forceinline__ void store_tile(uint16_t *k_lds, uint16_t *v_lds, int
 
 template <int FMT>
 __global__ __launch_bounds__(kThreads, 1) void paged_prefill_d256_kernel(const PrefillArgs a) {
-  const PrefillItem it = prefill_item<D, BM, BM>(a);
+  const PrefillItem it = prefill_item<BM, BM>(a);
   if (it.skip) {
     if (it.flags && threadIdx.x == 0) atomicOr(a.err, it.flags);
     return;

@@ -142,22 +142,13 @@ __device__ __forceinline__ PrefillItem prefill_item_of(const PrefillArgs &a, int
   return it;
 }
 
-// Tiles of a group that follow each other in the order below, before the next group's.  They read
-// the same keys at the same time, but put short sequences' items behind long ones'.  Head_dim 256,
-// items of 16 tokens (eight heads packed), 32 ragged sequences of up to 2500 + 256 tokens, six
-// draws (us): run of 1 280 - 390, run of 8 232 - 365; two heads packed: 149 - 213, run of 2
-// 170 - 212.  At head_dim 128, whose items hold twice the rows, runs of 1 are the faster ones.
-__device__ __forceinline__ int prefill_run(int head_dim, int pack) {
-  return head_dim == kD256HeadDim && pack >= 8 ? pack : 1;
-}
-
 // The item, or piece, of this workgroup L: number (L % 8) * ceil(N / 8) + L / 8 of N.
 // Nothing cut: N counts q_tiles items for every (sequence, head group), in that order; an XCD
 // whose items are whole (sequence, head group) groups takes the last tile of every group first,
-// the longest causal reach first, in runs of prefill_run tiles.  Else N counts the items and pieces there are, ordered
+// the longest causal reach first, in runs of a.run tiles.  Else N counts the items and pieces there are, ordered
 // (sequence, head group, piece, tile from the last), so ragged lengths leave no XCD idle.
 // Workgroups past N leave at once.
-template <int D, int BM, int CUT>
+template <int BM, int CUT>
 __device__ __forceinline__ PrefillItem prefill_item(const PrefillArgs &a) {
   const int L = blockIdx.x;
   PrefillItem none;
@@ -198,7 +189,7 @@ __device__ __forceinline__ PrefillItem prefill_item(const PrefillArgs &a) {
   int local = L / 8;
   if (per_xcd % a.q_tiles == 0) {
     const int groups = per_xcd / a.q_tiles;
-    const int run = prefill_run(D, a.pack);
+    const int run = CUT == 128 ? a.run : 1;  // (the head_dim-256 kernel)
     const int whole = a.q_tiles / run * run;  // tiles in whole runs
     const int i = L / 8 - groups * whole;
     if (i < 0) {
